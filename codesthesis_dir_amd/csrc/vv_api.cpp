@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "vv_internal.h"
+#include "vv_lines.h"
 
 namespace vv {
 
@@ -190,9 +191,44 @@ int upload_tab(vv_run *r, double **dst, const std::vector<double> &h)
     return VV_OK;
 }
 
+// The tables of the chunked line kernel in the order of its LDS (vv_lines.h):
+// LTC = 8 closing words, then over the head's places f | b | 1/b [| c], the
+// places before row 0 neutral (f = 0, b = 1).  Whether every row from the
+// 17th on (before the last, whose closing form has its own words) has the
+// settled factor and pivot and c = 1.
+constexpr int PK_CLOSE = 8;
+
+bool pack_head(std::vector<double> &t, const double *f, const double *b, const double *c, int N, bool with_c,
+               const std::vector<double> &close)
+{
+    const int sh = lshift(N), hw = lheadb(N) * LU;
+    t = close;
+    t.resize(PK_CLOSE, 0.0);
+    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 0.0 : f[p - sh]);
+    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : b[p - sh]);
+    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : 1.0 / b[p - sh]);
+    bool ok = true;
+    if (with_c)
+        for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : c[p - sh]);
+    for (int q = 0; q < N; ++q) {
+        if (!with_c || q + sh >= hw) ok = ok && c[q] == 1.0;
+        if (q + sh >= hw) ok = ok && f[q] == LF && b[q] == LB;
+    }
+    return ok;
+}
+
+// blocks of the N places (row q at q + lshift(N)) up to the last nonzero v[q]
+int blocks_used(const double *v, int N)
+{
+    int n = N;
+    while (n > 0 && v[n - 1] == 0.0) --n;
+    return n == 0 ? 0 : (n - 1 + lshift(N)) / LU + 1;
+}
+
 int build_tables(vv_run *r)
 {
     const int nr = r->nr, np = r->np;
+    bool ok = true;
     {   // Cr, thr at vorticity points: 1-4-1, n = nr-1 (rb.f:810-826)
         const int n = nr - 1;
         std::vector<double> a(n, 1.0), b(n, 4.0), c(n, 1.0);
@@ -203,7 +239,13 @@ int build_tables(vv_run *r)
         h.insert(h.end(), t.bp.begin(), t.bp.end());
         h.insert(h.end(), t.c.begin(), t.c.end());
         for (double v : t.bp) h.push_back(1.0 / v);
+        std::vector<double> pk;
+        ok = pack_head(pk, t.fact.data(), t.bp.data(), t.c.data(), n - 1, true,
+                             {t.fact[n - 1], t.bp[n - 1], 1.0 / t.bp[n - 1]}) && ok;
+        const size_t at = h.size();
+        h.insert(h.end(), pk.begin(), pk.end());
         int st = upload_tab(r, &r->tab_r1, h);
+        r->pk_r1 = r->tab_r1 + at;
         if (st) return st;
     }
     {   // thr at temperature points with closure rows (rb.f:1244-1262)
@@ -218,7 +260,13 @@ int build_tables(vv_run *r)
         h.insert(h.end(), t.bp.begin(), t.bp.end());
         h.insert(h.end(), t.c.begin(), t.c.end());
         for (double v : t.bp) h.push_back(1.0 / v);
+        std::vector<double> pk;
+        ok = pack_head(pk, t.fact.data(), t.bp.data(), t.c.data(), n - 1, true,
+                             {t.fact[n - 1], t.bp[n - 1], 1.0 / t.bp[n - 1]}) && ok;
+        const size_t at = h.size();
+        h.insert(h.end(), pk.begin(), pk.end());
         int st = upload_tab(r, &r->tab_rT, h);
+        r->pk_rT = r->tab_rT + at;
         if (st) return st;
     }
     {   // cyclic 1-4-1 on np+1 points (rb.f:833-845)
@@ -236,9 +284,29 @@ int build_tables(vv_run *r)
         h.push_back(t.fB);
         h.push_back(t.fC);
         for (double v : t.b) h.push_back(v != 0.0 ? 1.0 / v : 0.0);   // entry 0 is unused
+        const int N = n - 2, sh = lshift(N);
+        std::vector<double> pk;
+        ok = pack_head(pk, t.f1.data() + 1, t.b.data() + 1, t.c.data() + 1, N, false,
+                             {t.fA, t.fB, t.fC, t.b[n], 1.0 / t.b[n], t.c[n - 1], t.b[n - 1], 1.0 / t.b[n - 1]}) && ok;
+        // a over its places, a block of zeros, then the factors of rn: place p
+        // holds f2 of the row after p's
+        r->pk_na = std::max(blocks_used(t.a.data() + 1, N), lheadb(N));
+        r->pk_nf = blocks_used(t.f2.data() + 1, N);
+        const size_t ta = pk.size();
+        pk.resize(ta + (size_t)(r->pk_na + 1) * (LU + 1) + (size_t)r->pk_nf * LU, 0.0);
+        const size_t tg = ta + (size_t)(r->pk_na + 1) * (LU + 1);
+        for (int q = 0; q < N; ++q) {
+            const int p = q + sh;
+            if (p < r->pk_na * LU) pk[ta + lrow(p)] = t.a[q + 1];
+            if (q > 0 && p - 1 < r->pk_nf * LU) pk[tg + p - 1] = t.f2[q + 1];
+        }
+        const size_t at = h.size();
+        h.insert(h.end(), pk.begin(), pk.end());
         int st = upload_tab(r, &r->tab_p, h);
+        r->pk_p = r->tab_p + at;
         if (st) return st;
     }
+    if (!ok) { set_error("vv_create: a compact system's rows do not settle"); return VV_EINVAL; }
     return VV_OK;
 }
 

@@ -9,6 +9,8 @@
 // Field layout: F[k*ld + i], i = 0..nr+1 across the walls, k = 0..np.
 
 #include "vv_internal.h"
+#include "vv_gemm.h"
+#include "vv_lines.h"
 #include "vv_reduce.h"
 
 #include <algorithm>
@@ -21,22 +23,6 @@ namespace {
 constexpr int WG = 256;
 
 __device__ __forceinline__ size_t ix(int i, int k, int ld) { return (size_t)k * ld + i; }
-
-// x / b for b > 0, correctly rounded, from rb = 1/b correctly rounded
-// (computed on the host): q0 = x*rb is within one ulp of x/b, the remainder
-// is exact in one FMA, and q0 + rem*rb rounds to x/b (Markstein's theorem
-// for division with a fused multiply-add; no overflow or underflow occurs for
-// these operands).  The remainder is formed as t = b*q0 - x and applied as
-// -t: when it is zero, t = +0 and q0 + (-0)*rb keeps q0 and the sign of a
-// zero quotient, so no select is needed.  Three dependent operations replace
-// the IEEE division sequence on the recurrence's critical path, with the same
-// result.  The elimination tables are checked for b > 0 when they are built.
-__device__ __forceinline__ double div_rb(double x, double b, double rb)
-{
-    const double q0 = x * rb;
-    const double t = __builtin_fma(b, q0, -x);
-    return __builtin_fma(-t, rb, q0);
-}
 
 // single-precision literals of rb.f:660-668 promoted to double
 __device__ __forceinline__ double f23() { return (double)(2.f / 3.f); }
@@ -110,205 +96,345 @@ __device__ __forceinline__ double rhs_p(const CompactArgs &a, int i, int j)
     return 3.0 * (X[ix(i, k + 1, ld)] - X[ix(i, k - 1, ld)]) * dpi;
 }
 
-// Batched Thomas along r, the reference tdma (rb.f:3046-3064) with its
-// elimination factors from TdmaTab (fact | bp | c): the workgroup computes
-// the right-hand sides of its T columns into LDS with coalesced loads, one
-// thread per column then runs the recurrences in the reference's order, and
-// the workgroup writes the solutions back.  LDS row stride nP is odd.
-template <int FAM, bool TL>
-__device__ void tdma_tile(const CompactArgs &a, double *R, double *Tab, int T)
+// One compact line: rows 0..n-1 of family FAM (row q is the reference's row
+// q+1), nc = 1 (tdma) or 2 (ptdma) of them closed by themselves after the
+// others.  families 0-2 are lines along r (line = column k), 3-5 lines along
+// phi (line = row i).
+template <int FAM>
+__device__ __forceinline__ double line_rhs(const CompactArgs &a, int line, int q)
 {
-    const int nr = a.nr, ld = a.ld, np = a.np;
-    const int n = (FAM == 2) ? nr : nr - 1;
-    const int nP = n | 1;
-    const double *tab = (FAM == 2) ? a.tab_rT : a.tab_r1;
-    double *out = (FAM == 0) ? a.dCr : (FAM == 1) ? a.dthrC : a.dthrT;
-    const int k0 = blockIdx.x * T;
-    if (k0 > np) return;
-    const int tc = (np + 1 - k0 < T) ? np + 1 - k0 : T;
-    // the elimination factors go to LDS with the right-hand sides (when they
-    // fit), so the recurrences below read nothing from global memory
-    if (TL) {
-#pragma unroll 8
-        for (int idx = threadIdx.x; idx < 4 * n; idx += blockDim.x) Tab[idx] = tab[idx];
-    }
-    const double *tb = TL ? Tab : tab;
-    const double *fact = tb, *bp = tb + n, *cc = tb + 2 * n, *rbp = tb + 3 * n;
-#pragma unroll 8
-    for (int idx = threadIdx.x; idx < tc * n; idx += blockDim.x) {
-        const int c = idx / n, j = idx - c * n;
-        R[c * nP + j] = rhs_r<FAM>(a, j + 1, k0 + c);
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < tc) {
-        // the recurrences in blocks of U: the loads of a block are issued
-        // before its dependent chain, so only the arithmetic is serial
-        constexpr int U = 8;
-        double *r = R + threadIdx.x * nP;
-        double rp = r[0];
-        int j = 1;
-        for (; j + U <= n; j += U) {
-            double fr[U], rr[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) { fr[u] = fact[j + u]; rr[u] = r[j + u]; }
-#pragma unroll
-            for (int u = 0; u < U; ++u) { rp = rr[u] - fr[u] * rp; r[j + u] = rp; }
-        }
-        for (; j < n; ++j) {
-            rp = r[j] - fact[j] * rp;
-            r[j] = rp;
-        }
-        double y = div_rb(rp, bp[n - 1], rbp[n - 1]);
-        r[n - 1] = y;
-        j = n - 2;
-        for (; j - U + 1 >= 0; j -= U) {
-            double cr[U], br[U], ir[U], rr[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                cr[u] = cc[j - u]; br[u] = bp[j - u]; ir[u] = rbp[j - u]; rr[u] = r[j - u];
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) { y = div_rb(rr[u] - cr[u] * y, br[u], ir[u]); r[j - u] = y; }
-        }
-        for (; j >= 0; --j) {
-            y = div_rb(r[j] - cc[j] * y, bp[j], rbp[j]);
-            r[j] = y;
-        }
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (int idx = threadIdx.x; idx < tc * n; idx += blockDim.x) {
-        const int c = idx / n, j = idx - c * n;
-        out[ix(j + 1, k0 + c, ld)] = R[c * nP + j];
-    }
+    if constexpr (FAM < 3) return rhs_r<FAM>(a, q + 1, line);
+    else return rhs_p<FAM>(a, line, q + 1);
+}
+// Place of row q in a line's LDS: the N rows' places, the closing rows behind
+// them.
+__device__ __forceinline__ int line_pos(int q, int N)
+{
+    return q < N ? lrow(q + lshift(N)) : lwords(N) + (q - N);
 }
 
-// Batched cyclic solve along phi, the reference ptdma (rb.f:3066-3116) on
-// n = np+1 points with the factors of PtdmaTab (1-based, stride n+1:
-// f1 | f2 | a | b | c | fA fB fC).  LDS holds entry j of row c at
-// (j-1)*T + c, so the per-row recurrences of consecutive threads touch
-// consecutive words.
-template <int FAM, bool TL>
-__device__ void ptdma_tile(const CompactArgs &a, double *R, double *Tab, int T)
+// How a family's lines are split: P lanes a line (mb blocks each beyond the
+// warm-up), T lines a workgroup (T P <= WG).
+struct LineTile {
+    int P, lgP, T, mb;
+};
+struct CompactTiles {
+    LineTile r, p;
+    const double *pk1, *pkT, *pkp;   // the tables packed in LDS order (pack_tdma, pack_ptdma)
+    int na, nf;         // blocks of ptdma's a and f2 that are not all zero
+    int tabw;           // LDS words of the tables, in front of the lines
+};
+
+// The workgroup's lines: n rows, N of them before the closing ones, pitch
+// LDS words a line from word R on.  The tables' words: LTC closing words,
+// then over the head's places f | b | 1/b | c (r) or f | b | 1/b (phi), and
+// for phi a over all places (zeros left out, a block of zeros behind) and the
+// factors of rn, g_p = f2 of the next place, in whole blocks.
+constexpr int LTC = 8;
+struct LineSet {
+    int n, N, pitch, first, tc, R;
+    int hw;                 // places of the head
+    int Ta, Tg, taw, nf;    // phi: words of a and g, words of a before its zeros, blocks of g
+};
+
+// The reference tdma / ptdma (rb.f:3046-3116) row by row on one lane, from
+// the right-hand sides in the line's LDS at Q: lines whose chunks did not
+// meet.
+template <bool CYC>
+__device__ __forceinline__ void line_seq(const CompactArgs &a, int fam, double *S, int Q, int n)
 {
-    const int np = a.np, ld = a.ld;
-    const int n = np + 1;
-    const int s = n + 1;
-    const int rows = (FAM == 5) ? a.nr : a.nr - 1;   // rows 1..rows
-    const int i0 = 1 + blockIdx.x * T;
-    if (i0 > rows) return;
-    const int tc = (rows + 1 - i0 < T) ? rows + 1 - i0 : T;
-    double *out = (FAM == 3) ? a.dCh : (FAM == 4) ? a.dthhC : a.dthhT;
-    // elimination factors to LDS when they fit (see tdma_tile)
-    if (TL) {
-#pragma unroll 8
-        for (int idx = threadIdx.x; idx < 6 * s + 3; idx += blockDim.x) Tab[idx] = a.tab_p[idx];
-    }
-    const double *tb = TL ? Tab : a.tab_p;
-#pragma unroll 8
-    for (int idx = threadIdx.x; idx < tc * n; idx += blockDim.x) {
-        const int j = idx / tc, c = idx - j * tc;
-        R[j * T + c] = rhs_p<FAM>(a, i0 + c, j + 1);
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < tc) {
-        const double *f1 = tb, *f2 = tb + s, *aa = tb + 2 * s;
-        const double *bb = tb + 3 * s, *cc = tb + 4 * s;
-        const double fA = tb[5 * s], fB = tb[5 * s + 1], fC = tb[5 * s + 2];
-        const double *rbb = tb + 5 * s + 3;
-        const int c = threadIdx.x;
-#define R_(j) R[((j) - 1) * T + c]
-        constexpr int U = 8;   // blocked as in tdma_tile
-        double rn = R_(n);
-        double rm = R_(1);
-        int j = 2;
-        for (; j + U - 1 <= n - 2; j += U) {
-            double g1[U], g2[U], rr[U];
+    constexpr int U = LU;
+    const int N = CYC ? n - 2 : n - 1, st = n + 1;
+    const double *tb = CYC ? a.tab_p + 1 : (fam == 2) ? a.tab_rT : a.tab_r1;
+    const double *f1 = tb, *bb = CYC ? tb + 3 * st : tb + n, *cc = CYC ? tb + 4 * st : tb + 2 * n,
+                 *rbb = CYC ? tb + 5 * st + 3 : tb + 3 * n, *f2 = tb + st, *aa = tb + 2 * st;
+#define R_(q) S[Q + line_pos((q), N)]
+    double rm = R_(0), rn = CYC ? R_(n - 1) : 0.0;
+#pragma unroll 1
+    for (int q = 1; q < N; q += U) {
+        double g1[U], g2[U], rr[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) { g1[u] = f1[j + u]; g2[u] = f2[j + u]; rr[u] = R_(j + u); }
+        for (int u = 0; u < U; ++u) {
+            const int w = q + u < N ? q + u : N - 1;
+            g1[u] = f1[w];
+            g2[u] = CYC ? f2[w] : 0.0;
+            rr[u] = R_(w);
+        }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
+        for (int u = 0; u < U; ++u)
+            if (q + u < N) {
                 const double r = rr[u] - g1[u] * rm;
-                rn = rn - g2[u] * rm;
-                R_(j + u) = r;
+                if (CYC) rn = rn - g2[u] * rm;
+                R_(q + u) = r;
                 rm = r;
             }
-        }
-        for (; j <= n - 2; ++j) {
-            const double r = R_(j) - f1[j] * rm;
-            rn = rn - f2[j] * rm;
-            R_(j) = r;
-            rm = r;
-        }
-        const double rn1 = R_(n - 1) - fA * R_(n - 2);
-        rn = rn - fB * R_(n - 2);
-        rn = rn - fC * rn1;
-        const double yn = div_rb(rn, bb[n], rbb[n]);
-        double y = div_rb(rn1 - cc[n - 1] * yn, bb[n - 1], rbb[n - 1]);
-        R_(n) = yn;
-        R_(n - 1) = y;
-        j = n - 2;
-        for (; j - U + 1 >= 1; j -= U) {
-            double cr[U], ar[U], br[U], ir[U], rr[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                cr[u] = cc[j - u]; ar[u] = aa[j - u]; br[u] = bb[j - u]; ir[u] = rbb[j - u]; rr[u] = R_(j - u);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                y = div_rb(rr[u] - cr[u] * y - ar[u] * yn, br[u], ir[u]);
-                R_(j - u) = y;
-            }
-        }
-        for (; j >= 1; --j) {
-            y = div_rb(R_(j) - cc[j] * y - aa[j] * yn, bb[j], rbb[j]);
-            R_(j) = y;
-        }
-#undef R_
     }
-    __syncthreads();
-#pragma unroll 8
-    for (int idx = threadIdx.x; idx < tc * n; idx += blockDim.x) {
-        const int j = idx / tc, c = idx - j * tc;
-        out[ix(i0 + c, j, ld)] = R[j * T + c];
+    double y, yn = 0.0;
+    if (CYC) {
+        const double fA = tb[5 * st - 1], fB = tb[5 * st], fC = tb[5 * st + 1];
+        const double rn1 = R_(n - 2) - fA * rm;
+        rn = rn - fB * rm;
+        rn = rn - fC * rn1;
+        yn = line_div(rn, bb[n - 1], rbb[n - 1]);
+        y = line_div(rn1 - cc[n - 2] * yn, bb[n - 2], rbb[n - 2]);
+        R_(n - 1) = yn;
+        R_(n - 2) = y;
+    } else {
+        rm = R_(n - 1) - f1[n - 1] * rm;
+        y = line_div(rm, bb[n - 1], rbb[n - 1]);
+        R_(n - 1) = y;
+    }
+#pragma unroll 1
+    for (int q = N - 1; q >= 0; q -= U) {
+        double cr[U], ar[U], br[U], ir[U], rr[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int w = q - u >= 0 ? q - u : 0;
+            cr[u] = cc[w];
+            ar[u] = CYC ? aa[w] : 0.0;
+            br[u] = bb[w];
+            ir[u] = rbb[w];
+            rr[u] = R_(w);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (q - u >= 0) {
+                double x = rr[u] - cr[u] * y;
+                if (CYC) x = x - ar[u] * yn;
+                y = line_div(x, br[u], ir[u]);
+                R_(q - u) = y;
+            }
+    }
+#undef R_
+}
+
+// Right-hand sides of the workgroup's lines into LDS, zeros before row 0 and
+// in the word of max |r|.  r families: a wavefront per line, the end rows'
+// one-sided forms written over the interior form; phi families: consecutive
+// threads on consecutive rows i, the two columns of the period's ends reading
+// the same pair of neighbours.
+template <int FAM>
+__device__ __forceinline__ void line_stage(const CompactArgs &a, const LineSet &s, int T, double *S)
+{
+    const int tid = (int)threadIdx.x, ld = a.ld, np = a.np, sh = lshift(s.N);
+    if constexpr (FAM < 3) {
+        const double *X = FAM == 0 ? a.C : a.th;
+        for (int c = tid >> 6; c < s.tc; c += WG / 64) {
+            const int k = s.first + c, ka = (k == np) ? 1 : k + 1, Q = s.R + c * s.pitch;
+            const double *x = X + ix(0, k, ld), *xa = X + ix(0, ka, ld);
+            const int qe = (tid & 1) ? s.n - 1 : 0;
+            const double ve = (tid & 63) < 2 ? rhs_r<FAM>(a, qe + 1, k) : 0.0;
+#pragma unroll 4
+            for (int q = tid & 63; q < s.n; q += 64) {
+                double v;
+                if (FAM == 1) v = 1.5 * (x[q + 2] + xa[q + 2] - x[q + 1] - xa[q + 1]) * a.dri;
+                else v = 3.0 * (x[q + 2] - x[q]) * a.dri;
+                S[Q + line_pos(q, s.N)] = v;
+            }
+            wave_fence();
+            if ((tid & 63) < 2) S[Q + line_pos(qe, s.N)] = ve;
+            if ((tid & 63) < sh) S[Q + (tid & 63)] = 0.0;
+        }
+    } else {
+        const double *X = FAM == 3 ? a.C : a.th;
+        const int lgT = 31 - __clz(T);
+#pragma unroll 4
+        for (int e = tid; e < (s.n << lgT); e += WG) {
+            const int c = e & (T - 1), k = e >> lgT;
+            if (c < s.tc) {
+                const int i = s.first + c;
+                double v;
+                if (FAM == 4) {
+                    const int ka = (k == np) ? 1 : k + 1;
+                    v = 1.5 * (X[ix(i + 1, ka, ld)] + X[ix(i, ka, ld)] - X[ix(i + 1, k, ld)] - X[ix(i, k, ld)]) * a.dpi;
+                } else {
+                    const bool end = k == 0 || k == np;
+                    v = 3.0 * (X[ix(i, end ? 1 : k + 1, ld)] - X[ix(i, end ? np - 1 : k - 1, ld)]) * a.dpi;
+                }
+                S[s.R + c * s.pitch + line_pos(k, s.N)] = v;
+            }
+        }
+        const int c = tid >> 3, p = tid & 7;
+        if (c < s.tc) {   // T <= 16: one thread per line and place
+            if (p < sh) S[s.R + c * s.pitch + p] = 0.0;
+            if (p == 7) S[s.R + c * s.pitch + lwords(s.N) + 2] = 0.0;
+        }
     }
 }
 
-struct CompactTiles {
-    int Tr, Tp;    // columns per workgroup (r families), rows per workgroup (phi families)
-    int rwords;    // LDS words of the right-hand-side tile; the tables follow
-    int tab_lds;   // 1: the elimination tables are staged in LDS
-};
+// The settled rows of a line are run by its P lanes as chunks with proven
+// entries (vv_lines.h), the head's places and the closing rows by all of them
+// alike.  Bound by the chain's instructions: 2 (40 + 8 mb) + 48 rows a lane,
+// where one lane a line ran 2 n.  Measured, the whole kernel, one lane a line
+// against this: 12.7 -> 12.8 us at 65x33, 41 -> 14.5 at 97x337, 42 -> 19 at
+// 513x257, 154 -> 38 at 1025x513, 3265 -> 262 at 2049x2049 (where the tables
+// had left LDS as well).  Returns whether every entry was proven.
+template <bool CYC>
+__device__ __forceinline__ bool line_solve(const LineSet &s, const LineTile &L, double *S)
+{
+    const int tid = (int)threadIdx.x, li = tid >> L.lgP, c = tid & (L.P - 1);
+    const int hb = s.hw / LU, nb = lblocks(s.N) - hb;   // blocks of the head, settled blocks
+    const int Q = s.R + li * s.pitch, X = Q + lwords(s.N), Q0 = Q + hb * (LU + 1);
+    const int Th = LTC;
+    double rp = 0.0, mx = 0.0;
+#pragma unroll 1
+    for (int b = 0; b < hb; ++b) rp = block_fwd<true>(S, Q + b * (LU + 1), Th + b * LU, c == 0, rp);
+    bool ok = true;
+    if (nb > 0) {
+        ok = line_fwd<CYC>(S, Q0, nb, c, L.mb, L.P, rp, mx);
+        rp = S[X - 2];   // the last place
+    }
+    // closing rows
+    double y, yn = 0.0;
+    if (CYC) {
+        // rn takes f2_j r_{j-1} of every row in the reference's order;
+        // |f2_j+1| = |f2_j| / b_j falls off as 0.268^j, so once the rest
+        // cannot move rn's last bit (|f2| max|r| below 2^-57 |rn|) it is
+        // left out
+        if (nb > LWB) atomicMax(reinterpret_cast<unsigned long long *>(S) + X + 2, (unsigned long long)__double_as_longlong(mx));
+        wave_fence();
+        double rn = S[X + 1];
+        const double m = S[X + 2];
+        const int free = hb + LWB;   // blocks that m does not cover
+#pragma unroll 1
+        for (int b = 0; b < s.nf; ++b) {
+            double g[LU], r[LU];
+#pragma unroll
+            for (int u = 0; u < LU; ++u) {
+                g[u] = S[s.Tg + b * LU + u];
+                r[u] = S[Q + b * (LU + 1) + u];
+            }
+            if (b >= free && fabs(g[0]) * m <= 0x1p-57 * fabs(rn)) break;
+#pragma unroll
+            for (int u = 0; u < LU; ++u) rn = rn - g[u] * r[u];
+        }
+        const double rn1 = S[X] - S[0] * rp;
+        rn = rn - S[1] * rp;
+        rn = rn - S[2] * rn1;
+        yn = line_div(rn, S[3], S[4]);
+        y = line_div(rn1 - S[5] * yn, S[6], S[7]);
+        wave_fence();
+        if (c == 0) {
+            S[X + 1] = yn;
+            S[X] = y;
+        }
+    } else {
+        rp = S[X] - S[0] * rp;
+        y = line_div(rp, S[1], S[2]);
+        wave_fence();
+        if (c == 0) S[X] = y;
+    }
+    if (nb > 0) {
+        const int o = hb * (LU + 1);
+        ok = line_back<CYC>(S, Q0, nb, c, L.mb, L.P, y, s.Ta + o, s.taw - o, yn) && ok;
+        y = S[Q0];
+    }
+#pragma unroll 1
+    for (int b = hb - 1; b >= 0; --b)
+        y = block_back<true, CYC>(S, Q + b * (LU + 1), Th + s.hw + b * LU, Th + 2 * s.hw + b * LU, Th + 3 * s.hw + b * LU,
+                                  s.Ta + b * (LU + 1), c == 0, yn, y);
+    return ok;
+}
+
+__device__ __forceinline__ double line_rhs_any(const CompactArgs &a, int fam, int line, int q)
+{
+    switch (fam) {
+    case 0: return line_rhs<0>(a, line, q);
+    case 1: return line_rhs<1>(a, line, q);
+    case 2: return line_rhs<2>(a, line, q);
+    case 3: return line_rhs<3>(a, line, q);
+    case 4: return line_rhs<4>(a, line, q);
+    default: return line_rhs<5>(a, line, q);
+    }
+}
+
+template <bool CYC>
+__device__ __forceinline__ void line_finish(const CompactArgs &a, const LineTile &L, int fam, const LineSet &s, double *out,
+                                            double *S)
+{
+    const int tid = (int)threadIdx.x, N = s.N;
+    const int li = tid >> L.lgP, c = tid & (L.P - 1);
+    if (li < s.tc) {   // the P lanes of a line are one wavefront's, and leave together
+        const bool ok = line_solve<CYC>(s, L, S);
+        const unsigned long long lm = (L.P == 64 ? ~0ull : ((1ull << L.P) - 1)) << ((tid & 63) & ~(L.P - 1));
+        if ((__ballot(ok) & lm) != lm) {   // row by row, from the right-hand sides again
+            const int Q = s.R + li * s.pitch;
+            wave_fence();
+#pragma unroll 1
+            for (int q = c; q < s.n; q += L.P) S[Q + line_pos(q, N)] = line_rhs_any(a, fam, s.first + li, q);
+            wave_fence();
+            if (c == 0) line_seq<CYC>(a, fam, S, Q, s.n);
+        }
+    }
+    __syncthreads();
+    if (CYC) {
+        const int lgT = 31 - __clz(L.T);
+#pragma unroll 4
+        for (int e = tid; e < (s.n << lgT); e += WG) {
+            const int cc = e & (L.T - 1), q = e >> lgT;
+            if (cc < s.tc) out[ix(s.first + cc, q, a.ld)] = S[s.R + cc * s.pitch + line_pos(q, N)];
+        }
+    } else {
+        for (int cc = tid >> 6; cc < s.tc; cc += WG / 64)
+#pragma unroll 4
+            for (int q = tid & 63; q < s.n; q += 64)
+                out[ix(q + 1, s.first + cc, a.ld)] = S[s.R + cc * s.pitch + line_pos(q, N)];
+    }
+}
 
 __global__ void __launch_bounds__(WG) k_compact(CompactArgs a, CompactTiles t)
 {
-    extern __shared__ double R[];
+    extern __shared__ double S[];
     const int fam = blockIdx.y;
     if (!(a.mask & (1 << fam))) return;
-    // the table's place is a template parameter, so that the recurrences'
-    // table reads compile to LDS reads (a pointer chosen at run time between
-    // LDS and global memory would make them generic loads, whose every wait
-    // covers the global-memory counter as well)
-    if (t.tab_lds) {
-        double *Tab = R + t.rwords;
-        switch (fam) {
-        case 0: tdma_tile<0, true>(a, R, Tab, t.Tr); break;
-        case 1: tdma_tile<1, true>(a, R, Tab, t.Tr); break;
-        case 2: tdma_tile<2, true>(a, R, Tab, t.Tr); break;
-        case 3: ptdma_tile<3, true>(a, R, Tab, t.Tp); break;
-        case 4: ptdma_tile<4, true>(a, R, Tab, t.Tp); break;
-        case 5: ptdma_tile<5, true>(a, R, Tab, t.Tp); break;
-        }
-    } else {
-        switch (fam) {
-        case 0: tdma_tile<0, false>(a, R, nullptr, t.Tr); break;
-        case 1: tdma_tile<1, false>(a, R, nullptr, t.Tr); break;
-        case 2: tdma_tile<2, false>(a, R, nullptr, t.Tr); break;
-        case 3: ptdma_tile<3, false>(a, R, nullptr, t.Tp); break;
-        case 4: ptdma_tile<4, false>(a, R, nullptr, t.Tp); break;
-        case 5: ptdma_tile<5, false>(a, R, nullptr, t.Tp); break;
-        }
+    const bool cyc = fam >= 3;
+    const LineTile L = cyc ? t.p : t.r;
+    LineSet s;
+    s.n = cyc ? a.np + 1 : (fam == 2) ? a.nr : a.nr - 1;
+    s.N = cyc ? s.n - 2 : s.n - 1;
+    const int lines = cyc ? ((fam == 5) ? a.nr : a.nr - 1) : a.np + 1, l0 = cyc ? 1 : 0;
+    const unsigned nb = (unsigned)((lines + L.T - 1) / L.T);
+    if (blockIdx.x >= nb) return;
+    // neighbouring workgroups of a phi family read the same 128-byte lines:
+    // each XCD takes a contiguous range of them
+    s.first = l0 + (int)xcd_block(blockIdx.x, nb) * L.T;
+    s.tc = min(L.T, lines + l0 - s.first);
+    double *out = fam == 0 ? a.dCr : fam == 1 ? a.dthrC : fam == 2 ? a.dthrT : fam == 3 ? a.dCh : fam == 4 ? a.dthhC : a.dthhT;
+    s.pitch = lpitch(s.N, cyc ? 3 : 1);
+    s.R = t.tabw;
+    s.hw = lheadb(s.N) * LU;
+    s.Ta = LTC + 3 * s.hw;
+    s.taw = t.na * (LU + 1);
+    s.Tg = s.Ta + s.taw + LU + 1;
+    s.nf = t.nf;
+    // the tables of the chunked form, packed in LDS order; loaded before the
+    // right-hand sides and stored after them, so that both are in flight
+    const double *pk = cyc ? t.pkp : (fam == 2) ? t.pkT : t.pk1;
+    const int pw = cyc ? s.Tg + s.nf * LU : LTC + 4 * s.hw;
+    constexpr int PK = 5;
+    double pv[PK];
+#pragma unroll
+    for (int v = 0; v < PK; ++v) {
+        const int q = (int)threadIdx.x + v * WG;
+        pv[v] = pk[q < pw ? q : 0];
     }
+    switch (fam) {
+    case 0: line_stage<0>(a, s, L.T, S); break;
+    case 1: line_stage<1>(a, s, L.T, S); break;
+    case 2: line_stage<2>(a, s, L.T, S); break;
+    case 3: line_stage<3>(a, s, L.T, S); break;
+    case 4: line_stage<4>(a, s, L.T, S); break;
+    default: line_stage<5>(a, s, L.T, S); break;
+    }
+#pragma unroll
+    for (int v = 0; v < PK; ++v) {
+        const int q = (int)threadIdx.x + v * WG;
+        if (q < pw) S[q] = pv[v];
+    }
+    for (int q = (int)threadIdx.x + PK * WG; q < pw; q += WG) S[q] = pk[q];
+    __syncthreads();
+    if (cyc) line_finish<true>(a, L, fam, s, out, S);
+    else line_finish<false>(a, L, fam, s, out, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -463,8 +589,8 @@ __device__ void ptdma_scan(const CompactArgs &a, int i)
     double rn = Rn - sum;
     rn = rn - fB * rm2;
     rn = rn - fC * rn1;
-    const double yn = div_rb(rn, bbt[n], rbb[n]);
-    const double yn1 = div_rb(rn1 - cc[n - 1] * yn, bbt[n - 1], rbb[n - 1]);
+    const double yn = line_div(rn, bbt[n], rbb[n]);
+    const double yn1 = line_div(rn1 - cc[n - 1] * yn, bbt[n - 1], rbb[n - 1]);
     // back substitution: y_j = p_j + q_j y_{j+1}, p_j = (rm_j - a_j yn)/b_j
     double ba = 0.0, bb = 1.0;
 #pragma unroll
@@ -931,26 +1057,37 @@ static int compact_launch(vv_run *r, int mask)
     a.tab_r1 = r->tab_r1; a.tab_rT = r->tab_rT; a.tab_p = r->tab_p;
     a.nr = r->nr; a.np = r->np; a.ld = r->ld; a.mask = mask;
     a.dri = 1.0 / r->dr; a.dpi = 1.0 / r->dp;
-    // tiles sized for 32 KB of LDS per workgroup
-    const int budget = 32768 / 8;
-    const int nP = r->nr | 1;
     CompactTiles t;
-    t.Tr = budget / nP;
-    if (t.Tr > 64) t.Tr = 64;
-    if (t.Tr < 1) t.Tr = 1;
-    t.Tp = budget / (r->np + 1);
-    if (t.Tp > 64) t.Tp = 64;
-    if (t.Tp < 1) t.Tp = 1;
-    // a workgroup holds at least one whole line: Tp = 1 needs np+1 words,
-    // Tr = 1 nP words, either of which can exceed the budget
-    t.rwords = std::max(budget, std::max(t.Tr * nP, t.Tp * (r->np + 1)));
-    // + the elimination tables: 4n words (r families, n <= nr), 6(np+2)+3 (phi)
-    const int twords = (4 * r->nr > 6 * (r->np + 2) + 3) ? 4 * r->nr : 6 * (r->np + 2) + 3;
-    // dynamic LDS is kept within 64 KB; larger tables stay in global memory
-    t.tab_lds = ((size_t)(t.rwords + twords) * 8 <= 65536) ? 1 : 0;
-    const size_t lds = (size_t)(t.rwords + (t.tab_lds ? twords : 0)) * 8;
+    t.pk1 = r->pk_r1; t.pkT = r->pk_rT; t.pkp = r->pk_p;
+    t.na = r->pk_na; t.nf = r->pk_nf;
+    const int Nr = r->nr - 1, Np = r->np - 1;   // rows of the longest line before its closing rows
+    t.tabw = LTC + std::max(4 * lheadb(Nr) * LU, 3 * lheadb(Np) * LU + (t.na + 1) * (LU + 1) + t.nf * LU);
+    // lanes per line: enough for the shortest chains while the chip has
+    // lanes to spare (2 wavefronts a SIMD), fewer above (less warm-up work
+    // per row), but always so many that a workgroup's lines fit in LDS
+    const int nbr = lblocks(Nr) - lheadb(Nr), nbp = lblocks(Np) - lheadb(Np);
+    int Pr = 1, Pp = 1;
+    while (Pr < 64 && line_mb(nbr, Pr) > 1) Pr *= 2;
+    while (Pp < 64 && line_mb(nbp, Pp) > 1) Pp *= 2;
+    auto waves = [&] { return 3.0 * (r->np + 1.0) * Pr / 64 + 3.0 * r->nr * Pp / 64; };
+    while (waves() > 2048 && (Pr > 4 || Pp > 4)) {
+        if (Pr > 4) Pr /= 2;
+        if (Pp > 4) Pp /= 2;
+    }
+    auto tile = [&](LineTile &L, int P, int N, int nb, int nx) {
+        const int room = (int)(65536 / 8) - t.tabw, pitch = lpitch(N, nx);
+        while (P < 64 && (WG / P) * pitch > room) P *= 2;
+        L.P = P;
+        L.lgP = 31 - __builtin_clz(P);
+        L.mb = line_mb(nb, P);
+        L.T = std::min(WG / P, 16);
+        while (L.T > 1 && L.T * pitch > room) L.T /= 2;
+        return L.T * pitch;
+    };
+    const int wr = tile(t.r, Pr, Nr, nbr, 1), wp = tile(t.p, Pp, Np, nbp, 3);
+    const size_t lds = (size_t)(t.tabw + std::max(wr, wp)) * 8;
     if (lds > 160 * 1024) { set_error("compact-scheme line longer than the LDS of a CU holds"); return VV_EINVAL; }
-    const int gr = nblk(r->np + 1, t.Tr), gp = nblk(r->nr, t.Tp);
+    const int gr = nblk(r->np + 1, t.r.T), gp = nblk(r->nr, t.p.T);
     dim3 grid(gr > gp ? gr : gp, 6);
     // the scan form: a wavefront per line, lines of up to 64 SM_MAX rows
     const bool scan = r->cfg.lines == VV_LINES_SCAN && r->nr <= 64 * SM_MAX && r->np - 1 <= 64 * SM_MAX;

@@ -202,6 +202,11 @@ struct vv_run {
     double *tab_rT = nullptr;   // tdma with closure rows, n = nr
     double *tab_p = nullptr;    // ptdma 1-4-1, n = np+1: f1 | f2 | a | b | c | fA fB fC | 1/b
 
+    // the same tables as the chunked line kernel holds them in LDS, behind
+    // them in the same allocations, and the blocks of ptdma's a and f2 that are not all zero
+    const double *pk_r1 = nullptr, *pk_rT = nullptr, *pk_p = nullptr;
+    int pk_na = 0, pk_nf = 0;
+
     // multigrid
     vv::MgBatchDev mg{};
     double *mg_pool = nullptr;

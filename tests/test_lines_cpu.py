@@ -1,0 +1,48 @@
+"""The chunked line recurrences' arithmetic, on the CPU.
+
+The settled pivot's division is two operations, fma(x, LF, x * LFL)
+(csrc/vv_lines.h); it must give the correctly rounded quotient for every x.
+"""
+from __future__ import annotations
+
+import math
+from fractions import Fraction as F
+
+import numpy as np
+
+LB = float.fromhex("0x1.ddb3d742c2655p+1")
+LF = float.fromhex("0x1.126145e9ecd56p-2")
+LFL = float.fromhex("0x1.49c290bb649bfp-56")
+
+
+def settled_div(x: float) -> float:
+    return float(F(x) * F(LF) + F(float(F(x) * F(LFL))))
+
+
+def test_settled_rows_are_the_eliminations():
+    f, b = 0.0, 4.0
+    for _ in range(16):
+        f, b = 1.0 / b, 4.0 - 1.0 / b
+    assert (f, b) == (LF, LB)
+    assert LF == 1.0 / LB and LFL == float(F(1) / F(LB) - F(LF))
+
+
+def test_settled_division_is_correctly_rounded():
+    """The two-operation quotient is off by under 2^-106.3 of it before its
+    rounding, so it can only round wrong where X 2^k = d (mod B) with |d| <= 1
+    for the 53-bit significands X of x and B of the pivot: every X with
+    |d| <= 64 is tried."""
+    B = int(math.frexp(LB)[0] * 2 ** 53)
+    assert math.gcd(B, 2) == 1
+    tried = 0
+    for k in (53, 54):
+        inv = pow(pow(2, k, B), -1, B)
+        for d in range(-64, 65):
+            X = d * inv % B
+            if d and 2 ** 52 <= X < 2 ** 53:
+                tried += 1
+                assert settled_div(float(X)) == float(F(X) / F(LB)), (k, d, X)
+    assert tried > 50
+    rng = np.random.default_rng(5)
+    for x in rng.standard_normal(5000) * 2.0 ** rng.integers(-60, 60, 5000):
+        assert settled_div(float(x)) == float(F(float(x)) / F(LB))
