@@ -1,6 +1,7 @@
 // vv3_internal.h -- shared declarations of the 3D step (not part of the ABI).
 #pragma once
 
+#include "vv_fft.h"
 #include "vv_internal.h"
 
 #include "../../include/vvmi3.h"
@@ -45,8 +46,10 @@ struct Poisson3 {
     double *T = nullptr;     // np x mmax: z spectra, (i, l) with l fastest
     double *cp = nullptr;    // nm x mmax: elimination factors of the r solves
     double *S2 = nullptr, *T2 = nullptr, *cp2 = nullptr;   // a second set (a solve beside another), or none
-    double *tw = nullptr;    // np/2 complex (cos, -sin)(2 pi t/np): FFT twiddles (np a power of two)
-    bool fft = false;        // phi transforms by FFT (np a power of two, 8..4096) instead of GEMM
+    double *tw = nullptr;    // the FFT's tables (vv_fft.h)
+    vv::MrTables mr;         // phi transforms' plan
+    vv::MrPlan plan{};       // with its device pointers
+    bool fft = false;        // phi transforms by FFT (even np, 8..4096) instead of GEMM
 };
 
 // Host-side pieces, exposed so that they can be checked without a GPU.

@@ -32,9 +32,10 @@ namespace vv3 {
 namespace {
 
 using vv::bitrev;
-using vv::fft_combine;
 using vv::fft_pairs;
-using vv::fft_stages;
+using vv::mr_pos;
+using vv::mr_transform;
+using vv::MrPlan;
 using vv::mr_pos;
 using vv::gemm_f64;
 
@@ -97,40 +98,48 @@ struct PhiInv {
 };
 
 // ---------------------------------------------------------------- phi FFT
-// For even np (8 <= np <= 4096) the phi transforms are FFTs in LDS: radix 2
-// for a power of two (R = 0), otherwise np = b 2^bits with b odd, b radix-2
-// sub-lines per line and the in-place combination of fft_combine (R outputs
-// per thread).  Two real
-// lines (consecutive i at one j) share one complex transform, z = a + i b;
-// Z_m and Z_{np-m} separate them afterwards.  A workgroup holds LP such pairs
-// (LP np complex values, at most 64 KB); k' = k mod np indexes the line, so
-// k = np is position 0.  Stage s pairs positions p and p + h (h = 2^s) with
-// the twiddle e^{-i 2 pi (p mod h)/(2h)} (conjugated for the inverse).
+// For even np (8 <= np <= 4096) the phi transforms are FFTs in LDS (the
+// mixed-radix stages of vv_fft.h, R as there).  Two real lines (consecutive i
+// at one j) share one complex transform, z = a + i b; Z_m and Z_{np-m}
+// separate them afterwards.  A workgroup holds LP such pairs (LP np complex
+// values, at most 64 KB; LP a power of two up to 128, so that a thread stays
+// on one line and has B of its points in flight); k' = k mod np indexes the
+// line, so k = np is position 0.  At np = 150 (91 x 75 lines) 14.4 + 13.2 us a
+// call, where one combination over the odd factor 75 took 99 + 96; at np = 256
+// (128 x 128) 33.9 + 30.9 beside the other stream's kernels, 36.6 + 40.3 with
+// one point in flight per thread.
 
 // forward: S[m][u] = sum_k rhs(i,j,k) cos(2 pi m k/np) (m = 0..np/2) and
 // S[np/2+m][u] = sum_k rhs(i,j,k) sin(...) (0 < m < np/2), u = (j-1) i1 + (i-1)
 template <int R>
-__global__ void __launch_bounds__(256) k3_fft_fwd(const double *rhs, double *S, const double2 *tw, int np, int bits,
-                                                   int b, int LP, int i1, int j1, int ldi, int ldj, int mt)
+__global__ void __launch_bounds__(256) k3_fft_fwd(const double *rhs, double *S, MrPlan F, int LP, int i1, int j1,
+                                                   int ldi, int ldj, int mt)
 {
     extern __shared__ double2 z[];
-    const int j = blockIdx.y, ib = blockIdx.x * 2 * LP, nl = 2 * LP;
-    for (int e = threadIdx.x; e < nl * np; e += blockDim.x) {
-        const int l = e % nl, kq = e / nl;
-        const int i = ib + l, k = (kq == 0) ? np : kq;
-        const double v = (i < i1) ? rhs[((size_t)k * ldj + (size_t)(j + 1)) * ldi + (size_t)(i + 1)] : 0.0;
-        const int pos = R ? mr_pos(kq, b, np / b, bits) : (int)bitrev(kq, bits);
-        double *zz = reinterpret_cast<double *>(&z[(l >> 1) * np + pos]);
-        zz[l & 1] = v;
+    constexpr int B = 8;
+    const int np = F.n, j = blockIdx.y, nl = 2 * LP;
+    const int l = (int)threadIdx.x & (nl - 1), kst = (int)blockDim.x / nl, i = blockIdx.x * nl + l;
+    const size_t pl = (size_t)ldj * ldi;
+    const double *row = rhs + (size_t)(j + 1) * ldi + (size_t)(i + 1);
+    double *zl = reinterpret_cast<double *>(z + (l >> 1) * np) + (l & 1);
+    for (int k0 = (int)threadIdx.x / nl; k0 < np; k0 += B * kst) {
+        double x[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const int kq = k0 + u * kst, k = (kq == 0) ? np : kq;
+            x[u] = (i < i1 && kq < np) ? row[(size_t)k * pl] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const int kq = k0 + u * kst;
+            if (kq < np) zl[2 * mr_pos<R>(F, kq)] = x[u];
+        }
     }
     __syncthreads();
-    fft_stages<false>(z, tw, np / b, bits, LP * b);
-    if (R) fft_combine<false, R ? R : 1>(z, tw + (np / b) / 2, np, np / b, b, LP);
+    mr_transform<false, R>(z, F, F.tw, F.twc, LP);
+    if (i >= i1) return;
     const int half = np >> 1;
-    for (int e = threadIdx.x; e < nl * (half + 1); e += blockDim.x) {
-        const int l = e % nl, m = e / nl;
-        const int i = ib + l;
-        if (i >= i1) continue;
+    for (int m = (int)threadIdx.x / nl; m <= half; m += kst) {
         const double2 zm = z[(l >> 1) * np + m], zn = z[(l >> 1) * np + (m == 0 ? 0 : np - m)];
         // A = (Z_m + conj Z_{np-m})/2, B = (Z_m - conj Z_{np-m})/(2i)
         double re, im;
@@ -145,36 +154,44 @@ __global__ void __launch_bounds__(256) k3_fft_fwd(const double *rhs, double *S, 
 // inverse: psi(i,j,k) = (1/np) sum_m w_m (C_m cos + S_m sin), k = 1..np, and
 // k = 0 copied from k = np
 template <int R>
-__global__ void __launch_bounds__(256) k3_fft_inv(const double *S, double *psi, const double2 *tw, int np, int bits,
-                                                   int b, int LP, int i1, int j1, int ldi, int ldj, int mt)
+__global__ void __launch_bounds__(256) k3_fft_inv(const double *S, double *psi, MrPlan F, int LP, int i1, int j1,
+                                                   int ldi, int ldj, int mt)
 {
     extern __shared__ double2 z[];
-    const int j = blockIdx.y, ib = blockIdx.x * 2 * LP, nl = 2 * LP, half = np >> 1;
-    // Z_m = X_m + i Y_m with X_m = C_m - i S_m (m <= np/2), X_{np-m} = conj X_m
-    for (int e = threadIdx.x; e < LP * np; e += blockDim.x) {
-        const int pr = e % LP, m = e / LP;   // neighbouring threads: neighbouring lines, one spectral row
-        const int mm = (m <= half) ? m : np - m;
-        const double sg = (m <= half) ? -1.0 : 1.0;   // imaginary part of X_m is sg * S_mm
-        double xr = 0, xi = 0, yr = 0, yi = 0;
-        for (int h2 = 0; h2 < 2; ++h2) {
-            const int i = ib + 2 * pr + h2;
-            if (i >= i1) continue;
-            const size_t u = (size_t)j * i1 + i;
-            const double c = S[(size_t)mm * mt + u];
-            const double sn = (mm > 0 && mm < half) ? S[(size_t)(half + mm) * mt + u] : 0.0;
-            if (h2 == 0) { xr = c; xi = sg * sn; } else { yr = c; yi = sg * sn; }
+    constexpr int B = 4;
+    const int np = F.n, j = blockIdx.y, nl = 2 * LP, ib = blockIdx.x * nl, half = np >> 1;
+    // Z_m = X_m + i Y_m with X_m = C_m - i S_m (m <= np/2), Z_{np-m} = conj X_m + i conj Y_m
+    {
+        const int pr = (int)threadIdx.x & (LP - 1), mst = (int)blockDim.x / LP, i = ib + 2 * pr;
+        const double *Sl = S + (size_t)j * i1 + i;
+        for (int m0 = (int)threadIdx.x / LP; m0 <= half; m0 += B * mst) {
+            double c[B][2], sn[B][2];
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                const int m = m0 + u * mst;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool in = m <= half && i + h < i1;
+                    c[u][h] = in ? Sl[(size_t)m * mt + h] : 0.0;
+                    sn[u][h] = (in && m > 0 && m < half) ? Sl[(size_t)(half + m) * mt + h] : 0.0;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                const int m = m0 + u * mst;
+                if (m > half) break;
+                z[pr * np + mr_pos<R>(F, m)] = make_double2(c[u][0] + sn[u][1], c[u][1] - sn[u][0]);
+                if (m > 0 && m < half)
+                    z[pr * np + mr_pos<R>(F, np - m)] = make_double2(c[u][0] - sn[u][1], sn[u][0] + c[u][1]);
+            }
         }
-        const int pos = R ? mr_pos(m, b, np / b, bits) : (int)bitrev(m, bits);
-        z[pr * np + pos] = make_double2(xr - yi, xi + yr);
     }
     __syncthreads();
-    fft_stages<true>(z, tw, np / b, bits, LP * b);
-    if (R) fft_combine<true, R ? R : 1>(z, tw + (np / b) / 2, np, np / b, b, LP);
+    mr_transform<true, R>(z, F, F.tw, F.twc, LP);
     const double inv = 1.0 / np;
-    for (int e = threadIdx.x; e < nl * np; e += blockDim.x) {
-        const int l = e % nl, kq = e / nl;
-        const int i = ib + l;
-        if (i >= i1) continue;
+    const int l = (int)threadIdx.x & (nl - 1), i = ib + l;
+    if (i >= i1) return;
+    for (int kq = (int)threadIdx.x / nl; kq < np; kq += (int)blockDim.x / nl) {
         const double2 v = z[(l >> 1) * np + kq];
         const double x = ((l & 1) ? v.y : v.x) * inv;
         const size_t off = (size_t)(j + 1) * ldi + (size_t)(i + 1);
@@ -626,21 +643,10 @@ int poisson3_setup(Poisson3 &P, const Geo &g)
         VV_HIP(upload(&P.Wi, Wi));
     }
     if (P.fft) {
-        // (cos, -sin)(2 pi t/n1), t < n1/2, for the n1 = 2^bits point
-        // radix-2 sub-lines, then (np not a power of two) (cos, -sin)(2 pi t/np),
-        // t < np, for the mixed-radix combination
-        const int n1 = np & -np;
-        std::vector<double> tw;
-        for (int t = 0; t < n1 / 2; ++t) {
-            tw.push_back(std::cos(2.0 * pi * t / n1));
-            tw.push_back(-std::sin(2.0 * pi * t / n1));
-        }
-        if (n1 != np)
-            for (int t = 0; t < np; ++t) {
-                tw.push_back(std::cos(2.0 * pi * t / np));
-                tw.push_back(-std::sin(2.0 * pi * t / np));
-            }
-        VV_HIP(upload(&P.tw, tw));
+        P.mr = vv::mr_tables(np);
+        VV_HIP(hipMalloc(&P.tw, P.mr.bytes()));
+        VV_HIP(vv::mr_upload(P.mr, P.tw));
+        P.plan = P.mr.at(P.tw);
     }
     VV_HIP(upload(&P.lphi, lphi));
     const double hhz = g.dz * g.dz, hhp = g.dp * g.dp;
@@ -708,25 +714,23 @@ int poisson3_launch(const Poisson3 &P, const Geo &g, int which, double *psi, dou
     const int nm = P.nm, np = P.np, i1 = O.i1, j1 = O.j1, mt = O.m;
     hipLaunchKernelGGL(k3_psi_pre, dim3((unsigned)((g.ldi * g.ldj + 255) / 256), np + 1), dim3(256), 0, s, g, which,
                        i1, j1, psi, psip);
-    // LP line pairs per workgroup, few enough for about 256 workgroups
-    const int bits = P.fft ? __builtin_ctz((unsigned)np) : 0;
-    const int LP = std::max(1, std::min(fft_pairs(np), (i1 * j1) / 512));
-    const int fodd = np >> bits;                      // odd factor of np (1: radix 2 only)
-    // registers of the mixed-radix combination: LP np <= R 256
-    const int fR = (fodd == 1) ? 0 : (LP * np <= 8 * 256) ? 8 : 32;
+    // LP line pairs per workgroup (a power of two), few enough for about 256
+    // workgroups
+    const int LP = P.fft ? vv::pow2_floor(std::max(1, std::min({fft_pairs(np), (i1 * j1) / 512, 128}))) : 1;
+    const int R = P.fft ? vv::mr_r(P.mr, LP) : 0;
     if (P.fft && LP * np > 32 * 256) { vv::set_error("phi FFT line longer than 8192 points"); return VV_EINVAL; }
     const dim3 fgrid((unsigned)((i1 + 2 * LP - 1) / (2 * LP)), (unsigned)j1);
     const size_t flds = (size_t)LP * np * sizeof(double2);
-    const double2 *tw = (const double2 *)P.tw;
-    if (P.fft && fR == 0)
-        hipLaunchKernelGGL(k3_fft_fwd<0>, fgrid, dim3(256), flds, s, rhs, S, tw, np, bits, 1, LP, i1, j1, g.ldi,
-                           g.ldj, mt);
-    else if (P.fft && fR == 8)
-        hipLaunchKernelGGL(k3_fft_fwd<8>, fgrid, dim3(256), flds, s, rhs, S, tw, np, bits, fodd, LP, i1, j1, g.ldi,
-                           g.ldj, mt);
-    else if (P.fft)
-        hipLaunchKernelGGL(k3_fft_fwd<32>, fgrid, dim3(256), flds, s, rhs, S, tw, np, bits, fodd, LP, i1, j1,
-                           g.ldi, g.ldj, mt);
+    auto fwd = [&](auto k) {
+        hipLaunchKernelGGL(k, fgrid, dim3(256), flds, s, rhs, S, P.plan, LP, i1, j1, g.ldi, g.ldj, mt);
+    };
+    auto inv = [&](auto k) {
+        hipLaunchKernelGGL(k, fgrid, dim3(256), flds, s, (const double *)S, psi, P.plan, LP, i1, j1, g.ldi, g.ldj, mt);
+    };
+    if (P.fft && R == 0) fwd(k3_fft_fwd<0>);
+    else if (P.fft && R == 1) fwd(k3_fft_fwd<1>);
+    else if (P.fft && R == 8) fwd(k3_fft_fwd<8>);
+    else if (P.fft) fwd(k3_fft_fwd<32>);
     else
         gemm_f64<true, false>(PhiFwd{P.W, np, mt, np, rhs, S, i1, g.ldi, g.ldj}, 1, s);
     if (O.zsplit) vv::zsplit_fwd(O.Vinv, S, T, i1, j1, np, s);
@@ -735,15 +739,10 @@ int poisson3_launch(const Poisson3 &P, const Geo &g, int which, double *psi, dou
                        (const double *)O.rt, (const double *)O.lz, (const double *)P.lphi, i1, j1, np, O.e1, O.en);
     if (O.zsplit) vv::zsplit_inv(O.V, T, S, i1, j1, np, s);
     else gemm_f64<true, true>(ZInv{O.V, j1, i1, j1, T, S, mt}, np, s);
-    if (P.fft && fR == 0)
-        hipLaunchKernelGGL(k3_fft_inv<0>, fgrid, dim3(256), flds, s, (const double *)S, psi, tw, np, bits, 1, LP, i1,
-                           j1, g.ldi, g.ldj, mt);
-    else if (P.fft && fR == 8)
-        hipLaunchKernelGGL(k3_fft_inv<8>, fgrid, dim3(256), flds, s, (const double *)S, psi, tw, np, bits, fodd, LP,
-                           i1, j1, g.ldi, g.ldj, mt);
-    else if (P.fft)
-        hipLaunchKernelGGL(k3_fft_inv<32>, fgrid, dim3(256), flds, s, (const double *)S, psi, tw, np, bits, fodd,
-                           LP, i1, j1, g.ldi, g.ldj, mt);
+    if (P.fft && R == 0) inv(k3_fft_inv<0>);
+    else if (P.fft && R == 1) inv(k3_fft_inv<1>);
+    else if (P.fft && R == 8) inv(k3_fft_inv<8>);
+    else if (P.fft) inv(k3_fft_inv<32>);
     else
         gemm_f64<true, false>(PhiInv{P.Wi, np, mt, np, S, psi, i1, g.ldi, g.ldj}, 1, s);
     VV_HIP(hipGetLastError());

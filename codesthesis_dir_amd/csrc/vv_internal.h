@@ -10,6 +10,8 @@
 
 #include "../../include/vvmi.h"
 
+#include "vv_fft.h"
+
 namespace vv {
 
 // ----------------------------------------------------------------- errors
@@ -71,10 +73,8 @@ struct MgLevelDev {
     size_t tabsz;
     double *xm;
     const double *twid;
-    // direct level with FFTs (fft_cols): the twiddles (cos, -sin)(2 pi t/n1),
-    // t < n1/2, of its 2^bits = n1 point radix-2 sub-lines and, when ncol is
-    // not a power of two, (cos, -sin)(2 pi t/ncol), t < ncol, of the
-    // mixed-radix combination, in a buffer of their own; null elsewhere
+    // direct level with FFTs (fft_cols): the plan's tables (vv_fft.h), in a
+    // buffer of their own; null elsewhere
     const double *ftw;
     // mixed precision (VV_PREC_MIXED): the level's FP32 iterate buffers,
     // right-hand side, black-line changes and PCR tables (smoothed levels);
@@ -210,7 +210,9 @@ struct vv_run {
     // multigrid
     vv::MgBatchDev mg{};
     double *mg_pool = nullptr;
-    double *mg_ftw = nullptr;   // FFT twiddles of the direct level (see MgLevelDev::ftw)
+    double *mg_ftw = nullptr;   // FFT tables of the direct level (see MgLevelDev::ftw)
+    vv::MrTables mg_mr;         // its plan
+    vv::MrPlan mg_plan{};       // with its device pointers
     float *mg_pool32 = nullptr; // FP32 hierarchy of the mixed-precision V-cycle
     double *mg_hist = nullptr;  // [2][MG_HIST] relative residual after each cycle of the last solve
     // solver state, one device block read back with a single copy:

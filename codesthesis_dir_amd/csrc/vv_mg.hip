@@ -57,7 +57,6 @@ struct KLevT {
     T *u, *uo, *f;          // current iterate, output buffer of a sweep, rhs
     const T *lu;
     const double *twid;
-    const double2 *ftw;     // direct level: FFT twiddles (null: dense transforms)
     double *xm;
     T *dlt;                 // black-line changes of the last pre-sweep (level L-1)
     double cphi;
@@ -623,9 +622,7 @@ __global__ void __launch_bounds__(1024) k_mg_modes(KArgs a)
 }
 
 // The direct level's transforms as FFTs in LDS (C even, 8 <= C <= 8192):
-// radix 2 when C is a power of two (R = 0); otherwise C = b 2^bits with b odd,
-// b radix-2 sub-lines per line and the in-place combination of fft_combine
-// (R outputs per thread).  A workgroup transforms LP pairs of lines (rows i
+// the mixed-radix stages of vv_fft.h, R as there.  A workgroup transforms LP pairs of lines (rows i
 // of the level, two real lines per complex line), the problem is blockIdx.y.  The
 // projection writes the real lines of the modes, ml = 0 (m = 0), 2m-1 and 2m
 // (cos and sin of 0 < m < C/2), C-1 (m = C/2), i.e. X[ml][i] = sum_k W[ml][k]
@@ -634,7 +631,7 @@ __global__ void __launch_bounds__(1024) k_mg_modes(KArgs a)
 // (1/C) sum_m w_m (C_m cos + S_m sin) (w = 1 at m = 0, C/2, else 2) and
 // stores it into, or on refinement adds it to, the level's iterate.
 template <int R>
-__global__ void __launch_bounds__(256) k_mg_fft_fwd(KArgs a, int bits, int b, int LP)
+__global__ void __launch_bounds__(256) k_mg_fft_fwd(KArgs a, MrPlan F, int LP)
 {
     extern __shared__ double2 z[];
     const int p = blockIdx.y;
@@ -644,22 +641,31 @@ __global__ void __launch_bounds__(256) k_mg_fft_fwd(KArgs a, int bits, int b, in
     const int ib = blockIdx.x * nl;
     if (ib >= n || a.done[p]) return;   // uniform over the workgroup
     const bool from_res = a.lev0 && a.cycles[p] > 0;
-    for (int e = threadIdx.x; e < nl * C; e += blockDim.x) {
-        const int l = e % nl, k = e / nl;
-        const int i = ib + l;
-        double v = 0.0;
-        if (i < n) v = from_res ? resid_at(P, L, i, k) : L.f[(size_t)k * n + i];
-        const int pos = R ? mr_pos(k, b, C / b, bits) : (int)bitrev(k, bits);
-        double *zz = reinterpret_cast<double *>(&z[(l >> 1) * C + pos]);
-        zz[l & 1] = v;
+    // a thread stays on one line (nl divides the workgroup), B points in flight
+    constexpr int B = 8;
+    const int l = (int)threadIdx.x & (nl - 1), kst = (int)blockDim.x / nl, i = ib + l;
+    double *zl = reinterpret_cast<double *>(z + (l >> 1) * C) + (l & 1);
+    if (from_res) {
+        for (int k = (int)threadIdx.x / nl; k < C; k += kst) zl[2 * mr_pos<R>(F, k)] = i < n ? resid_at(P, L, i, k) : 0.0;
+    } else {
+        for (int k0 = (int)threadIdx.x / nl; k0 < C; k0 += B * kst) {
+            double x[B];
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                const int k = k0 + u * kst;
+                x[u] = (i < n && k < C) ? L.f[(size_t)k * n + i] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                const int k = k0 + u * kst;
+                if (k < C) zl[2 * mr_pos<R>(F, k)] = x[u];
+            }
+        }
     }
     __syncthreads();
-    fft_stages<false>(z, L.ftw, C / b, bits, LP * b);
-    if (R) fft_combine<false, R ? R : 1>(z, L.ftw + (C / b) / 2, C, C / b, b, LP);
-    for (int e = threadIdx.x; e < nl * (half + 1); e += blockDim.x) {
-        const int l = e % nl, m = e / nl;
-        const int i = ib + l;
-        if (i >= n) continue;
+    mr_transform<false, R>(z, F, F.tw, F.twc, LP);
+    if (i >= n) return;
+    for (int m = (int)threadIdx.x / nl; m <= half; m += kst) {
         const double2 zm = z[(l >> 1) * C + m], zn = z[(l >> 1) * C + (m == 0 ? 0 : C - m)];
         // A = (Z_m + conj Z_{C-m})/2, B = (Z_m - conj Z_{C-m})/(2i)
         double re, im;
@@ -677,7 +683,7 @@ __global__ void __launch_bounds__(256) k_mg_fft_fwd(KArgs a, int bits, int b, in
 }
 
 template <int R>
-__global__ void __launch_bounds__(256) k_mg_fft_inv(KArgs a, int bits, int b, int LP)
+__global__ void __launch_bounds__(256) k_mg_fft_inv(KArgs a, MrPlan F, int LP)
 {
     extern __shared__ double2 z[];
     const int p = blockIdx.y;
@@ -686,38 +692,40 @@ __global__ void __launch_bounds__(256) k_mg_fft_inv(KArgs a, int bits, int b, in
     const int n = P.n, C = L.ncol, half = C >> 1, nl = 2 * LP;
     const int ib = blockIdx.x * nl;
     if (ib >= n || a.done[p]) return;   // uniform over the workgroup
-    // Z_m = X_m + i Y_m of the pair, X_m = C_m - i S_m (m <= C/2), X_{C-m} = conj X_m
-    for (int e = threadIdx.x; e < LP * C; e += blockDim.x) {
-        const int pr = e % LP, m = e / LP;
-        const int mm = (m <= half) ? m : C - m;
-        const double sg = (m <= half) ? -1.0 : 1.0;
-        double xr = 0.0, xi = 0.0, yr = 0.0, yi = 0.0;
-        for (int h2 = 0; h2 < 2; ++h2) {
-            const int i = ib + 2 * pr + h2;
-            if (i >= n) continue;
-            double c, sn = 0.0;
-            if (mm == 0) {
-                c = L.xm[i];
-            } else if (mm == half) {
-                c = L.xm[(size_t)(C - 1) * n + i];
-            } else {
-                c = L.xm[(size_t)(2 * mm - 1) * n + i];
-                sn = L.xm[(size_t)(2 * mm) * n + i];
+    // Z_m = X_m + i Y_m of the pair, X_m = C_m - i S_m (m <= C/2), Z_{C-m} = conj X_m + i conj Y_m
+    constexpr int B = 4;
+    {
+        const int pr = (int)threadIdx.x & (LP - 1), mst = (int)blockDim.x / LP, i = ib + 2 * pr;
+        for (int m0 = (int)threadIdx.x / LP; m0 <= half; m0 += B * mst) {
+            double c[B][2], sn[B][2];
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                const int m = m0 + u * mst;
+                const size_t rc = (size_t)(m == 0 ? 0 : m == half ? C - 1 : 2 * m - 1) * n;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool in = m <= half && i + h < n;
+                    c[u][h] = in ? L.xm[rc + i + h] : 0.0;
+                    sn[u][h] = (in && m > 0 && m < half) ? L.xm[rc + n + i + h] : 0.0;
+                }
             }
-            if (h2 == 0) { xr = c; xi = sg * sn; } else { yr = c; yi = sg * sn; }
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                const int m = m0 + u * mst;
+                if (m > half) break;
+                z[pr * C + mr_pos<R>(F, m)] = make_double2(c[u][0] + sn[u][1], c[u][1] - sn[u][0]);
+                if (m > 0 && m < half)
+                    z[pr * C + mr_pos<R>(F, C - m)] = make_double2(c[u][0] - sn[u][1], sn[u][0] + c[u][1]);
+            }
         }
-        const int pos = R ? mr_pos(m, b, C / b, bits) : (int)bitrev(m, bits);
-        z[pr * C + pos] = make_double2(xr - yi, xi + yr);
     }
     __syncthreads();
-    fft_stages<true>(z, L.ftw, C / b, bits, LP * b);
-    if (R) fft_combine<true, R ? R : 1>(z, L.ftw + (C / b) / 2, C, C / b, b, LP);
+    mr_transform<true, R>(z, F, F.tw, F.twc, LP);
     const double inv = 1.0 / C;
     const bool store = !a.lev0 || a.cycles[p] == 0;
-    for (int e = threadIdx.x; e < nl * C; e += blockDim.x) {
-        const int l = e % nl, q = e / nl;
-        const int i = ib + l;
-        if (i >= n) continue;
+    const int l = (int)threadIdx.x & (nl - 1), i = ib + l;
+    if (i >= n) return;
+    for (int q = (int)threadIdx.x / nl; q < C; q += (int)blockDim.x / nl) {
         const double2 v = z[(l >> 1) * C + q];
         const double x = ((l & 1) ? v.y : v.x) * inv;
         double *d = L.u + cix(i, q, n);
@@ -1089,24 +1097,11 @@ int mg_build(vv_run *r)
     }
     {   // FFT twiddles of the direct level (both problems have its columns)
         const int C = r->mg.prob[0].lev[nlev - 1].ncol;
-        std::vector<double> tw;
         if (fft_cols(C)) {
-            // radix-2 twiddles of the n1 = 2^bits point sub-lines, then (C not
-            // a power of two) the C twiddles of the mixed-radix combination
-            const double pi = std::acos(-1.0);
-            const int n1 = C & -C;
-            for (int t = 0; t < n1 / 2; ++t) {
-                tw.push_back(std::cos(2.0 * pi * t / n1));
-                tw.push_back(-std::sin(2.0 * pi * t / n1));
-            }
-            if (n1 != C)
-                for (int t = 0; t < C; ++t) {
-                    tw.push_back(std::cos(2.0 * pi * t / C));
-                    tw.push_back(-std::sin(2.0 * pi * t / C));
-                }
-            VV_HIP(hipMalloc(&r->mg_ftw, tw.size() * sizeof(double)));
-            VV_HIP(hipMemcpyAsync(r->mg_ftw, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice,
-                                  r->stream));
+            r->mg_mr = mr_tables(C);
+            VV_HIP(hipMalloc(&r->mg_ftw, r->mg_mr.bytes()));
+            VV_HIP(mr_upload(r->mg_mr, r->mg_ftw));
+            r->mg_plan = r->mg_mr.at(r->mg_ftw);
             for (int p = 0; p < 2; ++p) r->mg.prob[p].lev[nlev - 1].ftw = r->mg_ftw;
         }
         VV_HIP(hipStreamSynchronize(r->stream));   // the host tables go out of scope
@@ -1139,7 +1134,6 @@ static KLev klev(const MgLevelDev &L, int cur)
     k.u = cur ? L.u2 : L.u;
     k.uo = cur ? L.u : L.u2;
     k.f = L.f; k.lu = L.lu; k.twid = L.twid; k.xm = L.xm; k.dlt = L.dlt;
-    k.ftw = reinterpret_cast<const double2 *>(L.ftw);
     k.cphi = L.cphi; k.ncol = L.ncol; k.nstep = L.nstep; k.tabsz = (int)L.tabsz;
     return k;
 }
@@ -1294,20 +1288,19 @@ static int enqueue_cycle(vv_run *r, int *check = nullptr)
         // against the dense transforms 1902 -> 2896 steps/s at 1025 x 513;
         // matrix-core GEMMs lose to both, their k loop being latency-bound)
         const bool fft = B.prob[0].lev[L].ftw != nullptr;
-        const int fbits = fft ? __builtin_ctz((unsigned)C) : 0;
-        const int fodd = C >> fbits;              // odd factor of C (1: radix 2 only)
-        const int LP = std::max(1, std::min(fft_pairs(C), n / 256));
+        const int LP = pow2_floor(std::max(1, std::min({fft_pairs(C), n / 256, 128})));
         const dim3 fg((unsigned)((n + 2 * LP - 1) / (2 * LP)), 2);
         const size_t flds = (size_t)LP * C * sizeof(double2);
-        // registers of the mixed-radix combination: LP C <= R 256
-        const int fR = (fodd == 1) ? 0 : (LP * C <= 8 * 256) ? 8 : 32;
+        const int R = fft ? mr_r(r->mg_mr, LP) : 0;
         if (fft && LP * C > 32 * 256) { set_error("FFT line longer than 8192 points"); return VV_EINVAL; }
+        auto launch = [&](auto k) { hipLaunchKernelGGL(k, fg, dim3(256), flds, r->stream, a, r->mg_plan, LP); };
         prof_begin(r, &pe);
         // projection (read the level, write the mode lines) and line solves
         // (read and write the mode lines)
-        if (fft && fR == 0) hipLaunchKernelGGL(k_mg_fft_fwd<0>, fg, dim3(256), flds, r->stream, a, fbits, 1, LP);
-        else if (fft && fR == 8) hipLaunchKernelGGL(k_mg_fft_fwd<8>, fg, dim3(256), flds, r->stream, a, fbits, fodd, LP);
-        else if (fft) hipLaunchKernelGGL(k_mg_fft_fwd<32>, fg, dim3(256), flds, r->stream, a, fbits, fodd, LP);
+        if (fft && R == 0) launch(k_mg_fft_fwd<0>);
+        else if (fft && R == 1) launch(k_mg_fft_fwd<1>);
+        else if (fft && R == 8) launch(k_mg_fft_fwd<8>);
+        else if (fft) launch(k_mg_fft_fwd<32>);
         else hipLaunchKernelGGL(k_mg_dft<0>, gd, dim3(256), 0, r->stream, a);
         if (two)
             hipLaunchKernelGGL(k_mg_modes<2>, dim3(C / 2 + 1, 2), dim3(zt), 0, r->stream, a);
@@ -1315,9 +1308,10 @@ static int enqueue_cycle(vv_run *r, int *check = nullptr)
             hipLaunchKernelGGL(k_mg_modes<1>, dim3(C / 2 + 1, 2), dim3(zt), 0, r->stream, a);
         prof_end(r, VV_K_DIRECT, pe, 32.0 * ntot * C);
         prof_begin(r, &pe);
-        if (fft && fR == 0) hipLaunchKernelGGL(k_mg_fft_inv<0>, fg, dim3(256), flds, r->stream, a, fbits, 1, LP);
-        else if (fft && fR == 8) hipLaunchKernelGGL(k_mg_fft_inv<8>, fg, dim3(256), flds, r->stream, a, fbits, fodd, LP);
-        else if (fft) hipLaunchKernelGGL(k_mg_fft_inv<32>, fg, dim3(256), flds, r->stream, a, fbits, fodd, LP);
+        if (fft && R == 0) launch(k_mg_fft_inv<0>);
+        else if (fft && R == 1) launch(k_mg_fft_inv<1>);
+        else if (fft && R == 8) launch(k_mg_fft_inv<8>);
+        else if (fft) launch(k_mg_fft_inv<32>);
         else hipLaunchKernelGGL(k_mg_dft<1>, gd, dim3(256), 0, r->stream, a);
         if (mixed) {   // the correction's FP32 copy for the prolongation
             for (int p = 0; p < 2; ++p) {

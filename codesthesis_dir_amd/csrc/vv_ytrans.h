@@ -7,16 +7,22 @@
 //            (faces), u = (j-1) i1 + (i-1), i = 1..i1, j = 1..mt/i1;
 //   inverse: psi(i, j, k) = sum_q w_q e_q(k) S[q'][u] on the same points,
 //            w_0 = 1/np, w_q = 2/np (cells), w_q = 2/np (faces).
-// np must be a power of two, 8..2048 (ytrans_fits).
+// np must be 8..2048 with no prime factor above 13 (ytrans_fits).  At np = 160
+// (32 x 32 lines) a transform takes 8.5 us, as a GEMM 16.5; at np = 100 (50 x 42)
+// 13 forward and 12 back, as GEMMs 17 and 9 + 4.
 #pragma once
+
+#include "vv_fft.h"
 
 #include <hip/hip_runtime.h>
 
 namespace vvt {
 
 struct YTrans {
-    int np = 0, ldi = 0, ldj = 0, bits = 0, lp = 0;
-    double2 *tw = nullptr;   // (cos, -sin)(2 pi t/(2 np)), t < np, then (cos, sin)(pi q/(2 np)), q < np
+    int np = 0, ldi = 0, ldj = 0, lp = 0;
+    void *tab = nullptr;     // the plan's tables (vv_fft.h), then cq
+    vv::MrPlan plan{};       // of 2 np points
+    double2 *cq = nullptr;   // (cos, sin)(pi q/(2 np)), q < np
 };
 
 bool ytrans_fits(int np);

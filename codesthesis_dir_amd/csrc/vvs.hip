@@ -20,7 +20,7 @@
 // difference with zero-flux faces (w, u: eigenvectors cos(m pi (k-1/2)/np),
 // m = 0..np-1) or with zero values on the faces (v: sin(m pi k/np),
 // m = 1..np-1), both with eigenvalues 2 cos(m pi/np) - 2, so a solve is
-//   1. the phi transform: by FFT in LDS for np a power of two (8..2048, the
+//   1. the phi transform: by FFT in LDS for np with no prime above 13 (8..2048, the
 //      tank's y transforms, vv_ytrans.h), else a GEMM with the eigenvector
 //      table,
 //   2. the eigenbasis of the z rows (a batched GEMM),
@@ -117,7 +117,7 @@ struct SPoisson {
     SOp op[3];
     double *S = nullptr, *T = nullptr, *cp = nullptr;
     double *S2 = nullptr, *T2 = nullptr, *cp2 = nullptr;   // a second set: v's solve beside w's and u's
-    bool fft = false;     // phi transforms by FFT (np a power of two, 8..2048) instead of the W / Wi GEMMs
+    bool fft = false;     // phi transforms by FFT (ytrans_fits) instead of the W / Wi GEMMs
     vvt::YTrans yt;
 };
 

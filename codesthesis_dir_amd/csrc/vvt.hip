@@ -13,8 +13,8 @@
 // Poisson: each operator L = D_y + D_z + D_x (Cartesian, constant rows) is
 // solved exactly: its y rows have cosine modes (u, w: mirrored at the
 // stress-free side walls) or sine modes (v: zero there), applied by FFTs in
-// LDS when np is a power of two (k_t_yfft_*) and as FP64 matrix-core GEMMs
-// otherwise; the z rows are diagonalised once (the eigenbasis of
+// LDS when np has no prime factor above 13 (k_t_yfft_*) and as FP64
+// matrix-core GEMMs otherwise; the z rows are diagonalised once (the eigenbasis of
 // rot3dmg.f's z rows, shared with the annulus solver); what remains per
 // (y mode, z eigenvalue) is one banded system along x, eliminated by one
 // thread (Thomas, the closure rows' third coefficient folded in).
@@ -868,7 +868,7 @@ __global__ void __launch_bounds__(WG) k_t_ycombine(TGeo g, const double *EO, dou
     if (km != kk) psi[(unsigned)km * pl + off] = E - O;
 }
 
-// y modes by FFT (np = N a power of two): a mode transform of a line along y
+// y modes by FFT (2N, N = np, with no prime above 13): a mode transform of a line along y
 // is the 2N-point DFT of its extension -- the cells' lines (u, w: modes
 // cos(pi q (k - 1/2)/N), mirrored at the side walls) even about the walls,
 // y_j = x_{j+1}, y_{2N-1-j} = x_{j+1}, whose DFT is 2 e^{i pi q/(2N)} S_q;
@@ -880,15 +880,24 @@ __global__ void __launch_bounds__(WG) k_t_ycombine(TGeo g, const double *EO, dou
 // inverse: the cells' DCT-III by the inverse DFT (times 1/(2N)) of the
 // conjugate-symmetric spectrum 2 e^{i pi q/(2N)} C_q, which is
 // sum_q C_q cos(pi q (k - 1/2)/N) / norm_q (norm_0 = N, else N/2); the
-// faces' DST-I being its own inverse (times 2/N).  tw: (cos, -sin)(2 pi t/(2N)), t < N; cq: (cos,
-// sin)(pi q/(2N)), q < N.
-using vv::bitrev;
-using vv::fft_stages;
+// faces' DST-I being its own inverse (times 2/N).  F: the plan of 2N points
+// (R as in vv_fft.h, 0 or 1), its twiddles staged in LDS behind the lines;
+// cq: (cos, sin)(pi q/(2N)), q < N.
+using vv::mr_pos;
+using vv::mr_transform;
+using vv::MrPlan;
 
-template <bool FACES>
+// the plan's twiddles to LDS: n1/2 of the radix-2 stages, then (R) n
+template <int R>
+__device__ __forceinline__ void ytwiddles(const MrPlan &F, double2 *twl)
+{
+    const int n = (1 << F.bits) / 2 + (R ? F.n : 0);
+    for (int t = threadIdx.x; t < n; t += blockDim.x) twl[t] = F.tw[t];
+}
+
+template <bool FACES, int R>
 __global__ void __launch_bounds__(512) k_t_yfft_fwd(TGeo g, const double *__restrict__ rhs, double *__restrict__ S,
-                                                    const double2 *tw, const double2 *cq, int i1, int mt, int LP,
-                                                    int bits)
+                                                    MrPlan F, const double2 *cq, int i1, int mt, int LP)
 {
     extern __shared__ double2 z[];
     const int N = g.np, N2 = 2 * N, nl = 2 * LP;
@@ -896,11 +905,11 @@ __global__ void __launch_bounds__(512) k_t_yfft_fwd(TGeo g, const double *__rest
     const unsigned pl = (unsigned)(g.ldi * g.ldj);
     double *zd = reinterpret_cast<double *>(z);
     double2 *twl = z + LP * N2;   // the stages' twiddles, staged in LDS
-    for (int t = threadIdx.x; t < N; t += blockDim.x) twl[t] = tw[t];
+    ytwiddles<R>(F, twl);
     if (FACES)
         for (int e = threadIdx.x; e < nl * 2; e += blockDim.x) {   // y_0 = y_N = 0
             const int l = e % nl, w = e / nl;
-            zd[2 * ((l >> 1) * N2 + (int)bitrev((unsigned)(w * N), bits)) + (l & 1)] = 0.0;
+            zd[2 * ((l >> 1) * N2 + mr_pos<R>(F, w * N)) + (l & 1)] = 0.0;
         }
     const int K = FACES ? N - 1 : N;
     // element e = (k-1) nl + l: line l of plane k; the line's offset in the
@@ -927,16 +936,16 @@ __global__ void __launch_bounds__(512) k_t_yfft_fwd(TGeo g, const double *__rest
             const int k = k0 + u * kstep;
             if (k > K) break;
             if (FACES) {
-                zl[2 * (int)bitrev((unsigned)k, bits)] = x[u];
-                zl[2 * (int)bitrev((unsigned)(N2 - k), bits)] = -x[u];
+                zl[2 * mr_pos<R>(F, k)] = x[u];
+                zl[2 * mr_pos<R>(F, N2 - k)] = -x[u];
             } else {
-                zl[2 * (int)bitrev((unsigned)(k - 1), bits)] = x[u];
-                zl[2 * (int)bitrev((unsigned)(N2 - k), bits)] = x[u];
+                zl[2 * mr_pos<R>(F, k - 1)] = x[u];
+                zl[2 * mr_pos<R>(F, N2 - k)] = x[u];
             }
         }
     }
     __syncthreads();
-    fft_stages<false>(z, twl, N2, bits, LP);
+    mr_transform<false, R>(z, F, twl, twl + (1 << F.bits) / 2, LP);
     if (n >= mt) return;
     const double2 *zp = z + (l >> 1) * N2;
     for (int qi = (int)threadIdx.x / nl; qi < K; qi += kstep) {
@@ -957,10 +966,9 @@ __global__ void __launch_bounds__(512) k_t_yfft_fwd(TGeo g, const double *__rest
     }
 }
 
-template <bool FACES>
+template <bool FACES, int R>
 __global__ void __launch_bounds__(512) k_t_yfft_inv(TGeo g, const double *__restrict__ S, double *__restrict__ psi,
-                                                    const double2 *tw, const double2 *cq, int i1, int mt, int LP,
-                                                    int bits)
+                                                    MrPlan F, const double2 *cq, int i1, int mt, int LP)
 {
     extern __shared__ double2 z[];
     const int N = g.np, N2 = 2 * N, nl = 2 * LP;
@@ -968,11 +976,11 @@ __global__ void __launch_bounds__(512) k_t_yfft_inv(TGeo g, const double *__rest
     const unsigned pl = (unsigned)(g.ldi * g.ldj);
     double *zd = reinterpret_cast<double *>(z);
     double2 *twl = z + LP * N2;   // the stages' twiddles, staged in LDS
-    for (int t = threadIdx.x; t < N; t += blockDim.x) twl[t] = tw[t];
+    ytwiddles<R>(F, twl);
     if (FACES) {
         for (int e = threadIdx.x; e < nl * 2; e += blockDim.x) {
             const int l = e % nl, w = e / nl;
-            zd[2 * ((l >> 1) * N2 + (int)bitrev((unsigned)(w * N), bits)) + (l & 1)] = 0.0;
+            zd[2 * ((l >> 1) * N2 + mr_pos<R>(F, w * N)) + (l & 1)] = 0.0;
         }
         const int l = (int)threadIdx.x % nl, n = nb + l;
         double *zl = zd + 2 * (l >> 1) * N2 + (l & 1);
@@ -989,8 +997,8 @@ __global__ void __launch_bounds__(512) k_t_yfft_inv(TGeo g, const double *__rest
             for (int u = 0; u < B; ++u) {
                 const int q = q0 + u * qstep;
                 if (q > N - 1) break;
-                zl[2 * (int)bitrev((unsigned)q, bits)] = x[u];
-                zl[2 * (int)bitrev((unsigned)(N2 - q), bits)] = -x[u];
+                zl[2 * mr_pos<R>(F, q)] = x[u];
+                zl[2 * mr_pos<R>(F, N2 - q)] = -x[u];
             }
         }
     } else {
@@ -1015,15 +1023,15 @@ __global__ void __launch_bounds__(512) k_t_yfft_inv(TGeo g, const double *__rest
             const double2 c = cq[q];
             const double ar = 2.0 * c.x * ca, ai = 2.0 * c.y * ca, br = 2.0 * c.x * cb, bi = 2.0 * c.y * cb;
             double2 *zp = z + pr * N2;
-            zp[bitrev((unsigned)q, bits)] = make_double2(ar - bi, ai + br);
-            if (q > 0) zp[bitrev((unsigned)(N2 - q), bits)] = make_double2(ar + bi, br - ai);
-            else zp[bitrev((unsigned)N, bits)] = make_double2(0.0, 0.0);
+            zp[mr_pos<R>(F, q)] = make_double2(ar - bi, ai + br);
+            if (q > 0) zp[mr_pos<R>(F, N2 - q)] = make_double2(ar + bi, br - ai);
+            else zp[mr_pos<R>(F, N)] = make_double2(0.0, 0.0);
         }
         }
     }
     __syncthreads();
-    if (FACES) fft_stages<false>(z, twl, N2, bits, LP);
-    else fft_stages<true>(z, twl, N2, bits, LP);
+    if (FACES) mr_transform<false, R>(z, F, twl, twl + (1 << F.bits) / 2, LP);
+    else mr_transform<true, R>(z, F, twl, twl + (1 << F.bits) / 2, LP);
     const int K = FACES ? N - 1 : N;
     const double sc = FACES ? 1.0 / N : 1.0 / N2;
     const int lo = (int)threadIdx.x % nl, no = nb + lo;
@@ -1210,14 +1218,23 @@ __global__ void __launch_bounds__(WG) k_t_energy_sum(const double *part, int nb,
 
 }  // namespace
 
-// the mode transforms of vv_ytrans.h: the kernels above with the tank's
-// launch shape (2 LP lines a workgroup of 512 threads, LP = min(4, 2048/np))
-bool ytrans_fits(int np) { return np >= 8 && np <= 2048 && (np & (np - 1)) == 0; }
+// the mode transforms of vv_ytrans.h: the kernels above, 2 lp lines a
+// workgroup of 512 threads: 8 lines (64 B of each plane) in 64 KB of LDS,
+// plus the twiddles, two workgroups per CU (16 lines in 128 KB, and 256 or
+// 1024 threads, measured slower)
+bool ytrans_fits(int np)
+{
+    if (np < 8 || np > 2048) return false;
+    int b = 2 * np;
+    for (int p : {2, 3, 5, 7, 11, 13})
+        while (b % p == 0) b /= p;
+    return b == 1;
+}
 
 int ytrans_setup(YTrans &T, int np, int ldi, int ldj)
 {
     if (!ytrans_fits(np)) {
-        vv::set_error("mode transform by FFT: np must be a power of two, 8..2048");
+        vv::set_error("mode transform by FFT: np must be 8..2048 with no prime factor above 13");
         return VV_EINVAL;
     }
     const double pi = std::acos(-1.0);
@@ -1225,22 +1242,24 @@ int ytrans_setup(YTrans &T, int np, int ldi, int ldj)
     T.np = np;
     T.ldi = ldi;
     T.ldj = ldj;
-    T.bits = __builtin_ctz((unsigned)N2);
-    T.lp = std::max(1, std::min(4, 4096 / N2));
-    std::vector<double2> t(2 * (size_t)np);
-    for (int q = 0; q < np; ++q) {
-        t[q] = make_double2(std::cos(2.0 * pi * q / N2), -std::sin(2.0 * pi * q / N2));
-        t[np + q] = make_double2(std::cos(pi * q / N2), std::sin(pi * q / N2));
-    }
-    VV_HIP(hipMalloc(&T.tw, t.size() * sizeof(double2)));
-    VV_HIP(hipMemcpy(T.tw, t.data(), t.size() * sizeof(double2), hipMemcpyHostToDevice));
+    T.lp = vv::pow2_floor(std::max(1, std::min(4, 4096 / N2)));
+    const vv::MrTables M = vv::mr_tables(N2);
+    // the plan's tables, then (cos, sin)(pi q/(2 np)) on a 16-byte boundary
+    const size_t at = (M.bytes() + 15) / 16 * 16;
+    std::vector<double2> c(np);
+    for (int q = 0; q < np; ++q) c[q] = make_double2(std::cos(pi * q / N2), std::sin(pi * q / N2));
+    VV_HIP(hipMalloc(&T.tab, at + c.size() * sizeof(double2)));
+    VV_HIP(vv::mr_upload(M, T.tab));
+    T.cq = reinterpret_cast<double2 *>(static_cast<char *>(T.tab) + at);
+    VV_HIP(hipMemcpy(T.cq, c.data(), c.size() * sizeof(double2), hipMemcpyHostToDevice));
+    T.plan = M.at(T.tab);
     return VV_OK;
 }
 
 void ytrans_free(YTrans &T)
 {
-    if (T.tw) (void)hipFree(T.tw);
-    T.tw = nullptr;
+    if (T.tab) (void)hipFree(T.tab);
+    T.tab = nullptr;
 }
 
 static TGeo ytrans_geo(const YTrans &T)
@@ -1252,28 +1271,32 @@ static TGeo ytrans_geo(const YTrans &T)
     return g;
 }
 
+static size_t ytrans_lds(const YTrans &T)
+{
+    const size_t tw = (size_t)(1 << T.plan.bits) / 2 + (T.plan.nst ? T.plan.n : 0);
+    return ((size_t)T.lp * T.plan.n + tw) * sizeof(double2);
+}
+
 void ytrans_fwd(const YTrans &T, bool faces, const double *rhs, double *S, int i1, int mt, hipStream_t s)
 {
-    const int LP = T.lp, nbk = (mt + 2 * LP - 1) / (2 * LP);
-    const size_t flds = ((size_t)LP * 2 * T.np + T.np) * sizeof(double2);
-    const TGeo g = ytrans_geo(T);
-    const double2 *tw = T.tw, *cq = T.tw + T.np;
-    if (faces)
-        hipLaunchKernelGGL(k_t_yfft_fwd<true>, dim3(nbk), dim3(512), flds, s, g, rhs, S, tw, cq, i1, mt, LP, T.bits);
-    else
-        hipLaunchKernelGGL(k_t_yfft_fwd<false>, dim3(nbk), dim3(512), flds, s, g, rhs, S, tw, cq, i1, mt, LP, T.bits);
+    const int nbk = (mt + 2 * T.lp - 1) / (2 * T.lp);
+    auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(nbk), dim3(512), ytrans_lds(T), s, ytrans_geo(T), rhs, S, T.plan, (const double2 *)T.cq,
+                           i1, mt, T.lp);
+    };
+    if (T.plan.nst) faces ? go(k_t_yfft_fwd<true, 1>) : go(k_t_yfft_fwd<false, 1>);
+    else faces ? go(k_t_yfft_fwd<true, 0>) : go(k_t_yfft_fwd<false, 0>);
 }
 
 void ytrans_inv(const YTrans &T, bool faces, const double *S, double *psi, int i1, int mt, hipStream_t s)
 {
-    const int LP = T.lp, nbk = (mt + 2 * LP - 1) / (2 * LP);
-    const size_t flds = ((size_t)LP * 2 * T.np + T.np) * sizeof(double2);
-    const TGeo g = ytrans_geo(T);
-    const double2 *tw = T.tw, *cq = T.tw + T.np;
-    if (faces)
-        hipLaunchKernelGGL(k_t_yfft_inv<true>, dim3(nbk), dim3(512), flds, s, g, S, psi, tw, cq, i1, mt, LP, T.bits);
-    else
-        hipLaunchKernelGGL(k_t_yfft_inv<false>, dim3(nbk), dim3(512), flds, s, g, S, psi, tw, cq, i1, mt, LP, T.bits);
+    const int nbk = (mt + 2 * T.lp - 1) / (2 * T.lp);
+    auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(nbk), dim3(512), ytrans_lds(T), s, ytrans_geo(T), S, psi, T.plan, (const double2 *)T.cq,
+                           i1, mt, T.lp);
+    };
+    if (T.plan.nst) faces ? go(k_t_yfft_inv<true, 1>) : go(k_t_yfft_inv<false, 1>);
+    else faces ? go(k_t_yfft_inv<true, 0>) : go(k_t_yfft_inv<false, 0>);
 }
 
 }  // namespace vvt
@@ -1325,9 +1348,8 @@ struct vvt_run {
     double *cS = nullptr, *cT = nullptr, *ccp = nullptr;
     double *ckp = nullptr;        // checkpoints of the y/z derivative lines: 8 jobs x ckp_seg x ckp_lines
     int ckp_seg = 0, ckp_lines = 0;
-    double2 *ytw = nullptr;       // y FFT: twiddles of 2np points (np), then (cos, sin)(pi q/(2np)) (np)
-    bool yfft = false;            // y modes by FFT (np a power of two, 8..2048)
-    int ylp = 1, ybits = 0;       // line pairs per workgroup, log2(2np)
+    YTrans yt;                    // y modes by FFT where np fits (ytrans_fits)
+    bool yfft = false;
     double *heat = nullptr;       // 2 nr column sums, trans1, trans2, then the flux terms
     double *kepart = nullptr;     // KE_MAXB partials, then the total
     // profiling
@@ -1409,19 +1431,10 @@ int setup_poisson(vvt_run *r)
     const int np = r->np;
     const double hhr = r->dr * r->dr, hhz = r->dz * r->dz, hhp = r->dp * r->dp;
     size_t mmax = 0, kmax = 0;
-    r->yfft = np >= 8 && np <= 2048 && (np & (np - 1)) == 0;
+    r->yfft = ytrans_fits(np);
     if (r->yfft) {
-        const int N2 = 2 * np;
-        r->ybits = __builtin_ctz((unsigned)N2);
-        // 8 lines a workgroup (64 B of each plane) in 64 KB of LDS, plus the
-        // twiddles: two workgroups per CU (16 lines in 128 KB measured slower)
-        r->ylp = std::max(1, std::min(4, 4096 / N2));
-        std::vector<double2> t(2 * (size_t)np);
-        for (int q = 0; q < np; ++q) {
-            t[q] = make_double2(std::cos(2.0 * pi * q / N2), -std::sin(2.0 * pi * q / N2));
-            t[np + q] = make_double2(std::cos(pi * q / N2), std::sin(pi * q / N2));
-        }
-        VV_HIP(upload(&r->ytw, t));
+        const int st = ytrans_setup(r->yt, np, r->ldi, r->ldj);
+        if (st) return st;
     }
     for (int w = 1; w <= 3; ++w) {
         TankOp &O = r->op[w - 1];
@@ -1711,18 +1724,9 @@ int launch_poisson(vvt_run *r, int which)
     P = r->f[psi];
     const bool split = (r->np % 2 == 0);
     const int h = r->np / 2;
-    const int LP = r->ylp, nbk = (mt + 2 * LP - 1) / (2 * LP);
-    const size_t flds = ((size_t)LP * 2 * r->np + r->np) * sizeof(double2);
-    const int yt = 512;    // threads: a multiple of the 2 LP lines (measured: 256 and 1024 slower)
-    const double2 *tw = r->ytw, *cq = r->ytw + r->np;
     if (r->yfft) {   // reads the right-hand side's unknowns, writes the spectra
         Prof p(r, VVT_K_YFFT_FWD, 8.0 * 2.0 * O.k1 * (double)mt);
-        if (which == 2)
-            hipLaunchKernelGGL(k_t_yfft_fwd<true>, dim3(nbk), dim3(yt), flds, s, g, (const double *)r->f[rhs], r->cS,
-                               tw, cq, O.i1, mt, LP, r->ybits);
-        else
-            hipLaunchKernelGGL(k_t_yfft_fwd<false>, dim3(nbk), dim3(yt), flds, s, g, (const double *)r->f[rhs], r->cS,
-                               tw, cq, O.i1, mt, LP, r->ybits);
+        ytrans_fwd(r->yt, which == 2, r->f[rhs], r->cS, O.i1, mt, s);
     } else {
         Prof p(r, VVT_K_YFWD, split ? 2.0 * (2.0 * h * h * (double)mt) : ftr_y);
         if (split)
@@ -1756,12 +1760,7 @@ int launch_poisson(vvt_run *r, int which)
     }
     if (r->yfft) {
         Prof p(r, VVT_K_YFFT_INV, 8.0 * 2.0 * O.k1 * (double)mt);
-        if (which == 2)
-            hipLaunchKernelGGL(k_t_yfft_inv<true>, dim3(nbk), dim3(yt), flds, s, g, (const double *)r->cS, P, tw, cq,
-                               O.i1, mt, LP, r->ybits);
-        else
-            hipLaunchKernelGGL(k_t_yfft_inv<false>, dim3(nbk), dim3(yt), flds, s, g, (const double *)r->cS, P, tw, cq,
-                               O.i1, mt, LP, r->ybits);
+        ytrans_inv(r->yt, which == 2, r->cS, P, O.i1, mt, s);
         if (which != 2)
             hipLaunchKernelGGL(k_t_psi_post, dim3(nblk((long long)r->ldi * r->ldj, WG)), dim3(WG), 0, s, g, P);
     } else {
@@ -1976,7 +1975,7 @@ int vvt_destroy(vvt_run *r)
         for (hipEvent_t e : {r->fork, r->join, r->forkd, r->joind})
             if (e) (void)hipEventDestroy(e);
         if (r->stream2) (void)hipStreamDestroy(r->stream2);
-        if (r->ytw) (void)hipFree(r->ytw);
+        ytrans_free(r->yt);
         if (r->ckp) (void)hipFree(r->ckp);
         for (hipEvent_t e : r->ev)
             if (e) (void)hipEventDestroy(e);
