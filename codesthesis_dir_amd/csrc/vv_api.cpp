@@ -191,32 +191,6 @@ int upload_tab(vv_run *r, double **dst, const std::vector<double> &h)
     return VV_OK;
 }
 
-// The tables of the chunked line kernel in the order of its LDS (vv_lines.h):
-// LTC = 8 closing words, then over the head's places f | b | 1/b [| c], the
-// places before row 0 neutral (f = 0, b = 1).  Whether every row from the
-// 17th on (before the last, whose closing form has its own words) has the
-// settled factor and pivot and c = 1.
-constexpr int PK_CLOSE = 8;
-
-bool pack_head(std::vector<double> &t, const double *f, const double *b, const double *c, int N, bool with_c,
-               const std::vector<double> &close)
-{
-    const int sh = lshift(N), hw = lheadb(N) * LU;
-    t = close;
-    t.resize(PK_CLOSE, 0.0);
-    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 0.0 : f[p - sh]);
-    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : b[p - sh]);
-    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : 1.0 / b[p - sh]);
-    bool ok = true;
-    if (with_c)
-        for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : c[p - sh]);
-    for (int q = 0; q < N; ++q) {
-        if (!with_c || q + sh >= hw) ok = ok && c[q] == 1.0;
-        if (q + sh >= hw) ok = ok && f[q] == LF && b[q] == LB;
-    }
-    return ok;
-}
-
 // blocks of the N places (row q at q + lshift(N)) up to the last nonzero v[q]
 int blocks_used(const double *v, int N)
 {
@@ -240,7 +214,7 @@ int build_tables(vv_run *r)
         h.insert(h.end(), t.c.begin(), t.c.end());
         for (double v : t.bp) h.push_back(1.0 / v);
         std::vector<double> pk;
-        ok = pack_head(pk, t.fact.data(), t.bp.data(), t.c.data(), n - 1, true,
+        ok = line_pack_head(pk, t.fact.data(), t.bp.data(), t.c.data(), n - 1, true,
                              {t.fact[n - 1], t.bp[n - 1], 1.0 / t.bp[n - 1]}) && ok;
         const size_t at = h.size();
         h.insert(h.end(), pk.begin(), pk.end());
@@ -261,7 +235,7 @@ int build_tables(vv_run *r)
         h.insert(h.end(), t.c.begin(), t.c.end());
         for (double v : t.bp) h.push_back(1.0 / v);
         std::vector<double> pk;
-        ok = pack_head(pk, t.fact.data(), t.bp.data(), t.c.data(), n - 1, true,
+        ok = line_pack_head(pk, t.fact.data(), t.bp.data(), t.c.data(), n - 1, true,
                              {t.fact[n - 1], t.bp[n - 1], 1.0 / t.bp[n - 1]}) && ok;
         const size_t at = h.size();
         h.insert(h.end(), pk.begin(), pk.end());
@@ -286,7 +260,7 @@ int build_tables(vv_run *r)
         for (double v : t.b) h.push_back(v != 0.0 ? 1.0 / v : 0.0);   // entry 0 is unused
         const int N = n - 2, sh = lshift(N);
         std::vector<double> pk;
-        ok = pack_head(pk, t.f1.data() + 1, t.b.data() + 1, t.c.data() + 1, N, false,
+        ok = line_pack_head(pk, t.f1.data() + 1, t.b.data() + 1, t.c.data() + 1, N, false,
                              {t.fA, t.fB, t.fC, t.b[n], 1.0 / t.b[n], t.c[n - 1], t.b[n - 1], 1.0 / t.b[n - 1]}) && ok;
         // a over its places, a block of zeros, then the factors of rn: place p
         // holds f2 of the row after p's

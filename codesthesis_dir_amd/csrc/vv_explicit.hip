@@ -113,28 +113,17 @@ __device__ __forceinline__ int line_pos(int q, int N)
     return q < N ? lrow(q + lshift(N)) : lwords(N) + (q - N);
 }
 
-// How a family's lines are split: P lanes a line (mb blocks each beyond the
-// warm-up), T lines a workgroup (T P <= WG).
-struct LineTile {
-    int P, lgP, T, mb;
-};
 struct CompactTiles {
     LineTile r, p;
-    const double *pk1, *pkT, *pkp;   // the tables packed in LDS order (pack_tdma, pack_ptdma)
+    const double *pk1, *pkT, *pkp;   // the tables packed in LDS order (vv_api.cpp)
     int na, nf;         // blocks of ptdma's a and f2 that are not all zero
     int tabw;           // LDS words of the tables, in front of the lines
 };
 
-// The workgroup's lines: n rows, N of them before the closing ones, pitch
-// LDS words a line from word R on.  The tables' words: LTC closing words,
-// then over the head's places f | b | 1/b | c (r) or f | b | 1/b (phi), and
-// for phi a over all places (zeros left out, a block of zeros behind) and the
-// factors of rn, g_p = f2 of the next place, in whole blocks.
-constexpr int LTC = 8;
+// The workgroup's lines: n rows, pitch LDS words a line from word R on.
 struct LineSet {
     int n, N, pitch, first, tc, R;
-    int hw;                 // places of the head
-    int Ta, Tg, taw, nf;    // phi: words of a and g, words of a before its zeros, blocks of g
+    LineTab tab;
 };
 
 // The reference tdma / ptdma (rb.f:3046-3116) row by row on one lane, from
@@ -262,80 +251,6 @@ __device__ __forceinline__ void line_stage(const CompactArgs &a, const LineSet &
     }
 }
 
-// The settled rows of a line are run by its P lanes as chunks with proven
-// entries (vv_lines.h), the head's places and the closing rows by all of them
-// alike.  Bound by the chain's instructions: 2 (40 + 8 mb) + 48 rows a lane,
-// where one lane a line ran 2 n.  Measured, the whole kernel, one lane a line
-// against this: 12.7 -> 12.8 us at 65x33, 41 -> 14.5 at 97x337, 42 -> 19 at
-// 513x257, 154 -> 38 at 1025x513, 3265 -> 262 at 2049x2049 (where the tables
-// had left LDS as well).  Returns whether every entry was proven.
-template <bool CYC>
-__device__ __forceinline__ bool line_solve(const LineSet &s, const LineTile &L, double *S)
-{
-    const int tid = (int)threadIdx.x, li = tid >> L.lgP, c = tid & (L.P - 1);
-    const int hb = s.hw / LU, nb = lblocks(s.N) - hb;   // blocks of the head, settled blocks
-    const int Q = s.R + li * s.pitch, X = Q + lwords(s.N), Q0 = Q + hb * (LU + 1);
-    const int Th = LTC;
-    double rp = 0.0, mx = 0.0;
-#pragma unroll 1
-    for (int b = 0; b < hb; ++b) rp = block_fwd<true>(S, Q + b * (LU + 1), Th + b * LU, c == 0, rp);
-    bool ok = true;
-    if (nb > 0) {
-        ok = line_fwd<CYC>(S, Q0, nb, c, L.mb, L.P, rp, mx);
-        rp = S[X - 2];   // the last place
-    }
-    // closing rows
-    double y, yn = 0.0;
-    if (CYC) {
-        // rn takes f2_j r_{j-1} of every row in the reference's order;
-        // |f2_j+1| = |f2_j| / b_j falls off as 0.268^j, so once the rest
-        // cannot move rn's last bit (|f2| max|r| below 2^-57 |rn|) it is
-        // left out
-        if (nb > LWB) atomicMax(reinterpret_cast<unsigned long long *>(S) + X + 2, (unsigned long long)__double_as_longlong(mx));
-        wave_fence();
-        double rn = S[X + 1];
-        const double m = S[X + 2];
-        const int free = hb + LWB;   // blocks that m does not cover
-#pragma unroll 1
-        for (int b = 0; b < s.nf; ++b) {
-            double g[LU], r[LU];
-#pragma unroll
-            for (int u = 0; u < LU; ++u) {
-                g[u] = S[s.Tg + b * LU + u];
-                r[u] = S[Q + b * (LU + 1) + u];
-            }
-            if (b >= free && fabs(g[0]) * m <= 0x1p-57 * fabs(rn)) break;
-#pragma unroll
-            for (int u = 0; u < LU; ++u) rn = rn - g[u] * r[u];
-        }
-        const double rn1 = S[X] - S[0] * rp;
-        rn = rn - S[1] * rp;
-        rn = rn - S[2] * rn1;
-        yn = line_div(rn, S[3], S[4]);
-        y = line_div(rn1 - S[5] * yn, S[6], S[7]);
-        wave_fence();
-        if (c == 0) {
-            S[X + 1] = yn;
-            S[X] = y;
-        }
-    } else {
-        rp = S[X] - S[0] * rp;
-        y = line_div(rp, S[1], S[2]);
-        wave_fence();
-        if (c == 0) S[X] = y;
-    }
-    if (nb > 0) {
-        const int o = hb * (LU + 1);
-        ok = line_back<CYC>(S, Q0, nb, c, L.mb, L.P, y, s.Ta + o, s.taw - o, yn) && ok;
-        y = S[Q0];
-    }
-#pragma unroll 1
-    for (int b = hb - 1; b >= 0; --b)
-        y = block_back<true, CYC>(S, Q + b * (LU + 1), Th + s.hw + b * LU, Th + 2 * s.hw + b * LU, Th + 3 * s.hw + b * LU,
-                                  s.Ta + b * (LU + 1), c == 0, yn, y);
-    return ok;
-}
-
 __device__ __forceinline__ double line_rhs_any(const CompactArgs &a, int fam, int line, int q)
 {
     switch (fam) {
@@ -355,7 +270,7 @@ __device__ __forceinline__ void line_finish(const CompactArgs &a, const LineTile
     const int tid = (int)threadIdx.x, N = s.N;
     const int li = tid >> L.lgP, c = tid & (L.P - 1);
     if (li < s.tc) {   // the P lanes of a line are one wavefront's, and leave together
-        const bool ok = line_solve<CYC>(s, L, S);
+        const bool ok = line_solve<CYC>(S, s.R + li * s.pitch, N, c, L, s.tab);
         const unsigned long long lm = (L.P == 64 ? ~0ull : ((1ull << L.P) - 1)) << ((tid & 63) & ~(L.P - 1));
         if ((__ballot(ok) & lm) != lm) {   // row by row, from the right-hand sides again
             const int Q = s.R + li * s.pitch;
@@ -402,15 +317,15 @@ __global__ void __launch_bounds__(WG) k_compact(CompactArgs a, CompactTiles t)
     double *out = fam == 0 ? a.dCr : fam == 1 ? a.dthrC : fam == 2 ? a.dthrT : fam == 3 ? a.dCh : fam == 4 ? a.dthhC : a.dthhT;
     s.pitch = lpitch(s.N, cyc ? 3 : 1);
     s.R = t.tabw;
-    s.hw = lheadb(s.N) * LU;
-    s.Ta = LTC + 3 * s.hw;
-    s.taw = t.na * (LU + 1);
-    s.Tg = s.Ta + s.taw + LU + 1;
-    s.nf = t.nf;
+    s.tab.hw = lheadb(s.N) * LU;
+    s.tab.Ta = LTC + 3 * s.tab.hw;
+    s.tab.taw = t.na * (LU + 1);
+    s.tab.Tg = s.tab.Ta + s.tab.taw + LU + 1;
+    s.tab.nf = t.nf;
     // the tables of the chunked form, packed in LDS order; loaded before the
     // right-hand sides and stored after them, so that both are in flight
     const double *pk = cyc ? t.pkp : (fam == 2) ? t.pkT : t.pk1;
-    const int pw = cyc ? s.Tg + s.nf * LU : LTC + 4 * s.hw;
+    const int pw = cyc ? s.tab.Tg + s.tab.nf * LU : LTC + 4 * s.tab.hw;
     constexpr int PK = 5;
     double pv[PK];
 #pragma unroll

@@ -34,6 +34,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 namespace vv {
 
 constexpr int LU = 8;                 // rows per block
@@ -160,26 +162,27 @@ __device__ __forceinline__ double block_back(double *S, int q, int tb, int tr, i
     return y;
 }
 
-// Settled rows forward over the nb > 0 blocks at q0 (block 0 first) from rp,
-// the row before block 0 (exact), on the P lanes of the line, this one c;
-// every lane runs LWB + mb blocks (past the last block it reads that one and
-// stores nothing).  MAX: mx gathers |r| of the rows behind the first LWB
-// blocks.  Returns whether the lane's entry is proven.
-template <bool MAX>
-__device__ __forceinline__ bool line_fwd(double *S, int q0, int nb, int c, int mb, int P, double rp, double &mx)
+// Rows forward over the nb > 0 blocks at q0 (block 0 first) from rp, the row
+// before block 0 (exact), on the P lanes of the line, this one c; every lane
+// runs LWB + mb blocks (past the last block it reads that one and stores
+// nothing).  TAB: factors at word tf, laid out as the rows; settled ones
+// otherwise.  MAX: mx gathers |r| of the rows behind the first LWB blocks.
+// Returns whether the lane's entry is proven.
+template <bool TAB, bool MAX>
+__device__ __forceinline__ bool line_fwd(double *S, int q0, int nb, int c, int mb, int P, int tf, double rp, double &mx)
 {
     const int b0 = c * mb;
     if (c) rp = 0.0;
 #pragma unroll 1
     for (int t = 0; t < LWB; ++t) {
-        const int b = b0 + t;
-        rp = block_fwd<false>(S, q0 + (b < nb ? b : nb - 1) * (LU + 1), 0, c == 0 && b < nb, rp);
+        const int b = b0 + t, o = (b < nb ? b : nb - 1) * (LU + 1);
+        rp = block_fwd<TAB>(S, q0 + o, tf + o, c == 0 && b < nb, rp);
     }
     const double ent = rp;
 #pragma unroll 1
     for (int b = b0 + LWB; b < b0 + LWB + mb; ++b) {
-        const int q = q0 + (b < nb ? b : nb - 1) * (LU + 1);
-        rp = block_fwd<false>(S, q, 0, b < nb, rp);
+        const int o = (b < nb ? b : nb - 1) * (LU + 1), q = q0 + o;
+        rp = block_fwd<TAB>(S, q, tf + o, b < nb, rp);
         if (MAX && b < nb) {
 #pragma unroll
             for (int u = 0; u < LU; ++u) mx = fmax(mx, fabs(S[q + u]));
@@ -189,17 +192,18 @@ __device__ __forceinline__ bool line_fwd(double *S, int q0, int nb, int c, int m
     return c == 0 || b0 + LWB >= nb || same_bits(prev, ent);
 }
 
-// Settled rows back over the same blocks from the last, from y, the row after
-// them (exact).  CYC: a's words at ta, zeros from word taw on (a block of
-// zeros is there).
-template <bool CYC>
-__device__ __forceinline__ bool line_back(double *S, int q0, int nb, int c, int mb, int P, double y, int ta, int taw, double yn)
+// Rows back over the same blocks from the last, from y, the row after them
+// (exact).  TAB: b, 1/b and c at words tb, tr, tc, laid out as the rows.  CYC:
+// a's words at ta, zeros from word taw on (a block of zeros is there).
+template <bool TAB, bool CYC>
+__device__ __forceinline__ bool line_back(double *S, int q0, int nb, int c, int mb, int P, double y, int tb, int tr, int tc,
+                                          int ta, int taw, double yn)
 {
     const int b0 = c * mb;
     if (c) y = 0.0;
     auto block = [&](int b, bool own) {
         const int o = (b < nb ? nb - 1 - b : 0) * (LU + 1);
-        y = block_back<false, CYC>(S, q0 + o, 0, 0, 0, ta + (o < taw ? o : taw), own && b < nb, yn, y);
+        y = block_back<TAB, CYC>(S, q0 + o, tb + o, tr + o, tc + o, ta + (o < taw ? o : taw), own && b < nb, yn, y);
     };
 #pragma unroll 1
     for (int b = b0; b < b0 + LWB; ++b) block(b, c == 0);
@@ -208,6 +212,119 @@ __device__ __forceinline__ bool line_back(double *S, int q0, int nb, int c, int 
     for (int b = b0 + LWB; b < b0 + LWB + mb; ++b) block(b, true);
     const double prev = __shfl_up(y, 1, P);
     return c == 0 || b0 + LWB >= nb || same_bits(prev, ent);
+}
+
+// How lines are split: P lanes a line (mb blocks each beyond the warm-up), T
+// lines a workgroup.
+struct LineTile {
+    int P, lgP, T, mb;
+};
+
+// Words of the tables in LDS: LTC closing words, then over the head's places
+// f | b | 1/b | c (tdma) or f | b | 1/b (ptdma, CYC), and for CYC a over all
+// places (zeros left out, a block of zeros behind) and the factors of rn,
+// g_p = f2 of the next place, in whole blocks.
+constexpr int LTC = 8;
+struct LineTab {
+    int hw;                 // places of the head
+    int Ta, Tg, taw, nf;    // CYC: words of a and g, words of a before its zeros, blocks of g
+};
+
+// One line of the constant 1-4-1 rows, N rows at word Q and the closing row
+// (tdma: one; ptdma: two) behind them, its tables from word 0 on: the settled
+// rows by the line's P lanes as chunks with proven entries, the head's places
+// and the closing rows by all of them alike.  Bound by the chain's
+// instructions: 2 (40 + 8 mb) + 48 rows a lane, where one lane a line ran 2 n.
+// Measured, the whole 2D kernel, one lane a line against this: 12.7 -> 12.8 us
+// at 65x33, 41 -> 14.5 at 97x337, 42 -> 19 at 513x257, 154 -> 38 at 1025x513,
+// 3265 -> 262 at 2049x2049 (where the tables had left LDS as well).  Returns
+// whether every entry was proven.
+template <bool CYC>
+__device__ __forceinline__ bool line_solve(double *S, int Q, int N, int c, const LineTile &L, const LineTab &t)
+{
+    const int hb = t.hw / LU, nb = lblocks(N) - hb;   // blocks of the head, settled blocks
+    const int X = Q + lwords(N), Q0 = Q + hb * (LU + 1), Th = LTC;
+    double rp = 0.0, mx = 0.0;
+#pragma unroll 1
+    for (int b = 0; b < hb; ++b) rp = block_fwd<true>(S, Q + b * (LU + 1), Th + b * LU, c == 0, rp);
+    bool ok = true;
+    if (nb > 0) {
+        ok = line_fwd<false, CYC>(S, Q0, nb, c, L.mb, L.P, 0, rp, mx);
+        rp = S[X - 2];   // the last place
+    }
+    // closing rows
+    double y, yn = 0.0;
+    if (CYC) {
+        // rn takes f2_j r_{j-1} of every row in the reference's order;
+        // |f2_j+1| = |f2_j| / b_j falls off as 0.268^j, so once the rest
+        // cannot move rn's last bit (|f2| max|r| below 2^-57 |rn|) it is
+        // left out
+        if (nb > LWB) atomicMax(reinterpret_cast<unsigned long long *>(S) + X + 2, (unsigned long long)__double_as_longlong(mx));
+        wave_fence();
+        double rn = S[X + 1];
+        const double m = S[X + 2];
+        const int free = hb + LWB;   // blocks that m does not cover
+#pragma unroll 1
+        for (int b = 0; b < t.nf; ++b) {
+            double g[LU], r[LU];
+#pragma unroll
+            for (int u = 0; u < LU; ++u) {
+                g[u] = S[t.Tg + b * LU + u];
+                r[u] = S[Q + b * (LU + 1) + u];
+            }
+            if (b >= free && fabs(g[0]) * m <= 0x1p-57 * fabs(rn)) break;
+#pragma unroll
+            for (int u = 0; u < LU; ++u) rn = rn - g[u] * r[u];
+        }
+        const double rn1 = S[X] - S[0] * rp;
+        rn = rn - S[1] * rp;
+        rn = rn - S[2] * rn1;
+        yn = line_div(rn, S[3], S[4]);
+        y = line_div(rn1 - S[5] * yn, S[6], S[7]);
+        wave_fence();
+        if (c == 0) {
+            S[X + 1] = yn;
+            S[X] = y;
+        }
+    } else {
+        rp = S[X] - S[0] * rp;
+        y = line_div(rp, S[1], S[2]);
+        wave_fence();
+        if (c == 0) S[X] = y;
+    }
+    if (nb > 0) {
+        const int o = hb * (LU + 1);
+        ok = line_back<false, CYC>(S, Q0, nb, c, L.mb, L.P, y, 0, 0, 0, t.Ta + o, t.taw - o, yn) && ok;
+        y = S[Q0];
+    }
+#pragma unroll 1
+    for (int b = hb - 1; b >= 0; --b)
+        y = block_back<true, CYC>(S, Q + b * (LU + 1), Th + t.hw + b * LU, Th + 2 * t.hw + b * LU, Th + 3 * t.hw + b * LU,
+                                  t.Ta + b * (LU + 1), c == 0, yn, y);
+    return ok;
+}
+
+// Host side: the closing words (at most LTC) and the head's tables in that
+// order, the places before row 0 neutral (f = 0, b = 1).  Returns whether
+// every row from the 17th on has the settled factor and pivot and c = 1, as
+// the chunks take them.
+inline bool line_pack_head(std::vector<double> &t, const double *f, const double *b, const double *c, int N, bool with_c,
+                           const std::vector<double> &close)
+{
+    const int sh = lshift(N), hw = lheadb(N) * LU;
+    t = close;
+    t.resize(LTC, 0.0);
+    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 0.0 : f[p - sh]);
+    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : b[p - sh]);
+    for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : 1.0 / b[p - sh]);
+    bool ok = true;
+    if (with_c)
+        for (int p = 0; p < hw; ++p) t.push_back(p < sh ? 1.0 : c[p - sh]);
+    for (int q = 0; q < N; ++q) {
+        if (!with_c || q + sh >= hw) ok = ok && c[q] == 1.0;
+        if (q + sh >= hw) ok = ok && f[q] == LF && b[q] == LB;
+    }
+    return ok;
 }
 
 }  // namespace vv

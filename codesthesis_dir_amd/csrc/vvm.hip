@@ -2,8 +2,8 @@
 // gfx950 (include/vvmerid.h).
 //
 // Explicit part: the compact advection derivatives as batched line solves
-// (lines along r and along z staged in LDS with their row tables, one
-// thread per line), with the row tables of the uneven nodes and their elimination
+// (lines along r and along z staged in LDS with their row tables, several
+// lanes per line in chunks with proven entries), with the row tables of the uneven nodes and their elimination
 // factors formed once on the host; then one thread per node for the
 // DuFort-Frankel step, the right-hand sides and the walls.  Every
 // expression is evaluated in the operation order of the oracle (the library
@@ -21,6 +21,7 @@
 
 #include "vv_eig.h"
 #include "vv_gemm.h"
+#include "vv_lines.h"
 #include "vv_reduce.h"
 
 #include "../../include/vvmerid.h"
@@ -38,12 +39,20 @@ namespace {
 constexpr int WG = 256;
 constexpr int MAXB = 1024;   // partials of the reductions
 
-// compact tables of one axis of n intervals: the forward rows (a, b, c of
-// the right-hand side, Thomas factor) 4 per node | the backward rows (beta,
-// b', 1/b', 0) 4 per node | alpha of row 1, beta of row n-1, the end
-// weights e0[5], en[5], 4 spare
-inline size_t ctab_size(int n) { return 8 * (size_t)(n + 1) + 16; }
+// compact tables of one axis of n intervals: the right-hand sides' weights
+// a, b, c, 3 per node | alpha of row 1, beta of row n-1, the end weights
+// e0[5], en[5], 4 spare | over the places of the N = n-1 rows (vv_lines.h)
+// the Thomas factor, b', 1/b' and beta (0 in the last row)
+__host__ __device__ inline size_t ctab_line(int n) { return 3 * (size_t)(n + 1) + 16; }
+inline size_t ctab_size(int n) { return ctab_line(n) + 4 * (size_t)vv::lwords(n - 1); }
+
 constexpr int LDS_WORDS = 8192;   // 64 KB of LDS per workgroup
+
+// how the lines of one direction are split: P lanes a line, mb blocks each
+// beyond the warm-up, T lines and nb workgroups a field
+struct MLines {
+    int P, lgP, T, mb, nb;
+};
 
 struct MGeo {
     int nr, nz, ld;
@@ -61,185 +70,127 @@ struct MGeo {
 
 inline int nblk(long long n, int b) { return (int)((n + b - 1) / b); }
 
-// x / b for a positive or negative pivot b with rb = RN(1/b): Markstein's
-// correction of q0 = x rb by the exact remainder, the correctly rounded
-// quotient in three dependent operations (the IEEE division of the oracle).
-__device__ __forceinline__ double qdiv(double x, double b, double rb)
-{
-    const double q0 = x * rb;
-    const double t = __builtin_fma(b, q0, -x);
-    return __builtin_fma(-t, rb, q0);
-}
-
 // ------------------------------------------------------- compact lines
 struct DF3 {
     const double *f[3];   // w, v, th
     double *d[6];         // w_r, w_z, v_r, v_z, th_r, th_z
 };
 
-// One line of n intervals, nodes L[0..n] in LDS, in two passes with the
-// matching half of the table in LDS (tab: 4 words per row, misc: the end
-// weights).  The forward pass leaves the eliminated right-hand sides in
-// L[1..n-1]; the backward pass the derivative.  A group's nodes are read
-// ahead of the rows that overwrite them.
-__device__ __forceinline__ void line_fwd(double *L, int n, const double *tab, const double *misc)
+// Right-hand side of row i of a line whose nodes are f[0], f[st], ...
+__device__ __forceinline__ double row_rhs(const double *__restrict__ f, unsigned st, int n, int i,
+                                          const double *__restrict__ T)
 {
-    const double *e0 = misc + 2, *en = misc + 7;
-    const double al1 = misc[0], bn1 = misc[1];
-    const double d0 = e0[0] * L[0] + e0[1] * L[1] + e0[2] * L[2] + e0[3] * L[3] + e0[4] * L[4];
-    const double dn = en[0] * L[n - 4] + en[1] * L[n - 3] + en[2] * L[n - 2] + en[3] * L[n - 1] + en[4] * L[n];
-    double fa = L[0], fb = L[1], rp = 0.0;
-    // the table and the nodes share the LDS with the rows being written: a
-    // group's reads are all issued before its first write
-    auto row = [&](int ii, const double *q, double fc) {
-        double r = q[0] * fa + q[1] * fb + q[2] * fc;
-        if (ii == 1) r = r - al1 * d0;
-        if (ii == n - 1) r = r - bn1 * dn;
-        rp = (ii == 1) ? r : r - q[3] * rp;
-        L[ii] = rp;
-        fa = fb;
-        fb = fc;
-    };
-    constexpr int U = 8;
-    int i = 1;
-    for (; i + U - 1 <= n - 1; i += U) {
-        double nx[U], qq[U][4];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            nx[u] = L[i + 1 + u];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) qq[u][k] = tab[4 * (i + u) + k];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) row(i + u, qq[u], nx[u]);
+    const double *q = T + 3 * i, *misc = T + 3 * (n + 1), *e0 = misc + 2, *en = misc + 7;
+    double r = q[0] * f[(unsigned)(i - 1) * st] + q[1] * f[(unsigned)i * st] + q[2] * f[(unsigned)(i + 1) * st];
+    if (i == 1) {
+        const double d0 = e0[0] * f[0] + e0[1] * f[st] + e0[2] * f[2 * st] + e0[3] * f[3 * st] + e0[4] * f[4 * st];
+        r = r - misc[0] * d0;
     }
-    for (; i <= n - 1; ++i) {
-        double qq[4];
-        for (int k = 0; k < 4; ++k) qq[k] = tab[4 * i + k];
-        row(i, qq, L[i + 1]);
+    if (i == n - 1) {
+        const double dn = en[0] * f[(unsigned)(n - 4) * st] + en[1] * f[(unsigned)(n - 3) * st] +
+                          en[2] * f[(unsigned)(n - 2) * st] + en[3] * f[(unsigned)(n - 1) * st] + en[4] * f[(unsigned)n * st];
+        r = r - misc[1] * dn;
     }
+    return r;
 }
 
-__device__ __forceinline__ void line_bwd(double *L, int n, const double *tab)
+// Workgroups [0, 3 R.nb) take lines along r (rows j, contiguous), the rest
+// lines along z (columns i): T lines each, their right-hand sides and the
+// axis's tables in LDS, P lanes a line running the recurrence in chunks with
+// proven entries (vv_lines.h; every row with its own factor and pivot, the
+// nodes being uneven).  A line with an entry that is not proven is done again
+// row by row.  Bound by the chain, 2 (40 + 8 mb) rows a lane, where one lane a
+// line ran 2 n: 18.9 us at 513x257 (was 67), the step 67 us (was 117).
+__global__ void __launch_bounds__(WG) k_m_deriv(MGeo g, DF3 F, MLines R, MLines Z)
 {
-    double y = qdiv(L[n - 1], tab[4 * (n - 1) + 1], tab[4 * (n - 1) + 2]);
-    L[n - 1] = y;
-    constexpr int U = 8;
-    int i = n - 2;
-    for (; i - U + 1 >= 1; i -= U) {
-        double rr[U], qq[U][3];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            rr[u] = L[i - u];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) qq[u][k] = tab[4 * (i - u) + k];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            y = qdiv(rr[u] - qq[u][0] * y, qq[u][1], qq[u][2]);
-            L[i - u] = y;
-        }
-    }
-    for (; i >= 1; --i) {
-        const double *q = tab + 4 * i;
-        y = qdiv(L[i] - q[0] * y, q[1], q[2]);
-        L[i] = y;
-    }
-}
-
-// dst[0..n) <- src[0..n) through a 64-thread workgroup, 16 loads in flight
-// per thread before their LDS stores
-__device__ __forceinline__ void lds_fill(double *dst, const double *__restrict__ src, int n, int tid)
-{
-    constexpr int B = 16;
-    for (int e0 = 0; e0 < n; e0 += B * 64) {
-        double v[B];
-#pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const int e = e0 + u * 64 + tid;
-            if (e < n) v[u] = src[e];
-        }
-#pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const int e = e0 + u * 64 + tid;
-            if (e < n) dst[e] = v[u];
-        }
-    }
-}
-
-// Workgroups [0, nbr) take nlr lines along r (rows j, contiguous), the rest
-// nlz lines along z (columns i, loaded row by row and stored transposed);
-// each line sits in LDS with an odd pitch, one thread runs it, and the
-// derivative goes back the way the nodes came.
-__global__ void __launch_bounds__(64) k_m_deriv(MGeo g, DF3 F, int nbr, int nlr, int nlz)
-{
-    extern __shared__ double sh[];
+    using namespace vv;
+    extern __shared__ double S[];
     const int tid = threadIdx.x;
-    const bool rdir = (int)blockIdx.x < nbr;
-    const int n = rdir ? g.nr : g.nz;
-    const double *__restrict__ T = rdir ? g.cr : g.cz;
-    const int tw = 4 * (n + 1), sp = (n + 1) | 1;
-    double *tab = sh, *misc = sh + tw, *lines = sh + tw + 16;
-    int q, o0, nlines;
-    if (rdir) {
-        const int tiles = (g.nz - 1 + nlr - 1) / nlr;
-        q = blockIdx.x / tiles;
-        o0 = 1 + (blockIdx.x - q * tiles) * nlr;     // first row j
-        nlines = min(nlr, g.nz - o0);
-    } else {
-        const int b = blockIdx.x - nbr, tiles = (g.nr - 1 + nlz - 1) / nlz;
-        q = b / tiles;
-        o0 = 1 + (b - q * tiles) * nlz;              // first column i
-        nlines = min(nlz, g.nr - o0);
-    }
+    const bool rdir = (int)blockIdx.x < 3 * R.nb;
+    const MLines L = rdir ? R : Z;
+    const int n = rdir ? g.nr : g.nz, N = n - 1, lines = (rdir ? g.nz : g.nr) - 1;
+    const int bid = rdir ? blockIdx.x : blockIdx.x - 3 * R.nb;
+    const int q = bid / L.nb, o0 = 1 + (bid - q * L.nb) * L.T, tc = min(L.T, lines + 1 - o0);
     const double *__restrict__ f = F.f[q];
     double *__restrict__ d = F.d[2 * q + (rdir ? 0 : 1)];
-    // element e of the tile is (major, minor) = (e / mn, e % mn): r tiles
-    // (line, node), z tiles (node, line); walked in steps of 64 without
-    // divisions
-    {
-        const int mn = rdir ? n + 1 : nlines, total = nlines * (n + 1);
-        const int q64 = 64 / mn, r64 = 64 - q64 * mn;
-        int ma = tid / mn, mi = tid - ma * mn;
-        for (int e0 = 0; e0 < total; e0 += 16 * 64) {
-            double v[16];
-            int li[16];
+    const double *__restrict__ T = rdir ? g.cr : g.cz;
+    const int w = lwords(N), sh = lshift(N), pitch = lpitch(N, 0);
+    const int Tf = 0, Tb = w, Tr = 2 * w, Tc = 3 * w, Q0 = 4 * w;
+    const unsigned st = rdir ? 1u : (unsigned)g.ld, sl = rdir ? (unsigned)g.ld : 1u;   // along the line, between lines
+    {   // tables: loaded first, stored behind the right-hand sides' loads
+        const double *src = T + ctab_line(n);
+        constexpr int PK = 4;
+        double v[PK];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                li[u] = -1;
-                if (e0 + u * 64 + tid < total) {
-                    v[u] = rdir ? f[(unsigned)((o0 + ma) * g.ld + mi)] : f[(unsigned)(ma * g.ld + o0 + mi)];
-                    li[u] = rdir ? ma * sp + mi : mi * sp + ma;
-                }
-                ma += q64;
-                mi += r64;
-                if (mi >= mn) { mi -= mn; ++ma; }
+        for (int u = 0; u < PK; ++u) {
+            const int e = tid + u * WG;
+            v[u] = src[e < 4 * w ? e : 0];
+        }
+        if (rdir) {
+            for (int c = tid >> 6; c < tc; c += WG / 64) {
+                const double *x = f + (unsigned)(o0 + c) * sl;
+#pragma unroll 4
+                for (int e = tid & 63; e < N; e += 64) S[Q0 + c * pitch + lrow(e + sh)] = row_rhs(x, 1u, n, e + 1, T);
+                if ((tid & 63) < sh) S[Q0 + c * pitch + (tid & 63)] = 0.0;
             }
+        } else {
+            const int lgT = 31 - __clz(L.T);
+#pragma unroll 4
+            for (int e = tid; e < (N << lgT); e += WG) {
+                const int c = e & (L.T - 1), r = e >> lgT;
+                if (c < tc) S[Q0 + c * pitch + lrow(r + sh)] = row_rhs(f + o0 + c, st, n, r + 1, T);
+            }
+            const int c = tid >> 3, p = tid & 7;   // T <= 32
+            if (c < tc && p < sh) S[Q0 + c * pitch + p] = 0.0;
+        }
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                if (li[u] >= 0) lines[li[u]] = v[u];
+        for (int u = 0; u < PK; ++u) {
+            const int e = tid + u * WG;
+            if (e < 4 * w) S[e] = v[u];
+        }
+        for (int e = tid + PK * WG; e < 4 * w; e += WG) S[e] = src[e];
+    }
+    __syncthreads();
+    const int li = tid >> L.lgP, c = tid & (L.P - 1);
+    if (li < tc) {
+        const int Q = Q0 + li * pitch, nb = lblocks(N);
+        double mx = 0.0;
+        bool ok = line_fwd<true, false>(S, Q, nb, c, L.mb, L.P, Tf, 0.0, mx);
+        ok = line_back<true, false>(S, Q, nb, c, L.mb, L.P, 0.0, Tb, Tr, Tc, 0, 0, 0.0) && ok;
+        const unsigned long long lm = (L.P == 64 ? ~0ull : ((1ull << L.P) - 1)) << ((tid & 63) & ~(L.P - 1));
+        if ((__ballot(ok) & lm) != lm) {
+            const double *x = f + (unsigned)(o0 + li) * sl;
+            wave_fence();
+#pragma unroll 1
+            for (int r = c; r < N; r += L.P) S[Q + lrow(r + sh)] = row_rhs(x, st, n, r + 1, T);
+            if (c < sh) S[Q + c] = 0.0;
+            if (L.P < sh)
+                for (int p = L.P + c; p < sh; p += L.P) S[Q + p] = 0.0;
+            wave_fence();
+            if (c == 0) {
+                double rp = 0.0, y = 0.0;
+#pragma unroll 1
+                for (int b = 0; b < nb; ++b) rp = block_fwd<true>(S, Q + b * (LU + 1), Tf + b * (LU + 1), true, rp);
+#pragma unroll 1
+                for (int b = nb - 1; b >= 0; --b) {
+                    const int o = b * (LU + 1);
+                    y = block_back<true, false>(S, Q + o, Tb + o, Tr + o, Tc + o, 0, true, 0.0, y);
+                }
+            }
         }
     }
-    lds_fill(tab, T, tw, tid);
-    if (tid < 16) misc[tid] = T[2 * tw + tid];
     __syncthreads();
-    if (tid < nlines) line_fwd(lines + tid * sp, n, tab, misc);
-    __syncthreads();
-    lds_fill(tab, T + tw, tw, tid);
-    __syncthreads();
-    if (tid < nlines) line_bwd(lines + tid * sp, n, tab);
-    __syncthreads();
-    // interior nodes back: r tiles (line, node 1..n-1), z tiles (node
-    // 1..n-1, line), walked as the loads
-    const int mn = rdir ? n - 1 : nlines, tot = nlines * (n - 1);
-    const int q64 = 64 / mn, r64 = 64 - q64 * mn;
-    int ma = tid / mn, mi = tid - ma * mn;
-    for (int e = tid; e < tot; e += 64) {
-        if (rdir) d[(unsigned)((o0 + ma) * g.ld + 1 + mi)] = lines[ma * sp + 1 + mi];
-        else d[(unsigned)((1 + ma) * g.ld + o0 + mi)] = lines[mi * sp + 1 + ma];
-        ma += q64;
-        mi += r64;
-        if (mi >= mn) { mi -= mn; ++ma; }
+    if (rdir) {
+        for (int cc = tid >> 6; cc < tc; cc += WG / 64)
+#pragma unroll 4
+            for (int e = tid & 63; e < N; e += 64) d[(unsigned)(o0 + cc) * sl + e + 1] = S[Q0 + cc * pitch + lrow(e + sh)];
+    } else {
+        const int lgT = 31 - __clz(L.T);
+#pragma unroll 4
+        for (int e = tid; e < (N << lgT); e += WG) {
+            const int cc = e & (L.T - 1), r = e >> lgT;
+            if (cc < tc) d[(unsigned)(r + 1) * st + o0 + cc] = S[Q0 + cc * pitch + lrow(r + sh)];
+        }
     }
 }
 
@@ -590,15 +541,16 @@ void compact_tables(int n, const double *x, double *T)
         fact[i] = R[5 * i + 0] / bp[i - 1];
         bp[i] = 1.0 - fact[i] * R[5 * (i - 1) + 1];
     }
-    double *fw = T, *bw = T + 4 * (n + 1), *misc = T + 8 * (n + 1);
+    double *misc = T + 3 * (n + 1), *line = T + ctab_line(n);
+    const int N = n - 1, w = vv::lwords(N), sh = vv::lshift(N);
+    for (int p = 0; p < sh; ++p) line[w + p] = line[2 * w + p] = 1.0;   // places before row 1
     for (int i = 1; i <= n - 1; ++i) {
-        fw[4 * i + 0] = R[5 * i + 2];
-        fw[4 * i + 1] = R[5 * i + 3];
-        fw[4 * i + 2] = R[5 * i + 4];
-        fw[4 * i + 3] = fact[i];
-        bw[4 * i + 0] = R[5 * i + 1];
-        bw[4 * i + 1] = bp[i];
-        bw[4 * i + 2] = 1.0 / bp[i];
+        for (int q = 0; q < 3; ++q) T[3 * i + q] = R[5 * i + 2 + q];
+        const int o = vv::lrow(i - 1 + sh);
+        line[o] = fact[i];
+        line[w + o] = bp[i];
+        line[2 * w + o] = 1.0 / bp[i];
+        line[3 * w + o] = i < n - 1 ? R[5 * i + 1] : 0.0;
     }
     misc[0] = R[5 * 1 + 0];
     misc[1] = R[5 * (n - 1) + 1];
@@ -640,7 +592,7 @@ struct vvm_run {
     double *geo = nullptr;   // r nodes | wr | wz | cr | cz | hz | hr | heat weights
     MGeo g;
     const double *hz = nullptr, *hr = nullptr, *hw = nullptr;
-    int nlr = 1, nlz = 1, nbr = 0, nbz = 0;
+    MLines lr{}, lz{};
     size_t dlds = 0;
     // Poisson
     double *V = nullptr, *Vi = nullptr, *lam = nullptr, *rt = nullptr;   // rt: [2][3][nr-1]
@@ -691,8 +643,7 @@ int launch_derivatives(vvm_run *r)
     F.f[2] = r->f[VVM_TH];
     for (int d = 0; d < 6; ++d) F.d[d] = r->dv[d];
     Prof P(r, VVM_K_DERIV, 9.0 * 8.0 * npts(r));
-    hipLaunchKernelGGL(k_m_deriv, dim3(r->nbr + r->nbz), dim3(64), r->dlds, r->stream, r->g, F, r->nbr, r->nlr,
-                       r->nlz);
+    hipLaunchKernelGGL(k_m_deriv, dim3(3 * (r->lr.nb + r->lz.nb)), dim3(WG), r->dlds, r->stream, r->g, F, r->lr, r->lz);
     VV_HIP(hipGetLastError());
     return VV_OK;
 }
@@ -840,15 +791,31 @@ int setup(vvm_run *r, const double *rn, const double *zn)
     g.rn = r->geo + o_r; g.wr = r->geo + o_wr; g.wz = r->geo + o_wz;
     g.cr = r->geo + o_cr; g.cz = r->geo + o_cz;
     r->hz = r->geo + o_hz; r->hr = r->geo + o_hr; r->hw = r->geo + o_hw;
-    // derivative launch shape: per direction the half table (4 words a node),
-    // 16 words of end weights and as many lines as fit in 64 KB of LDS
-    auto lines_fit = [](int n) { return (LDS_WORDS - 4 * (n + 1) - 16) / ((n + 1) | 1); };
-    r->nlr = std::max(1, std::min(64, lines_fit(nr)));
-    r->nlz = std::max(1, std::min(16, lines_fit(nz)));
-    r->nbr = 3 * ((nz - 1 + r->nlr - 1) / r->nlr);
-    r->nbz = 3 * ((nr - 1 + r->nlz - 1) / r->nlz);
-    r->dlds = sizeof(double) * std::max(4 * (size_t)(nr + 1) + 16 + (size_t)r->nlr * ((nr + 1) | 1),
-                                        4 * (size_t)(nz + 1) + 16 + (size_t)r->nlz * ((nz + 1) | 1));
+    // derivative launch shape: lanes per line enough for the shortest chains
+    // while the chip has lanes to spare (2 wavefronts a SIMD), fewer above,
+    // but so many that a workgroup's lines fit in 64 KB of LDS beside the
+    // axis's tables (160 KB for the longest)
+    const int br = vv::lblocks(nr - 1), bz = vv::lblocks(nz - 1);
+    int Pr = 1, Pz = 1;
+    while (Pr < 64 && vv::line_mb(br, Pr) > 1) Pr *= 2;
+    while (Pz < 64 && vv::line_mb(bz, Pz) > 1) Pz *= 2;
+    while (3.0 / 64 * ((nz - 1.0) * Pr + (nr - 1.0) * Pz) > 2048 && (Pr > 4 || Pz > 4)) {
+        if (Pr > 4) Pr /= 2;
+        if (Pz > 4) Pz /= 2;
+    }
+    auto shape = [&](MLines &L, int P, int n, int nlines) {
+        const int w = vv::lwords(n - 1), pitch = vv::lpitch(n - 1, 0), room = std::max(LDS_WORDS - 4 * w, pitch);
+        while (P < 64 && WG / P * pitch > room) P *= 2;
+        L.P = P;
+        L.lgP = __builtin_ctz((unsigned)P);
+        L.mb = vv::line_mb(vv::lblocks(n - 1), P);
+        L.T = std::min(WG / P, 16);
+        while (L.T > 1 && L.T * pitch > room) L.T /= 2;
+        L.nb = (nlines + L.T - 1) / L.T;
+        return sizeof(double) * (4 * (size_t)w + (size_t)L.T * pitch);
+    };
+    const size_t sr = shape(r->lr, Pr, nr, nz - 1), sz = shape(r->lz, Pz, nz, nr - 1);
+    r->dlds = std::max(sr, sz);
     // Poisson: z eigenbasis, r rows of both operators
     const int M = nz - 1, N = nr - 1;
     std::vector<double> za(M), zb(M), zc(M);
