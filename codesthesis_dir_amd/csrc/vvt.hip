@@ -2,8 +2,9 @@
 // (include/vvtank.h).
 //
 // Explicit part: the compact advection derivatives as batched line solves
-// (one thread per line, the elimination tables of the constant rows computed
-// once on the host in the order of the reference's tdma), then the A, B, C
+// (several lanes per line in chunks with proven entries, the elimination
+// tables of the constant rows computed once on the host in the order of the
+// reference's tdma), then the A, B, C
 // and temperature updates in one pass (one thread per (i, j) column marching
 // along y), one thread per point for the right-hand sides and the
 // boundaries.  Every expression is evaluated in the operation order the
@@ -22,6 +23,7 @@
 #include "vv3_internal.h"
 #include "vv_fft.h"
 #include "vv_gemm.h"
+#include "vv_lines.h"
 #include "vv_reduce.h"
 #include "vv_ytrans.h"
 #include "vv_zsplit.h"
@@ -54,13 +56,14 @@ inline int nblk(long long n, int b) { return (int)((n + b - 1) / b); }
 // `type` (0: nodes equally spaced, velvor2dperiodicrbconv.f:613-620; 1: walls
 // half a spacing away, its 1085-1097), m unknowns, the lines' other two
 // indices in [1, n1] x [1, n2] (x lines (j, k), y lines (i, j), z lines
-// (i, k)), tables fact | bp | c | 1/bp (1-based, m+1 each), nl lines per
-// workgroup (x lines, staged in LDS).
+// (i, k)), tables fact | bp | c | 1/bp (1-based, m+1 each), then the chunked
+// kernel's (vv_lines.h).
 struct DJob {
     const double *f;
     double *d;
     const double *tab;
-    int axis, type, m, n1, n2, nl;
+    int axis, type, m, n1, n2;
+    vv::LineTile L;
     double dri;
 };
 struct DJobs {
@@ -94,233 +97,120 @@ __device__ __forceinline__ double line_rhs(int type, int m, int i, double dri, d
     return 3.0 * (fp1 - fm1) * dri;
 }
 
-// Lines along y and z: one thread per line, consecutive threads on
-// consecutive i (coalesced).  The lines (256-514 rows) are too long to keep
-// their eliminated right-hand sides r' in registers, so the forward sweep
-// keeps only every CK-th one (a checkpoint, in ckp: 1/CK of the line), and
-// the back substitution works segment by segment from the last: it reads
-// the segment's nodes again, recomputes its r' from the checkpoint before it
-// in registers -- the same operations on the same values, so the same bits
-// -- and substitutes back through them.  Per line that is two reads of the
-// nodes and one write of the derivative, against one read, a write and a
-// read of r' and the final write when r' went through d.  The forward rows
-// are processed in groups of U with their loads issued ahead of the chain.
-constexpr int CK = 32;
-
-// TLDS: the job's tables (fact | b' | c | 1/b', 4 (m+1) words) are copied to
-// LDS first; lines longer than DYZ_LDS_MAXM read them from global memory
-constexpr int DYZ_LDS_MAXM = 2047;
-
-template <bool TLDS>
-__global__ void __launch_bounds__(WG) k_t_deriv_yz(TGeo g, DJobs jobs, int j0, double *__restrict__ ckp, int nseg_max,
-                                                   int nls)
+// The compact lines: a workgroup takes L.T lines neighbouring in their first
+// index (y and z lines: consecutive i, so that 16 of them fill the 128-byte
+// lines of a row), their right-hand sides in LDS, P lanes a line running the
+// recurrences as chunks with proven entries (vv_lines.h), and stores the
+// derivatives from there: every node is read once from HBM and every
+// derivative written once, which bounds it (1.35 ms for the 12 at 512x256x256
+// at the rate of a copy).  One thread per line, as before, could hold neither
+// its rows nor its eliminated right-hand sides, and read the nodes twice (y,
+// z) or passed them through LDS twice (x): 1.39 + 1.23 ms, now 1.08 + 0.67.
+// Workgroups go round the 8 XCDs, so each XCD gets a contiguous eighth of the
+// tiles: a y or z tile's rows start one word past a 128-byte line, and
+// neighbouring tiles share a line for every row, which only one L2 can merge
+// (1.83 ms for y and z without).  A line with an entry that is not proven is
+// done again row by row.
+__global__ void __launch_bounds__(512) k_t_deriv(TGeo g, DJobs jobs)
 {
-    extern __shared__ double tabl[];
-    const DJob J = jobs.j[j0 + blockIdx.y];
-    if constexpr (TLDS) {
-        for (int e = threadIdx.x; e < 4 * (J.m + 1); e += WG) tabl[e] = J.tab[e];
-        __syncthreads();
-    }
-    const int t = blockIdx.x * WG + threadIdx.x;
-    if (t >= J.n1 * J.n2) return;
-    const int q = t / J.n1, p = t - q * J.n1;
-    const int P1 = p + 1, Q1 = q + 1;
-    unsigned base, s;
-    if (J.axis == 1) { base = (unsigned)(Q1 * g.ldi + P1); s = (unsigned)(g.ldi * g.ldj); }
-    else { base = (unsigned)(Q1 * g.ldj * g.ldi + P1); s = (unsigned)g.ldi; }
-    const double *__restrict__ f = J.f;
-    double *__restrict__ d = J.d;
-    double *__restrict__ cp = ckp + (size_t)blockIdx.y * nseg_max * nls + t;   // segment sg at cp[sg * nls]
-    const int m = J.m, type = J.type;
+    using namespace vv;
+    extern __shared__ double S[];
+    const DJob &J = jobs.j[blockIdx.y];
+    const LineTile L = J.L;
+    const int m = J.m, type = J.type, N = m - 1, nt = (int)blockDim.x, tid = (int)threadIdx.x;
+    const int tiles = (J.n1 + L.T - 1) / L.T;
+    const int per = (tiles * J.n2 + 7) >> 3, wg = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || wg >= tiles * J.n2) return;
+    const int q = wg / tiles, p0 = (wg - q * tiles) * L.T, tc = min(L.T, J.n1 - p0);
+    const bool xdir = J.axis == 0;
+    // line p of the tile: nodes f[base + p sl + i st]
+    const unsigned pl = (unsigned)(g.ldi * g.ldj);
+    const unsigned st = xdir ? 1u : J.axis == 1 ? pl : (unsigned)g.ldi, sl = xdir ? (unsigned)g.ldi : 1u;
+    const unsigned base = xdir ? (unsigned)(q + 1) * pl + (unsigned)((p0 + 1) * g.ldi)
+                        : J.axis == 1 ? (unsigned)((q + 1) * g.ldi + p0 + 1)
+                                      : (unsigned)(q + 1) * pl + (unsigned)(p0 + 1);
+    const double *__restrict__ f = J.f + base;
+    double *__restrict__ d = J.d + base;
     const double dri = J.dri;
-    const double *T = TLDS ? tabl : J.tab;
-    const double *fact = T, *bp = T + (m + 1), *cc = T + 2 * (m + 1), *rbp = T + 3 * (m + 1);
-    const double f4 = (type == 1) ? f[base + 4u * s] : 0.0;
-    const double fm3 = (type == 1) ? f[base + (unsigned)(m - 3) * s] : 0.0;
-    const double f2 = f[base + 2u * s];
-    double fa = f[base], fb = f[base + s];   // f[i-1], f[i]
-    double rp = 0.0;
-    constexpr int U = 8;
-    int i = 1;
-    for (; i + U - 1 <= m; i += U) {
-        double nx[U];   // f[i+1 .. i+U]
-#pragma unroll
-        for (int u = 0; u < U; ++u) nx[u] = f[base + (unsigned)(i + 1 + u) * s];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int ii = i + u;
-            const double r = line_rhs(type, m, ii, dri, fm3, fa, fb, nx[u], f2, f4);
-            rp = (ii == 1) ? r : r - fact[ii] * rp;
-            if (ii % CK == 0) cp[(size_t)(ii / CK - 1) * nls] = rp;
-            fa = fb;
-            fb = nx[u];
-        }
-    }
-    for (; i <= m; ++i) {
-        const double fc = f[base + (unsigned)(i + 1) * s];
-        const double r = line_rhs(type, m, i, dri, fm3, fa, fb, fc, f2, f4);
-        rp = (i == 1) ? r : r - fact[i] * rp;
-        if (i % CK == 0) cp[(size_t)(i / CK - 1) * nls] = rp;
-        fa = fb;
-        fb = fc;
-    }
-    double y = 0.0;
-    for (int sg = (m + CK - 1) / CK - 1; sg >= 0; --sg) {
-        const int r0 = sg * CK + 1, r1 = min(r0 + CK - 1, m);
-        double rq = (sg == 0) ? 0.0 : cp[(size_t)(sg - 1) * nls];
-        double fv[CK + 2];   // nodes r0-1 .. r0+CK
-#pragma unroll
-        for (int u = 0; u < CK + 2; ++u) {
-            const int row = r0 - 1 + u;
-            fv[u] = (row <= r1 + 1) ? f[base + (unsigned)row * s] : 0.0;
-        }
-        double rr[CK];
-#pragma unroll
-        for (int u = 0; u < CK; ++u) {
-            const int ii = r0 + u;
-            rr[u] = 0.0;
-            if (ii <= r1) {
-                const double r = line_rhs(type, m, ii, dri, fm3, fv[u], fv[u + 1], fv[u + 2], f2, f4);
-                rq = (ii == 1) ? r : r - fact[ii] * rq;
-                rr[u] = rq;
-            }
-        }
-#pragma unroll
-        for (int u = CK - 1; u >= 0; --u) {
-            const int ii = r0 + u;
-            if (ii <= r1) {
-                y = (ii == m) ? qdiv(rr[u], bp[m], rbp[m]) : qdiv(rr[u] - cc[ii] * y, bp[ii], rbp[ii]);
-                d[base + (unsigned)ii * s] = y;
-            }
-        }
-    }
-}
-
-// Lines along x (contiguous in memory): a workgroup of one wave takes 64
-// lines (consecutive j of one plane k), thread l line l.  The lines pass
-// through LDS in chunks of CX rows (nodes r0-1 .. r0+CX, odd pitch, loaded
-// coalesced along the lines): the forward sweep runs chunk by chunk and
-// keeps one checkpoint of the eliminated right-hand side per chunk (ckp, as
-// the y/z lines); the back substitution takes the chunks from the last,
-// reloads one, recomputes its r' from the checkpoint before it in registers
-// (the same operations, the same bits), substitutes back into the tile and
-// stores the chunk's rows coalesced.
-constexpr int CX = 20, XSP = CX + 3;   // rows per chunk; tile pitch (odd)
-
-__global__ void __launch_bounds__(64) k_t_deriv_x(TGeo g, DJobs jobs, double *__restrict__ ckp, int nseg_max, int nls)
-{
-    __shared__ double sh[64 * XSP];
-    __shared__ double tb[4][CX];   // the chunk's table rows: fact, b', c, 1/b'
-    const DJob J = jobs.j[3 * blockIdx.y];
-    const int m = J.m, type = J.type;
-    const int tiles = (J.n1 + 63) / 64;
-    const int q = blockIdx.x / tiles, p0 = (blockIdx.x - q * tiles) * 64;
-    if (q >= J.n2) return;
-    const int nlines = min(64, J.n1 - p0);
-    const int tid = threadIdx.x;
-    // line l: (j, k) = (p0 + l + 1, q + 1), nodes contiguous from node 0
-    const unsigned base0 = (unsigned)(((q + 1) * g.ldj + (p0 + 1)) * g.ldi);
-    const double *__restrict__ f = J.f;
-    double *__restrict__ d = J.d;
-    const bool act = tid < nlines;
-    const unsigned mybase = base0 + (unsigned)(tid * g.ldi);
-    double *__restrict__ cp = ckp + (size_t)blockIdx.y * nseg_max * nls + (size_t)q * J.n1 + p0 + tid;
-    const double dri = J.dri;
-    const double *fact = J.tab, *bp = J.tab + (m + 1), *cc = J.tab + 2 * (m + 1), *rbp = J.tab + 3 * (m + 1);
-    const double f4 = (act && type == 1) ? f[mybase + 4u] : 0.0;
-    const double fm3 = (act && type == 1) ? f[mybase + (unsigned)(m - 3)] : 0.0;
-    const double f2 = act ? f[mybase + 2u] : 0.0;
-    const int nseg = (m + CX - 1) / CX;
-    double *L = sh + tid * XSP;
-    // nodes r0-1 .. r1+1 of chunk sg into the tile (coalesced: consecutive
-    // threads on consecutive nodes of a line)
-    auto load = [&](int sg) {
-        const int r0 = sg * CX + 1, r1 = min(r0 + CX - 1, m), len = r1 - r0 + 3;
-        const int total = nlines * len;
-        for (int e0 = 0; e0 < total; e0 += 8 * 64) {
-            double v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int e = e0 + u * 64 + tid;
-                if (e < total) {
-                    const int l = e / len, o = e - l * len;
-                    v[u] = f[base0 + (unsigned)(l * g.ldi + r0 - 1 + o)];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int e = e0 + u * 64 + tid;
-                if (e < total) {
-                    const int l = e / len, o = e - l * len;
-                    sh[l * XSP + o] = v[u];
-                }
-            }
-        }
-        if (tid < CX) {   // table rows r0 .. r0+CX-1 (only rows <= r1 are read)
-            const int ii = min(r0 + tid, m);
-            tb[0][tid] = fact[ii];
-            tb[1][tid] = bp[ii];
-            tb[2][tid] = cc[ii];
-            tb[3][tid] = rbp[ii];
-        }
-        __syncthreads();
+    const int pitch = lpitch(N, 1), sh = lshift(N), w = lwords(N);
+    LineTab t{};
+    t.hw = lheadb(N) * LU;
+    const int pw = LTC + 4 * t.hw, R0 = LTC + 4 * LHEAD;
+    const double *pk = J.tab + 4 * (m + 1);
+    auto place = [&](int r) { return r < N ? lrow(r + sh) : w; };   // row r (0-based) of a line
+    auto rhs = [&](const double *x, int r) {                        // its right-hand side
+        const int i = r + 1;
+        return line_rhs(type, m, i, dri, type == 1 ? x[(unsigned)(m - 3) * st] : 0.0, x[(unsigned)(i - 1) * st],
+                        x[(unsigned)i * st], x[(unsigned)(i + 1) * st], x[2u * st], type == 1 ? x[4u * st] : 0.0);
     };
-    double rp = 0.0;
-    for (int sg = 0; sg < nseg; ++sg) {
-        load(sg);
-        const int r0 = sg * CX + 1, r1 = min(r0 + CX - 1, m);
-        if (act) {
-            double fv[CX + 2];
-#pragma unroll
-            for (int u = 0; u < CX + 2; ++u) fv[u] = L[u];
-#pragma unroll
-            for (int u = 0; u < CX; ++u) {
-                const int ii = r0 + u;
-                if (ii <= r1) {
-                    const double r = line_rhs(type, m, ii, dri, fm3, fv[u], fv[u + 1], fv[u + 2], f2, f4);
-                    rp = (ii == 1) ? r : r - tb[0][u] * rp;
-                }
-            }
-            if (sg + 1 < nseg) cp[(size_t)sg * nls] = rp;
+    if (tid < pw) S[tid] = pk[tid];
+    for (int e = tid + nt; e < pw; e += nt) S[e] = pk[e];
+    // rows 2 .. m-1 in their interior form, then the two end rows
+    if (xdir) {
+        for (int c = tid >> 6; c < tc; c += nt >> 6) {
+            const double *x = f + (unsigned)c * sl;
+            const int Q = R0 + c * pitch;
+#pragma unroll 4
+            for (int r = 1 + (tid & 63); r < m - 1; r += 64) S[Q + place(r)] = 3.0 * (x[r + 2] - x[r]) * dri;
         }
-        __syncthreads();
+    } else {   // a thread per line and 8 rows: 10 loads in flight
+        const int lgT = 31 - __clz(L.T), c = tid & (L.T - 1), Q = R0 + c * pitch;
+        if (c < tc)
+            for (int r0 = 1 + (tid >> lgT) * LU; r0 < m - 1; r0 += (nt >> lgT) * LU) {
+                double x[LU + 2];
+#pragma unroll
+                for (int u = 0; u < LU + 2; ++u) x[u] = f[(unsigned)min(r0 + u, m + 1) * st + c];
+#pragma unroll
+                for (int u = 0; u < LU; ++u)
+                    if (r0 + u < m - 1) S[Q + place(r0 + u)] = 3.0 * (x[u + 2] - x[u]) * dri;
+            }
     }
-    double y = 0.0;
-    for (int sg = nseg - 1; sg >= 0; --sg) {
-        load(sg);
-        const int r0 = sg * CX + 1, r1 = min(r0 + CX - 1, m);
-        if (act) {
-            double rq = (sg == 0) ? 0.0 : cp[(size_t)(sg - 1) * nls];
-            double fv[CX + 2], rr[CX];
-#pragma unroll
-            for (int u = 0; u < CX + 2; ++u) fv[u] = L[u];
-#pragma unroll
-            for (int u = 0; u < CX; ++u) {
-                const int ii = r0 + u;
-                rr[u] = 0.0;
-                if (ii <= r1) {
-                    const double r = line_rhs(type, m, ii, dri, fm3, fv[u], fv[u + 1], fv[u + 2], f2, f4);
-                    rq = (ii == 1) ? r : r - tb[0][u] * rq;
-                    rr[u] = rq;
+    for (int e = tid; e < 2 * tc; e += nt) {
+        const int r = (e & 1) ? m - 1 : 0;
+        S[R0 + (e >> 1) * pitch + place(r)] = rhs(f + (unsigned)(e >> 1) * sl, r);
+    }
+    for (int e = tid; e < LU * tc; e += nt)
+        if ((e & 7) < sh) S[R0 + (e >> 3) * pitch + (e & 7)] = 0.0;
+    __syncthreads();
+    const int li = tid >> L.lgP, c = tid & (L.P - 1);
+    if (li < tc) {
+        const int Q = R0 + li * pitch;
+        const bool ok = line_solve<false>(S, Q, N, c, L, t);
+        const unsigned long long lm = (L.P == 64 ? ~0ull : ((1ull << L.P) - 1)) << ((tid & 63) & ~(L.P - 1));
+        if ((__ballot(ok) & lm) != lm) {
+            const double *x = f + (unsigned)li * sl;
+            wave_fence();
+#pragma unroll 1
+            for (int r = c; r < m; r += L.P) S[Q + place(r)] = rhs(x, r);
+            wave_fence();
+            if (c == 0) {   // tdma, row by row
+                const double *fact = J.tab + 1, *bp = fact + (m + 1), *cc = bp + (m + 1), *rb = cc + (m + 1);
+                double v = S[Q + place(0)];
+#pragma unroll 1
+                for (int r = 1; r < m; ++r) {
+                    v = S[Q + place(r)] - fact[r] * v;
+                    S[Q + place(r)] = v;
                 }
-            }
-#pragma unroll
-            for (int u = CX - 1; u >= 0; --u) {
-                const int ii = r0 + u;
-                if (ii <= r1) {
-                    y = (ii == m) ? qdiv(rr[u], tb[1][u], tb[3][u])
-                                  : qdiv(rr[u] - tb[2][u] * y, tb[1][u], tb[3][u]);
-                    L[u + 1] = y;   // row ii sits at tile position ii - r0 + 1
+                v = line_div(v, bp[m - 1], rb[m - 1]);
+                S[Q + place(m - 1)] = v;
+#pragma unroll 1
+                for (int r = m - 2; r >= 0; --r) {
+                    v = line_div(S[Q + place(r)] - cc[r] * v, bp[r], rb[r]);
+                    S[Q + place(r)] = v;
                 }
             }
         }
-        __syncthreads();
-        const int len = r1 - r0 + 1, total = nlines * len;
-        for (int e = tid; e < total; e += 64) {
-            const int l = e / len, o = e - l * len;
-            d[base0 + (unsigned)(l * g.ldi + r0 + o)] = sh[l * XSP + 1 + o];
-        }
-        __syncthreads();
+    }
+    __syncthreads();
+    if (xdir) {
+        for (int cc = tid >> 6; cc < tc; cc += nt >> 6)
+#pragma unroll 4
+            for (int r = tid & 63; r < m; r += 64) d[(unsigned)cc * sl + r + 1] = S[R0 + cc * pitch + place(r)];
+    } else {
+        const int lgT = 31 - __clz(L.T), cc = tid & (L.T - 1);
+        if (cc < tc)
+#pragma unroll 4
+            for (int r = tid >> lgT; r < m; r += nt >> lgT) d[(unsigned)(r + 1) * st + cc] = S[R0 + cc * pitch + place(r)];
     }
 }
 
@@ -1339,15 +1229,11 @@ struct vvt_run {
     hipStream_t stream2 = nullptr;
     double *S2 = nullptr, *T2 = nullptr, *cp2 = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
-    // the x derivatives run on the second stream beside the y and z ones,
-    // with checkpoints of their own (4 jobs)
-    double *ckpx = nullptr;
+    // the x derivatives run on the second stream beside the y and z ones
     hipEvent_t forkd = nullptr, joind = nullptr;
     // the stream and work arrays launch_rhs / launch_poisson use
     hipStream_t cur = nullptr;
     double *cS = nullptr, *cT = nullptr, *ccp = nullptr;
-    double *ckp = nullptr;        // checkpoints of the y/z derivative lines: 8 jobs x ckp_seg x ckp_lines
-    int ckp_seg = 0, ckp_lines = 0;
     YTrans yt;                    // y modes by FFT where np fits (ytrans_fits)
     bool yfft = false;
     double *heat = nullptr;       // 2 nr column sums, trans1, trans2, then the flux terms
@@ -1380,7 +1266,7 @@ hipError_t upload(T **dst, const std::vector<T> &src)
 
 // the tables of a compact line, as the oracle (and the reference's tdma)
 // forms them: rows 1-4-1, type 1's end rows (1, 2) and (2, 1)
-void compact_tables(int type, int m, std::vector<double> &out)
+bool compact_tables(int type, int m, std::vector<double> &out)
 {
     std::vector<double> a(m + 1, 1.0), b(m + 1, 4.0), c(m + 1, 1.0), fact(m + 1, 0.0);
     if (type == 1) {
@@ -1399,6 +1285,11 @@ void compact_tables(int type, int m, std::vector<double> &out)
     out.insert(out.end(), b.begin(), b.end());
     out.insert(out.end(), c.begin(), c.end());
     out.insert(out.end(), rb.begin(), rb.end());
+    std::vector<double> pk;
+    const bool ok = vv::line_pack_head(pk, fact.data() + 1, b.data() + 1, c.data() + 1, m - 1, true,
+                                       {fact[m], b[m], 1.0 / b[m]});
+    out.insert(out.end(), pk.begin(), pk.end());
+    return ok;
 }
 
 // (field, axis) -> (type, m, n1, n2): the staggering of A, B, C, th
@@ -1529,7 +1420,6 @@ int setup_poisson(vvt_run *r)
     const size_t w2 = kmax * mmax * sizeof(double);
     if (hipMalloc(&r->S2, w2) == hipSuccess && hipMalloc(&r->T2, w2) == hipSuccess &&
         hipMalloc(&r->cp2, w2) == hipSuccess &&
-        hipMalloc(&r->ckpx, 4 * (size_t)r->ckp_seg * r->ckp_lines * sizeof(double)) == hipSuccess &&
         hipStreamCreateWithFlags(&r->stream2, hipStreamNonBlocking) == hipSuccess &&
         hipEventCreateWithFlags(&r->fork, hipEventDisableTiming) == hipSuccess &&
         hipEventCreateWithFlags(&r->join, hipEventDisableTiming) == hipSuccess &&
@@ -1537,7 +1427,7 @@ int setup_poisson(vvt_run *r)
         hipEventCreateWithFlags(&r->joind, hipEventDisableTiming) == hipSuccess)
         return VV_OK;
     (void)hipGetLastError();
-    for (double **p : {&r->S2, &r->T2, &r->cp2, &r->ckpx})
+    for (double **p : {&r->S2, &r->T2, &r->cp2})
         if (*p) { (void)hipFree(*p); *p = nullptr; }
     if (r->stream2) { (void)hipStreamDestroy(r->stream2); r->stream2 = nullptr; }
     for (hipEvent_t *e : {&r->fork, &r->join, &r->forkd, &r->joind})
@@ -1581,70 +1471,80 @@ VF vfields(vvt_run *r)
     return F;
 }
 
+// How the lines of m rows, `lines` of them along `axis`, are split.  8 lanes a
+// line leave a lane 64 rows of 512 and its 40 rows of warm-up (y and z lines
+// at 512x256x256: 1.08 ms; 4 lanes 1.14, 16 lanes 1.26), and more only where
+// the lines are too few for a machine's wavefronts.  T: 16 lines along y and
+// z, a row's 128 bytes (8 lines: 1.27 ms), 8 along x, whose lines are
+// contiguous anyway (x lines 0.67 ms; 16 lines 0.75), within 80 KB, for two
+// workgroups a CU.
+vv::LineTile line_tile(int m, long long lines, int axis)
+{
+    const int N = m - 1, nb = vv::lblocks(N) - vv::lheadb(N), pitch = vv::lpitch(N, 1);
+    int P = 8;
+    while (P < 64 && lines * P < 64 * 2048 && vv::line_mb(nb, P) > 1) P *= 2;
+    vv::LineTile L;
+    L.P = P;
+    L.lgP = __builtin_ctz((unsigned)P);
+    L.mb = vv::line_mb(nb, P);
+    L.T = axis ? std::min(16, 512 / P) : 8;
+    while (L.T > 1 && L.T * pitch > 10240) L.T /= 2;
+    return L;
+}
+
+// The threads of its workgroup: as the lanes that solve are few, the others
+// are there for the loads in flight, one for each 8 rows of a y or z tile (y
+// and z lines: 512 threads 1.08 ms, 256 1.18; at 100x42x50, where they would
+// have nothing to load, 128 and 512 threads 31 and 39 us) and four wavefronts
+// for x (0.67 ms; two 0.78, eight 0.94).
+unsigned line_threads(const vv::LineTile &L, int m, int axis)
+{
+    int n = 64;
+    while (n < 512 && n < (axis ? L.T * vv::lblocks(m) : 256)) n *= 2;
+    return (unsigned)std::max(n, L.T * L.P);
+}
+
 int launch_derivatives(vvt_run *r)
 {
-    DJobs J;
-    int nyz = 0, nx = 0, maxm = 0, maxmx = 0, nlx = 0;
-    double byz = 0.0, bx = 0.0;
+    // one launch per axis: a launch has one workgroup size and LDS size
+    DJobs J[3]{};
+    struct Shape { unsigned grid = 0, threads = 64; size_t lds = 0; int n = 0; double bytes = 0.0; } sh[3];
     const double *src[4] = {r->f[VV3_A], r->f[VV3_B], r->f[VV3_C], r->f[VV3_TH]};
     const double dri[3] = {1.0 / r->dr, 1.0 / r->dp, 1.0 / r->dz};
     for (int d = 0; d < 12; ++d) {
         const DSpec s = dspec(r, d);
-        const int nl = (d % 3 == 0) ? 64 : 1;
-        J.j[d] = DJob{src[d / 3], r->dv[d], r->tabs + r->tab_off[d], d % 3, s.type, s.m, s.n1, s.n2, nl, dri[d % 3]};
-        const double b = 8.0 * (2.0 * s.m + 2.0) * s.n1 * s.n2;
-        if (d % 3 == 0) bx += b;
-        else byz += b;
-        if (d % 3 == 0) {
-            nx = std::max(nx, ((s.n1 + nl - 1) / nl) * s.n2);
-            maxmx = std::max(maxmx, s.m);
-            nlx = std::max(nlx, s.n1 * s.n2);
-        } else {
-            nyz = std::max(nyz, s.n1 * s.n2);
-            maxm = std::max(maxm, s.m);
-        }
+        Shape &h = sh[d % 3];
+        DJob &j = J[d % 3].j[h.n++];
+        j = DJob{src[d / 3], r->dv[d], r->tabs + r->tab_off[d], d % 3, s.type, s.m, s.n1, s.n2,
+                 line_tile(s.m, 4LL * s.n1 * s.n2, d % 3), dri[d % 3]};
+        h.bytes += 8.0 * (2.0 * s.m + 2.0) * s.n1 * s.n2;
+        h.grid = std::max(h.grid, ((unsigned)((s.n1 + j.L.T - 1) / j.L.T) * s.n2 + 7) / 8 * 8);
+        h.threads = std::max(h.threads, line_threads(j.L, s.m, d % 3));
+        h.lds = std::max(h.lds, sizeof(double) * (vv::LTC + 4 * vv::LHEAD + (size_t)j.L.T * vv::lpitch(s.m - 1, 1)));
     }
-    // the y and z jobs in one launch: jobs 1, 2, 4, 5, ... are reached as
-    // j0 + blockIdx.y with blockIdx.y over a compacted list
-    DJobs Jyz;
-    int c = 0;
-    for (int d = 0; d < 12; ++d)
-        if (d % 3 != 0) Jyz.j[c++] = J.j[d];
-    if (r->stream2 && !r->prof) {   // the x jobs start from the state the y and z jobs read
+    auto go = [&](int axis, hipStream_t st) {
+        hipLaunchKernelGGL(k_t_deriv, dim3(sh[axis].grid, sh[axis].n), dim3(sh[axis].threads), sh[axis].lds, st, geo(r),
+                           J[axis]);
+    };
+    const bool two = r->stream2 && !r->prof;
+    if (two) {   // the x jobs start from the state the y and z jobs read
         VV_HIP(hipEventRecord(r->forkd, r->stream));
         VV_HIP(hipStreamWaitEvent(r->stream2, r->forkd, 0));
     }
     {
-        Prof p(r, VVT_K_DERIV_YZ, byz);
-        if (c > 8 || maxm > r->ckp_seg * CK || nyz > r->ckp_lines) {
-            vv::set_error("vvt: derivative checkpoints exceed their buffer");
-            return VV_EINVAL;
-        }
-        if (maxm <= DYZ_LDS_MAXM)
-            hipLaunchKernelGGL(k_t_deriv_yz<true>, dim3(nblk(nyz, WG), c), dim3(WG),
-                               4 * (size_t)(maxm + 1) * sizeof(double), r->stream, geo(r), Jyz, 0, r->ckp,
-                               r->ckp_seg, r->ckp_lines);
-        else
-            hipLaunchKernelGGL(k_t_deriv_yz<false>, dim3(nblk(nyz, WG), c), dim3(WG), 0, r->stream, geo(r), Jyz, 0,
-                               r->ckp, r->ckp_seg, r->ckp_lines);
+        Prof p(r, VVT_K_DERIV_YZ, sh[1].bytes + sh[2].bytes);
+        go(1, r->stream);
+        go(2, r->stream);
     }
     {
-        Prof p(r, VVT_K_DERIV_X, bx);
-        if ((maxmx + CX - 1) / CX > r->ckp_seg || nlx > r->ckp_lines) {
-            vv::set_error("vvt: derivative checkpoints exceed their buffer");
-            return VV_EINVAL;
-        }
-        if (r->stream2 && !r->prof) {
-            // on the second stream (from the state the y and z jobs also
-            // read), joined before the explicit updates read the derivatives
-            hipLaunchKernelGGL(k_t_deriv_x, dim3(nx, 4), dim3(64), 0, r->stream2, geo(r), J, r->ckpx, r->ckp_seg,
-                               r->ckp_lines);
-            VV_HIP(hipEventRecord(r->joind, r->stream2));
-            VV_HIP(hipStreamWaitEvent(r->stream, r->joind, 0));
-        } else {
-            hipLaunchKernelGGL(k_t_deriv_x, dim3(nx, 4), dim3(64), 0, r->stream, geo(r), J, r->ckp, r->ckp_seg,
-                               r->ckp_lines);
-        }
+        // on the second stream (from the state the y and z jobs also read),
+        // joined before the explicit updates read the derivatives
+        Prof p(r, VVT_K_DERIV_X, sh[0].bytes);
+        go(0, two ? r->stream2 : r->stream);
+    }
+    if (two) {
+        VV_HIP(hipEventRecord(r->joind, r->stream2));
+        VV_HIP(hipStreamWaitEvent(r->stream, r->joind, 0));
     }
     VV_HIP(hipGetLastError());
     return VV_OK;
@@ -1924,20 +1824,12 @@ int vvt_create(const vvt_config *cfg, int device, vvt_run **out)
         for (int d = 0; d < 12; ++d) {
             const DSpec s = dspec(r, d);
             r->tab_off[d] = tabs.size();
-            compact_tables(s.type, s.m, tabs);
+            if (!compact_tables(s.type, s.m, tabs)) {
+                vv::set_error("vvt_create: a compact system's rows do not settle");
+                return fail(VV_EINVAL);
+            }
         }
         if (upload(&r->tabs, tabs) != hipSuccess) return fail(VV_ENOMEM);
-        // checkpoints of the derivative lines (y and z: 8 jobs, one per CK
-        // rows; then x: 4 jobs, one per CX rows, in the same buffer)
-        int segs = 0, nl = 0;
-        for (int d = 0; d < 12; ++d) {
-            const DSpec s = dspec(r, d);
-            segs = std::max(segs, (s.m + ((d % 3 == 0) ? CX : CK) - 1) / ((d % 3 == 0) ? CX : CK));
-            nl = std::max(nl, s.n1 * s.n2);
-        }
-        r->ckp_seg = segs;
-        r->ckp_lines = nl;
-        if (hipMalloc(&r->ckp, 8 * (size_t)r->ckp_seg * nl * sizeof(double)) != hipSuccess) return fail(VV_ENOMEM);
     }
     {   // column sums (2 nr), trans1 and trans2, then the terms of rows k = np/2 .. np
         const size_t nh = 2 * (size_t)r->nr + 2 + 2 * (size_t)(cfg->np - cfg->np / 2 + 1) * r->nr;
@@ -1970,13 +1862,12 @@ int vvt_destroy(vvt_run *r)
             for (double *p : {O.W, O.Wi, O.ly, O.V, O.Vinv, O.lz, O.rt})
                 if (p) (void)hipFree(p);
         if (r->stream2) (void)hipStreamSynchronize(r->stream2);
-        for (double *p : {r->tabs, r->S, r->T, r->cp, r->S2, r->T2, r->cp2, r->ckpx, r->heat, r->kepart})
+        for (double *p : {r->tabs, r->S, r->T, r->cp, r->S2, r->T2, r->cp2, r->heat, r->kepart})
             if (p) (void)hipFree(p);
         for (hipEvent_t e : {r->fork, r->join, r->forkd, r->joind})
             if (e) (void)hipEventDestroy(e);
         if (r->stream2) (void)hipStreamDestroy(r->stream2);
         ytrans_free(r->yt);
-        if (r->ckp) (void)hipFree(r->ckp);
         for (hipEvent_t e : r->ev)
             if (e) (void)hipEventDestroy(e);
         if (r->stream) (void)hipStreamDestroy(r->stream);
