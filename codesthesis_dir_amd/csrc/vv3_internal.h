@@ -2,6 +2,7 @@
 #pragma once
 
 #include "vv_fft.h"
+#include "vv_rlines.h"
 #include "vv_internal.h"
 
 #include "../../include/vvmi3.h"
@@ -44,8 +45,8 @@ struct Poisson3 {
     double *lphi = nullptr;  // nm: 2 cos(2 pi mode/np) - 2
     double *S = nullptr;     // np x mmax: phi spectra, then the z-inverse result
     double *T = nullptr;     // np x mmax: z spectra, (i, l) with l fastest
-    double *cp = nullptr;    // nm x mmax: elimination factors of the r solves
-    double *S2 = nullptr, *T2 = nullptr, *cp2 = nullptr;   // a second set (a solve beside another), or none
+    vv::RSolve rs;           // the r solves, nm modes of two parts
+    double *S2 = nullptr, *T2 = nullptr;   // a second set (a solve beside another), or none
     double *tw = nullptr;    // the FFT's tables (vv_fft.h)
     vv::MrTables mr;         // phi transforms' plan
     vv::MrPlan plan{};       // with its device pointers

@@ -9,8 +9,8 @@
 //   1. a real DFT over k (a GEMM with a cos/sin table): one (r,z) problem
 //      per Fourier mode and part,
 //   2. the z eigenbasis: y = V^-1 x along j (a batched GEMM),
-//   3. per (mode, z eigenvalue) one banded system in r, eliminated by a
-//      thread (Thomas, with the two wall rows' extra coefficient folded in),
+//   3. per (mode, z eigenvalue) one banded system in r, its two
+//      sweeps run as chunks (vv_rlines.h, the two wall rows' extra coefficient removed),
 //   4. x = V y along j, the inverse DFT into psi.
 // The result is the exact solution of the reference's discrete equations to
 // rounding (the reference iterates multigrid V-cycles to an absolute
@@ -219,116 +219,6 @@ __global__ void __launch_bounds__(256) k3_psi_pre(Geo g, int which, int i1, int 
     if (i > ri || j > rj) return;
     psip[t] = psi[t];
     if (!(i >= 1 && i <= i1 && j >= 1 && j <= j1)) psi[t] = 0.0;
-}
-
-// 3. per (mode, l): (R + lphi(mode) diag(1/(dp r)^2) + lz(l)) x = y for the
-// cos part (spectral row mode) and, for 0 < mode < np/2, the sin part (row
-// np/2 + mode), x overwriting y in T (layout [q][i][l]).  Row 1 has an extra
-// coefficient e1 at i = 3, removed with row 2; row i1 has en at i1 - 2,
-// removed with the eliminated row i1 - 2.  Thomas factors go to cp.
-__global__ void __launch_bounds__(64) k3_rsolve(double *__restrict__ T, double *__restrict__ cp,
-                                                 const double *__restrict__ rt, const double *__restrict__ lz,
-                                                 const double *__restrict__ lphi, int i1, int j1, int np, double e1,
-                                                 double en)
-{
-    const int nm = np / 2 + 1;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nm * j1) return;
-    const int mode = t / j1, l = t - mode * j1;
-    const size_t mt = (size_t)i1 * j1;
-    const bool two = (mode > 0 && 2 * mode < np);
-    double *__restrict__ xc = T + (size_t)mode * mt + l;
-    double *__restrict__ xs = T + (size_t)(two ? np / 2 + mode : mode) * mt + l;
-    double *__restrict__ c = cp + (size_t)mode * mt + l;
-    const double *sub = rt, *dia = rt + i1, *sup = rt + 2 * i1, *ir2 = rt + 3 * i1;
-    const double mu = lphi[mode], lam = lz[l];
-    auto diag = [&](int i) { return dia[i] + mu * ir2[i] + lam; };
-    double d0 = diag(0), s0 = sup[0], yc = xc[0], ys = two ? xs[0] : 0.0;
-    if (e1 != 0.0) {
-        const double f = e1 / sup[1];
-        d0 -= f * sub[1];
-        s0 -= f * diag(1);
-        yc -= f * xc[j1];
-        if (two) ys -= f * xs[j1];
-    }
-    double cprev = s0 / d0;
-    yc /= d0;
-    ys /= d0;
-    c[0] = cprev;
-    xc[0] = yc;
-    if (two) xs[0] = ys;
-    // rows 1 .. i1-2 in groups of U with their loads issued ahead
-    constexpr int U = 8;
-    int i = 1;
-    for (; i + U <= i1 - 1; i += U) {
-        double rcu[U], rsu[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            rcu[u] = xc[(size_t)(i + u) * j1];
-            rsu[u] = two ? xs[(size_t)(i + u) * j1] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int ii = i + u;
-            const size_t o = (size_t)ii * j1;
-            const double a = sub[ii];
-            const double den = diag(ii) - a * cprev;
-            cprev = sup[ii] / den;
-            yc = (rcu[u] - a * yc) / den;
-            ys = (rsu[u] - a * ys) / den;
-            c[o] = cprev;
-            xc[o] = yc;
-            if (two) xs[o] = ys;
-        }
-    }
-    for (; i < i1; ++i) {
-        const size_t o = (size_t)i * j1;
-        double a = sub[i], rc = xc[o], rs = two ? xs[o] : 0.0;
-        if (i == i1 - 1 && en != 0.0) {
-            const size_t o2 = (size_t)(i - 2) * j1;
-            a -= en * c[o2];
-            rc -= en * xc[o2];
-            if (two) rs -= en * xs[o2];
-        }
-        const double den = diag(i) - a * cprev;
-        cprev = sup[i] / den;
-        yc = (rc - a * yc) / den;
-        ys = (rs - a * ys) / den;
-        c[o] = cprev;
-        xc[o] = yc;
-        if (two) xs[o] = ys;
-    }
-    i = i1 - 2;
-    for (; i - U + 1 >= 0; i -= U) {
-        double fu[U], xcu[U], xsu[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const size_t o = (size_t)(i - u) * j1;
-            fu[u] = c[o];
-            xcu[u] = xc[o];
-            xsu[u] = two ? xs[o] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const size_t o = (size_t)(i - u) * j1;
-            yc = xcu[u] - fu[u] * yc;
-            xc[o] = yc;
-            if (two) {
-                ys = xsu[u] - fu[u] * ys;
-                xs[o] = ys;
-            }
-        }
-    }
-    for (; i >= 0; --i) {
-        const size_t o = (size_t)i * j1;
-        const double f = c[o];
-        yc = xc[o] - f * yc;
-        xc[o] = yc;
-        if (two) {
-            ys = xs[o] - f * ys;
-            xs[o] = ys;
-        }
-    }
 }
 
 // ---------------------------------------------------------------- host side
@@ -683,12 +573,16 @@ int poisson3_setup(Poisson3 &P, const Geo &g)
     }
     VV_HIP(hipMalloc(&P.S, (size_t)np * mmax * sizeof(double)));
     VV_HIP(hipMalloc(&P.T, (size_t)np * mmax * sizeof(double)));
-    VV_HIP(hipMalloc(&P.cp, (size_t)nm * mmax * sizeof(double)));
+    for (int o = 0; o < 3; ++o) {
+        const PoissonOp &O = P.op[o];
+        P.rs.op[o] = vv::RLines{O.rt, O.lz, P.lphi, nullptr, O.i1, O.j1, nm, np / 2, 1, O.e1, O.en};
+    }
+    VV_HIP(vv::rsolve_setup(P.rs));
+    if (P.rs.shared) return VV_OK;
     if (hipMalloc(&P.S2, (size_t)np * mmax * sizeof(double)) != hipSuccess ||
-        hipMalloc(&P.T2, (size_t)np * mmax * sizeof(double)) != hipSuccess ||
-        hipMalloc(&P.cp2, (size_t)nm * mmax * sizeof(double)) != hipSuccess) {
+        hipMalloc(&P.T2, (size_t)np * mmax * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
-        for (double **q : {&P.S2, &P.T2, &P.cp2})
+        for (double **q : {&P.S2, &P.T2})
             if (*q) { (void)hipFree(*q); *q = nullptr; }
     }
     return VV_OK;
@@ -696,9 +590,10 @@ int poisson3_setup(Poisson3 &P, const Geo &g)
 
 void poisson3_free(Poisson3 &P)
 {
-    for (double *p : {P.W, P.Wi, P.lphi, P.S, P.T, P.cp, P.S2, P.T2, P.cp2, P.tw})
+    for (double *p : {P.W, P.Wi, P.lphi, P.S, P.T, P.S2, P.T2, P.tw})
         if (p) (void)hipFree(p);
-    P.W = P.Wi = P.lphi = P.S = P.T = P.cp = P.S2 = P.T2 = P.cp2 = P.tw = nullptr;
+    P.W = P.Wi = P.lphi = P.S = P.T = P.S2 = P.T2 = P.tw = nullptr;
+    vv::rsolve_free(P.rs);
     for (auto &O : P.op) {
         for (double *p : {O.V, O.Vinv, O.rt, O.lz})
             if (p) (void)hipFree(p);
@@ -710,8 +605,8 @@ int poisson3_launch(const Poisson3 &P, const Geo &g, int which, double *psi, dou
                     hipStream_t s, bool second)
 {
     const PoissonOp &O = P.op[which - 1];
-    double *const S = second ? P.S2 : P.S, *const T = second ? P.T2 : P.T, *const cpw = second ? P.cp2 : P.cp;
-    const int nm = P.nm, np = P.np, i1 = O.i1, j1 = O.j1, mt = O.m;
+    double *const S = second ? P.S2 : P.S, *const T = second ? P.T2 : P.T;
+    const int np = P.np, i1 = O.i1, j1 = O.j1, mt = O.m;
     hipLaunchKernelGGL(k3_psi_pre, dim3((unsigned)((g.ldi * g.ldj + 255) / 256), np + 1), dim3(256), 0, s, g, which,
                        i1, j1, psi, psip);
     // LP line pairs per workgroup (a power of two), few enough for about 256
@@ -735,8 +630,7 @@ int poisson3_launch(const Poisson3 &P, const Geo &g, int which, double *psi, dou
         gemm_f64<true, false>(PhiFwd{P.W, np, mt, np, rhs, S, i1, g.ldi, g.ldj}, 1, s);
     if (O.zsplit) vv::zsplit_fwd(O.Vinv, S, T, i1, j1, np, s);
     else gemm_f64<false, true>(ZFwd{O.Vinv, i1, j1, j1, S, T, mt}, np, s);
-    hipLaunchKernelGGL(k3_rsolve, dim3((unsigned)((nm * j1 + 63) / 64)), dim3(64), 0, s, T, cpw,
-                       (const double *)O.rt, (const double *)O.lz, (const double *)P.lphi, i1, j1, np, O.e1, O.en);
+    vv::rsolve_launch(P.rs, which - 1, T, s);
     if (O.zsplit) vv::zsplit_inv(O.V, T, S, i1, j1, np, s);
     else gemm_f64<true, true>(ZInv{O.V, j1, i1, j1, T, S, mt}, np, s);
     if (P.fft && R == 0) inv(k3_fft_inv<0>);

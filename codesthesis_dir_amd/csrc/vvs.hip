@@ -115,8 +115,9 @@ struct SOp {
 
 struct SPoisson {
     SOp op[3];
-    double *S = nullptr, *T = nullptr, *cp = nullptr;
-    double *S2 = nullptr, *T2 = nullptr, *cp2 = nullptr;   // a second set: v's solve beside w's and u's
+    double *S = nullptr, *T = nullptr;
+    vv::RSolve rs;
+    double *S2 = nullptr, *T2 = nullptr;   // a second set: v's solve beside w's and u's
     bool fft = false;     // phi transforms by FFT (ytrans_fits) instead of the W / Wi GEMMs
     vvt::YTrans yt;
 };
@@ -821,89 +822,6 @@ struct PhiInv {
     }
 };
 
-// 3. per (phi mode q, z eigenvalue l) the r system (R + lphi(q) diag(1/(dp
-// r)^2) + lz(l)) x = y, x overwriting y in T (layout [q][i][l]); row 1 has an
-// extra coefficient e1 two points inward, removed with row 2, row i1 one
-// (en) removed with the eliminated row i1 - 2.  Thomas factors go to cp.
-__global__ void __launch_bounds__(64) ks_rsolve(double *__restrict__ T, double *__restrict__ cp,
-                                                 const double *__restrict__ rt, const double *__restrict__ lz,
-                                                 const double *__restrict__ lphi, int i1, int j1, int k1, double e1,
-                                                 double en)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= k1 * j1) return;
-    const int q = t / j1, l = t - q * j1;
-    const size_t mt = (size_t)i1 * j1;
-    double *__restrict__ x = T + (size_t)q * mt + l;
-    double *__restrict__ c = cp + (size_t)q * mt + l;
-    const double *sub = rt, *dia = rt + i1, *sup = rt + 2 * i1, *ir2 = rt + 3 * i1;
-    const double mu = lphi[q], lam = lz[l];
-    auto diag = [&](int i) { return dia[i] + mu * ir2[i] + lam; };
-    double d0 = diag(0), s0 = sup[0], y = x[0];
-    if (e1 != 0.0) {
-        const double f = e1 / sup[1];
-        d0 -= f * sub[1];
-        s0 -= f * diag(1);
-        y -= f * x[j1];
-    }
-    double cprev = s0 / d0;
-    y /= d0;
-    c[0] = cprev;
-    x[0] = y;
-    // rows 1 .. i1-2 in groups of U with their loads issued ahead
-    constexpr int U = 8;
-    int i = 1;
-    for (; i + U <= i1 - 1; i += U) {
-        double rv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) rv[u] = x[(size_t)(i + u) * j1];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const size_t o = (size_t)(i + u) * j1;
-            const double a = sub[i + u];
-            const double den = diag(i + u) - a * cprev;
-            cprev = sup[i + u] / den;
-            y = (rv[u] - a * y) / den;
-            c[o] = cprev;
-            x[o] = y;
-        }
-    }
-    for (; i < i1; ++i) {
-        const size_t o = (size_t)i * j1;
-        double a = sub[i], rv = x[o];
-        if (i == i1 - 1 && en != 0.0) {
-            const size_t o2 = (size_t)(i - 2) * j1;
-            a -= en * c[o2];
-            rv -= en * x[o2];
-        }
-        const double den = diag(i) - a * cprev;
-        cprev = sup[i] / den;
-        y = (rv - a * y) / den;
-        c[o] = cprev;
-        x[o] = y;
-    }
-    i = i1 - 2;
-    for (; i - U + 1 >= 0; i -= U) {
-        double fu[U], xu[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const size_t o = (size_t)(i - u) * j1;
-            fu[u] = c[o];
-            xu[u] = x[o];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            y = xu[u] - fu[u] * y;
-            x[(size_t)(i - u) * j1] = y;
-        }
-    }
-    for (; i >= 0; --i) {
-        const size_t o = (size_t)i * j1;
-        y = x[o] - c[o] * y;
-        x[o] = y;
-    }
-}
-
 template <class T>
 hipError_t upload(T **dst, const std::vector<T> &src)
 {
@@ -959,7 +877,7 @@ int spoisson_setup(SPoisson &P, const Geo &g)
     using vv::set_error;
     const double pi = std::acos(-1.0);
     const double hhz = g.dz * g.dz, hhp = g.dp * g.dp;
-    size_t smax = 0, cmax = 0;
+    size_t smax = 0;
     P.fft = vvt::ytrans_fits(g.np);
     if (P.fft) {
         const int st = vvt::ytrans_setup(P.yt, g.np, g.ldi, g.ldj);
@@ -1014,16 +932,19 @@ int spoisson_setup(SPoisson &P, const Geo &g)
         VV_HIP(upload(&O.lz, lam));
         VV_HIP(upload(&O.rt, rt));
         smax = std::max(smax, (size_t)k1 * O.m);
-        cmax = std::max(cmax, (size_t)k1 * O.m);
     }
     VV_HIP(hipMalloc(&P.S, smax * sizeof(double)));
     VV_HIP(hipMalloc(&P.T, smax * sizeof(double)));
-    VV_HIP(hipMalloc(&P.cp, cmax * sizeof(double)));
+    for (int o = 0; o < 3; ++o) {
+        const SOp &O = P.op[o];
+        P.rs.op[o] = vv::RLines{O.rt, O.lz, O.lphi, nullptr, O.i1, O.j1, O.k1, 0, 1, O.e1, O.en};
+    }
+    VV_HIP(vv::rsolve_setup(P.rs));
+    if (P.rs.shared) return VV_OK;
     // the second set is optional: without it the solves run in turn
-    if (hipMalloc(&P.S2, smax * sizeof(double)) != hipSuccess || hipMalloc(&P.T2, smax * sizeof(double)) != hipSuccess ||
-        hipMalloc(&P.cp2, cmax * sizeof(double)) != hipSuccess) {
+    if (hipMalloc(&P.S2, smax * sizeof(double)) != hipSuccess || hipMalloc(&P.T2, smax * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
-        for (double **q : {&P.S2, &P.T2, &P.cp2})
+        for (double **q : {&P.S2, &P.T2})
             if (*q) { (void)hipFree(*q); *q = nullptr; }
     }
     return VV_OK;
@@ -1031,9 +952,10 @@ int spoisson_setup(SPoisson &P, const Geo &g)
 
 void spoisson_free(SPoisson &P)
 {
-    for (double *p : {P.S, P.T, P.cp, P.S2, P.T2, P.cp2})
+    for (double *p : {P.S, P.T, P.S2, P.T2})
         if (p) (void)hipFree(p);
-    P.S = P.T = P.cp = P.S2 = P.T2 = P.cp2 = nullptr;
+    P.S = P.T = P.S2 = P.T2 = nullptr;
+    vv::rsolve_free(P.rs);
     vvt::ytrans_free(P.yt);
     for (auto &O : P.op) {
         for (double *p : {O.W, O.Wi, O.lphi, O.V, O.Vinv, O.lz, O.rt})
@@ -1046,7 +968,7 @@ int spoisson_launch(const SPoisson &P, const Geo &g, int which, double *psi, dou
                     hipStream_t s, bool second)
 {
     const SOp &O = P.op[which - 1];
-    double *S = second ? P.S2 : P.S, *T = second ? P.T2 : P.T, *cp = second ? P.cp2 : P.cp;
+    double *S = second ? P.S2 : P.S, *T = second ? P.T2 : P.T;
     const int i1 = O.i1, j1 = O.j1, k1 = O.k1, mt = O.m;
     const dim3 pg((unsigned)((g.ldi * g.ldj + 255) / 256), (unsigned)(g.np + 2));
     hipLaunchKernelGGL(ks_psi_pre, pg, dim3(256), 0, s, g, which, (const double *)psi, psip);
@@ -1054,8 +976,7 @@ int spoisson_launch(const SPoisson &P, const Geo &g, int which, double *psi, dou
     else vv::gemm_f64<true, false>(PhiFwd{O.W, k1, mt, k1, rhs, S, i1, g.ldi, g.ldj}, 1, s);
     if (O.zsplit) vv::zsplit_fwd(O.Vinv, S, T, i1, j1, k1, s);
     else vv::gemm_f64<false, true>(ZFwd{O.Vinv, i1, j1, j1, S, T, mt}, k1, s);
-    hipLaunchKernelGGL(ks_rsolve, dim3((unsigned)((k1 * j1 + 63) / 64)), dim3(64), 0, s, T, cp,
-                       (const double *)O.rt, (const double *)O.lz, (const double *)O.lphi, i1, j1, k1, O.e1, O.en);
+    vv::rsolve_launch(P.rs, which - 1, T, s);
     if (O.zsplit) vv::zsplit_inv(O.V, T, S, i1, j1, k1, s);
     else vv::gemm_f64<true, true>(ZInv{O.V, j1, i1, j1, T, S, mt}, k1, s);
     if (P.fft) vvt::ytrans_inv(P.yt, which == 2, S, psi, i1, mt, s);

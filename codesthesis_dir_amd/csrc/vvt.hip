@@ -17,8 +17,8 @@
 // LDS when np has no prime factor above 13 (k_t_yfft_*) and as FP64
 // matrix-core GEMMs otherwise; the z rows are diagonalised once (the eigenbasis of
 // rot3dmg.f's z rows, shared with the annulus solver); what remains per
-// (y mode, z eigenvalue) is one banded system along x, eliminated by one
-// thread (Thomas, the closure rows' third coefficient folded in).
+// (y mode, z eigenvalue) is one banded system along x, its two
+// sweeps run as chunks (vv_rlines.h, the closure rows' third coefficient removed).
 
 #include "vv3_internal.h"
 #include "vv_fft.h"
@@ -963,121 +963,6 @@ __global__ void __launch_bounds__(WG) k_t_psi_post(TGeo g, double *psi)
     psi[(unsigned)(g.np + 1) * pl + tp] = psi[(unsigned)g.np * pl + tp];
 }
 
-// per (y mode q, z eigenvalue l): (D_x + mu_q + lz_l) x = y along i, x
-// overwriting y in T (layout [q][i][l]).  Row 1 has an extra coefficient e1
-// two points inward, removed with row 2; row i1 has en, removed with the
-// eliminated row i1 - 2.  Thomas elimination, one thread per line (threads
-// on consecutive l: coalesced), without a factor array: the forward sweep
-// keeps only the state (c, y) entering every XCK-th row (in ckp, 2/XCK of
-// T), and the back substitution takes the segments from the last: it reads
-// the segment's right-hand sides again, repeats their elimination in
-// registers from the state before it -- the same operations, so the same
-// bits -- and substitutes back.  T is read twice and written once (against
-// reading it twice, writing it twice and the factors once each).
-constexpr int XCK = 16;
-
-__global__ void __launch_bounds__(64) k_t_xsolve(double *__restrict__ T, double *__restrict__ ckp,
-                                                     const double *__restrict__ rt, const double *__restrict__ lz,
-                                                     const double *__restrict__ ly, int i1, int j1, int k1, double e1,
-                                                     double en)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nlines = k1 * j1;
-    if (t >= nlines) return;
-    const int q = t / j1, l = t - q * j1;
-    const size_t mt = (size_t)i1 * j1;
-    double *__restrict__ x = T + (size_t)q * mt + l;
-    // (c, y) entering segment sg at ck[(2 sg + w) nlines]
-    double *__restrict__ ck = ckp + t;
-    const double *sub = rt, *dia = rt + i1, *sup = rt + 2 * i1;
-    const double shift = ly[q] + lz[l];
-    const int nseg = (i1 + XCK - 1) / XCK;
-    // row 0, its third coefficient folded in with row 1
-    double d0 = dia[0] + shift, s0 = sup[0];
-    const double x0 = x[0], x1 = x[j1];
-    double f0 = 0.0;
-    if (e1 != 0.0) {
-        f0 = e1 / sup[1];
-        d0 -= f0 * sub[1];
-        s0 -= f0 * (dia[1] + shift);
-    }
-    // one elimination row: a and r as given (the last row's fold applied by the caller)
-    auto row = [&](int i, double a, double r, double &c, double &y) {
-        const double den = dia[i] + shift - a * c;
-        c = sup[i] / den;
-        y = (r - a * y) / den;
-    };
-    auto row0 = [&](double &c, double &y) {
-        y = x0;
-        if (e1 != 0.0) y -= f0 * x1;
-        c = s0 / d0;
-        y /= d0;
-    };
-    // forward sweep: rows in groups of XCK with their loads issued ahead
-    double c, y, c3 = 0.0, y3 = 0.0;   // (c, y) of row i1-3 for the last row's fold
-    row0(c, y);
-    if (i1 == 3) { c3 = c; y3 = y; }
-    for (int sg = 0; sg < nseg; ++sg) {
-        const int r0 = sg * XCK;
-        if (sg > 0) {
-            ck[(size_t)(2 * sg) * nlines] = c;
-            ck[(size_t)(2 * sg + 1) * nlines] = y;
-        }
-        double ru[XCK];
-#pragma unroll
-        for (int u = 0; u < XCK; ++u) ru[u] = (r0 + u < i1) ? x[(size_t)(r0 + u) * j1] : 0.0;
-#pragma unroll
-        for (int u = 0; u < XCK; ++u) {
-            const int i = r0 + u;
-            if (i == 0 || i >= i1) continue;
-            double a = sub[i], r = ru[u];
-            if (i == i1 - 1 && en != 0.0) {
-                a -= en * c3;
-                r -= en * y3;
-            }
-            row(i, a, r, c, y);
-            if (i == i1 - 3) { c3 = c; y3 = y; }
-        }
-    }
-    // back substitution, segment by segment from the last
-    double xn = 0.0;
-    for (int sg = nseg - 1; sg >= 0; --sg) {
-        const int r0 = sg * XCK;
-        double ru[XCK], cv[XCK], yv[XCK];
-#pragma unroll
-        for (int u = 0; u < XCK; ++u) ru[u] = (r0 + u < i1) ? x[(size_t)(r0 + u) * j1] : 0.0;
-        if (sg > 0) {
-            c = ck[(size_t)(2 * sg) * nlines];
-            y = ck[(size_t)(2 * sg + 1) * nlines];
-        }
-#pragma unroll
-        for (int u = 0; u < XCK; ++u) {
-            const int i = r0 + u;
-            if (i < i1) {
-                if (i == 0) {
-                    row0(c, y);
-                } else {
-                    double a = sub[i], r = ru[u];
-                    if (i == i1 - 1 && en != 0.0) {
-                        a -= en * c3;
-                        r -= en * y3;
-                    }
-                    row(i, a, r, c, y);
-                }
-            }
-            cv[u] = c;
-            yv[u] = y;
-        }
-#pragma unroll
-        for (int u = XCK - 1; u >= 0; --u) {
-            const int i = r0 + u;
-            if (i >= i1) continue;
-            xn = (i == i1 - 1) ? yv[u] : yv[u] - cv[u] * xn;
-            x[(size_t)i * j1] = xn;
-        }
-    }
-}
-
 __global__ void __launch_bounds__(WG) k_t_energy(TGeo g, const double *uel, const double *vel, const double *wel,
                                                   double *part)
 {
@@ -1223,17 +1108,18 @@ struct vvt_run {
     double *tabs = nullptr;       // compact elimination tables
     size_t tab_off[12] = {0};
     TankOp op[3];
-    double *S = nullptr, *T = nullptr, *cp = nullptr;   // Poisson work (kmax x mmax each)
+    double *S = nullptr, *T = nullptr;   // Poisson work (kmax x mmax each)
+    vv::RSolve rs;                       // its x systems
     // v's right-hand side and solve run beside w's and u's (one_step): a
     // second stream with work arrays of its own, and the fork / join events
     hipStream_t stream2 = nullptr;
-    double *S2 = nullptr, *T2 = nullptr, *cp2 = nullptr;
+    double *S2 = nullptr, *T2 = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
     // the x derivatives run on the second stream beside the y and z ones
     hipEvent_t forkd = nullptr, joind = nullptr;
     // the stream and work arrays launch_rhs / launch_poisson use
     hipStream_t cur = nullptr;
-    double *cS = nullptr, *cT = nullptr, *ccp = nullptr;
+    double *cS = nullptr, *cT = nullptr;
     YTrans yt;                    // y modes by FFT where np fits (ytrans_fits)
     bool yfft = false;
     double *heat = nullptr;       // 2 nr column sums, trans1, trans2, then the flux terms
@@ -1414,12 +1300,16 @@ int setup_poisson(vvt_run *r)
     }
     VV_HIP(hipMalloc(&r->S, kmax * mmax * sizeof(double)));
     VV_HIP(hipMalloc(&r->T, kmax * mmax * sizeof(double)));
-    VV_HIP(hipMalloc(&r->cp, kmax * mmax * sizeof(double)));
-    r->cur = r->stream; r->cS = r->S; r->cT = r->T; r->ccp = r->cp;
+    for (int o = 0; o < 3; ++o) {
+        const TankOp &O = r->op[o];
+        r->rs.op[o] = vv::RLines{O.rt, O.lz, O.ly, nullptr, O.i1, O.j1, O.k1, 0, 0, O.e1, O.en};
+    }
+    VV_HIP(vv::rsolve_setup(r->rs));
+    r->cur = r->stream; r->cS = r->S; r->cT = r->T;
     // the second solve stream: without its memory the solves run in turn
     const size_t w2 = kmax * mmax * sizeof(double);
+    if (r->rs.shared) return VV_OK;
     if (hipMalloc(&r->S2, w2) == hipSuccess && hipMalloc(&r->T2, w2) == hipSuccess &&
-        hipMalloc(&r->cp2, w2) == hipSuccess &&
         hipStreamCreateWithFlags(&r->stream2, hipStreamNonBlocking) == hipSuccess &&
         hipEventCreateWithFlags(&r->fork, hipEventDisableTiming) == hipSuccess &&
         hipEventCreateWithFlags(&r->join, hipEventDisableTiming) == hipSuccess &&
@@ -1427,7 +1317,7 @@ int setup_poisson(vvt_run *r)
         hipEventCreateWithFlags(&r->joind, hipEventDisableTiming) == hipSuccess)
         return VV_OK;
     (void)hipGetLastError();
-    for (double **p : {&r->S2, &r->T2, &r->cp2})
+    for (double **p : {&r->S2, &r->T2})
         if (*p) { (void)hipFree(*p); *p = nullptr; }
     if (r->stream2) { (void)hipStreamDestroy(r->stream2); r->stream2 = nullptr; }
     for (hipEvent_t *e : {&r->fork, &r->join, &r->forkd, &r->joind})
@@ -1646,10 +1536,7 @@ int launch_poisson(vvt_run *r, int which)
     }
     {   // reads T and writes it (algorithmic: once each)
         Prof p(r, VVT_K_XSOLVE, 8.0 * 2.0 * O.k1 * (double)mt);
-        // checkpoints in cp: 2 ceil(i1/XCK) k1 j1 <= i1 k1 j1 words (i1 >= 5)
-        hipLaunchKernelGGL(k_t_xsolve, dim3(nblk((long long)O.k1 * O.j1, 64)), dim3(64), 0, s, r->cT, r->ccp,
-                           (const double *)O.rt, (const double *)O.lz, (const double *)O.ly, O.i1, O.j1, O.k1, O.e1,
-                           O.en);
+        vv::rsolve_launch(r->rs, which - 1, r->cT, s);
     }
     if (O.zsplit) {
         Prof p(r, VVT_K_ZINV, ftr_zs);
@@ -1756,11 +1643,11 @@ int one_step(vvt_run *r)
         // waits for both
         VV_HIP(hipEventRecord(r->fork, r->stream));
         VV_HIP(hipStreamWaitEvent(r->stream2, r->fork, 0));
-        r->cur = r->stream2; r->cS = r->S2; r->cT = r->T2; r->ccp = r->cp2;
+        r->cur = r->stream2; r->cS = r->S2; r->cT = r->T2;
         st = launch_heat(r);
         if (!st) st = launch_rhs(r, 2);
         if (!st) st = launch_poisson(r, 2);
-        r->cur = r->stream; r->cS = r->S; r->cT = r->T; r->ccp = r->cp;
+        r->cur = r->stream; r->cS = r->S; r->cT = r->T;
         if (st) return st;
         VV_HIP(hipEventRecord(r->join, r->stream2));
         for (int w = 1; w <= 3; w += 2) {
@@ -1862,12 +1749,13 @@ int vvt_destroy(vvt_run *r)
             for (double *p : {O.W, O.Wi, O.ly, O.V, O.Vinv, O.lz, O.rt})
                 if (p) (void)hipFree(p);
         if (r->stream2) (void)hipStreamSynchronize(r->stream2);
-        for (double *p : {r->tabs, r->S, r->T, r->cp, r->S2, r->T2, r->cp2, r->heat, r->kepart})
+        for (double *p : {r->tabs, r->S, r->T, r->S2, r->T2, r->heat, r->kepart})
             if (p) (void)hipFree(p);
         for (hipEvent_t e : {r->fork, r->join, r->forkd, r->joind})
             if (e) (void)hipEventDestroy(e);
         if (r->stream2) (void)hipStreamDestroy(r->stream2);
         ytrans_free(r->yt);
+        vv::rsolve_free(r->rs);
         for (hipEvent_t e : r->ev)
             if (e) (void)hipEventDestroy(e);
         if (r->stream) (void)hipStreamDestroy(r->stream);
