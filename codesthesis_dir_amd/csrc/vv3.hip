@@ -640,10 +640,11 @@ __global__ void __launch_bounds__(WG) k3_explicit(Geo g, Kc K, Fields F)
     else if (which == 1) { ni = nr - 1; nj = nz - 1; }
     else if (which == 2) { ni = nr - 1; nj = nz; }
     else { ni = nr; j0 = 0; nj = nz + 2; }
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned lb = vv::xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    const int t = (int)(lb % gridDim.x) * WG + (int)threadIdx.x;
     if (t >= ni * nj) return;
     const int jj = t / ni;
-    const int i = i0 + (t - jj * ni), j = j0 + jj, k = blockIdx.y;
+    const int i = i0 + (t - jj * ni), j = j0 + jj, k = (int)(lb / gridDim.x);
     const int km = (k == 0) ? g.np - 1 : k - 1, ka = (k == g.np) ? 1 : k + 1;
     const unsigned o = (unsigned)(j * g.ldi + i), pl = (unsigned)(g.ldi * g.ldj);
     const GView fv{F, {(unsigned)km * pl + o, (unsigned)k * pl + o, (unsigned)ka * pl + o}, g.ldi};
@@ -867,10 +868,11 @@ __global__ void __launch_bounds__(WG) k3_rhs(Geo g, RhsF F, int which)
     const double dr = g.dr, dz = g.dz, dp = g.dp;
     const int ni = (which == 3) ? nr - 1 : nr;
     const int nj = (which == 1) ? nz - 1 : nz;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned lb = vv::xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    const int t = (int)(lb % gridDim.x) * WG + (int)threadIdx.x;
     if (t >= ni * nj) return;
     const int jj = t / ni;
-    const int i = 1 + (t - jj * ni), j = 1 + jj, k = blockIdx.y;
+    const int i = 1 + (t - jj * ni), j = 1 + jj, k = (int)(lb / gridDim.x);
     const int km = (k == 0) ? np - 1 : k - 1;
     const double *An = F.An, *Bn = F.Bn, *Cn = F.Cn, *wel = F.wel;
     if (which == 1) {

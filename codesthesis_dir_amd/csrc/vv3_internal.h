@@ -4,6 +4,7 @@
 #include "vv_fft.h"
 #include "vv_rlines.h"
 #include "vv_internal.h"
+#include "vv_xcd.h"
 
 #include "../../include/vvmi3.h"
 

@@ -515,9 +515,11 @@ __global__ void __launch_bounds__(WG) k_t_rhs(TGeo g, RF F, int which)
     const double dr = g.dr, dz = g.dz, dp = g.dp;
     const int ni = (which == 3) ? nr - 1 : nr;
     const int nj = (which == 1) ? nz - 1 : nz;
-    const int t = blockIdx.x * WG + threadIdx.x;
+    int bx, by;
+    xcd_tile(gridDim.x, gridDim.y, bx, by);
+    const int t = bx * WG + (int)threadIdx.x;
     if (t >= ni * nj) return;
-    const int jj = t / ni, i = 1 + (t - jj * ni), j = 1 + jj, k = 1 + blockIdx.y;
+    const int jj = t / ni, i = 1 + (t - jj * ni), j = 1 + jj, k = 1 + by;
     const double *An = F.An, *Bn = F.Bn, *Cn = F.Cn;
     if (which == 1) {
         const double Ah = (X(An, i, j, k) - X(An, i, j, k - 1)) / dp;
@@ -791,7 +793,7 @@ __global__ void __launch_bounds__(512) k_t_yfft_fwd(TGeo g, const double *__rest
 {
     extern __shared__ double2 z[];
     const int N = g.np, N2 = 2 * N, nl = 2 * LP;
-    const int nb = blockIdx.x * nl;
+    const int nb = (int)vv::xcd_block(blockIdx.x, gridDim.x) * nl;
     const unsigned pl = (unsigned)(g.ldi * g.ldj);
     double *zd = reinterpret_cast<double *>(z);
     double2 *twl = z + LP * N2;   // the stages' twiddles, staged in LDS
@@ -862,7 +864,7 @@ __global__ void __launch_bounds__(512) k_t_yfft_inv(TGeo g, const double *__rest
 {
     extern __shared__ double2 z[];
     const int N = g.np, N2 = 2 * N, nl = 2 * LP;
-    const int nb = blockIdx.x * nl;
+    const int nb = (int)vv::xcd_block(blockIdx.x, gridDim.x) * nl;
     const unsigned pl = (unsigned)(g.ldi * g.ldj);
     double *zd = reinterpret_cast<double *>(z);
     double2 *twl = z + LP * N2;   // the stages' twiddles, staged in LDS
