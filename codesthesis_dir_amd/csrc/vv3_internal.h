@@ -93,7 +93,8 @@ int poisson3_setup(Poisson3 &P, const Geo &g);
 void poisson3_free(Poisson3 &P);
 // solve L psi = rhs for operator `which`; psip <- old psi and walls 0 on the
 // range the reference writes (rot3dmg.f:1294-1318, 1400-1424, 1509-1533)
-// second: with the second set of work arrays (P.S2 != nullptr)
+// second: with the second set of work arrays (P.S2 != nullptr).  psip null:
+// psi's walls are 0 already and its old values are not asked for.
 int poisson3_launch(const Poisson3 &P, const Geo &g, int which, double *psi, double *psip, const double *rhs,
                     hipStream_t s, bool second = false);
 

@@ -609,8 +609,9 @@ int poisson3_launch(const Poisson3 &P, const Geo &g, int which, double *psi, dou
     const PoissonOp &O = P.op[which - 1];
     double *const S = second ? P.S2 : P.S, *const T = second ? P.T2 : P.T;
     const int np = P.np, i1 = O.i1, j1 = O.j1, mt = O.m;
-    hipLaunchKernelGGL(k3_psi_pre, dim3((unsigned)((g.ldi * g.ldj + 255) / 256), np + 1), dim3(256), 0, s, g, which,
-                       i1, j1, psi, psip);
+    if (psip)
+        hipLaunchKernelGGL(k3_psi_pre, dim3((unsigned)((g.ldi * g.ldj + 255) / 256), np + 1), dim3(256), 0, s, g, which,
+                           i1, j1, psi, psip);
     // LP line pairs per workgroup (a power of two), few enough for about 256
     // workgroups
     const int LP = P.fft ? vv::pow2_floor(std::max(1, std::min({fft_pairs(np), (i1 * j1) / 512, 128}))) : 1;

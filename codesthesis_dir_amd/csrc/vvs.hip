@@ -31,6 +31,7 @@
 
 #include "vv3_internal.h"
 #include "vv_gemm.h"
+#include "vv_levels.h"
 #include "vv_ytrans.h"
 #include "vv_zsplit.h"
 #include "../../include/vvsector.h"
@@ -703,23 +704,6 @@ __global__ void __launch_bounds__(256) ks_update_walls(Geo g, SF F)
     else if (i == nr + 1) X(F.thn, nr + 1, j, k) = 1.0;
 }
 
-// ... then the time levels rotate (sect360v2mg.f:981-993): Ap <- A <- An by
-// exchanging the buffers, and the old Ap buffer, which becomes An, receives
-// a copy of the new A, so every level holds what the reference's copies
-// leave (An keeps its values where no routine writes)
-struct Copy4 {
-    const double *src[4];
-    double *dst[4];
-};
-
-__global__ void __launch_bounds__(256) ks_copy4(Copy4 C, size_t n)
-{
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int q = blockIdx.y;
-    C.dst[q][t] = C.src[q][t];
-}
-
 // ---------------------------------------------------------------- Poisson
 
 // psip <- psi on the range poisson1/2/3 copy (sect360v2mg.f:1427-1432,
@@ -971,7 +955,7 @@ int spoisson_launch(const SPoisson &P, const Geo &g, int which, double *psi, dou
     double *S = second ? P.S2 : P.S, *T = second ? P.T2 : P.T;
     const int i1 = O.i1, j1 = O.j1, k1 = O.k1, mt = O.m;
     const dim3 pg((unsigned)((g.ldi * g.ldj + 255) / 256), (unsigned)(g.np + 2));
-    hipLaunchKernelGGL(ks_psi_pre, pg, dim3(256), 0, s, g, which, (const double *)psi, psip);
+    if (psip) hipLaunchKernelGGL(ks_psi_pre, pg, dim3(256), 0, s, g, which, (const double *)psi, psip);
     if (P.fft) vvt::ytrans_fwd(P.yt, which == 2, rhs, S, i1, mt, s);
     else vv::gemm_f64<true, false>(PhiFwd{O.W, k1, mt, k1, rhs, S, i1, g.ldi, g.ldj}, 1, s);
     if (O.zsplit) vv::zsplit_fwd(O.Vinv, S, T, i1, j1, k1, s);
@@ -1060,30 +1044,24 @@ static int launch_rhs(vvs_run *r, int which, hipStream_t s)
     return VV_OK;
 }
 
-static int launch_poisson(vvs_run *r, int which, hipStream_t s, bool second = false)
+// keep: psip <- psi first
+static int launch_poisson(vvs_run *r, int which, hipStream_t s, bool second, bool keep)
 {
     static const int PSI[3][3] = {{VV3_WEL, VV3_WELP, VV3_WRH}, {VV3_VEL, VV3_VELP, VV3_VRH},
                                   {VV3_UEL, VV3_UELP, VV3_URH}};
     const int *p = PSI[which - 1];
-    return spoisson_launch(r->pois, r->g, which, r->f[p[0]], r->f[p[1]], r->f[p[2]], s, second);
+    return spoisson_launch(r->pois, r->g, which, r->f[p[0]], keep ? r->f[p[1]] : nullptr, r->f[p[2]], s, second);
 }
 
-static int launch_update(vvs_run *r)
+// again: another step follows at once
+static int launch_update(vvs_run *r, bool again)
 {
     const SF F = sfields(r);
     hipLaunchKernelGGL(ks_update_walls, pgrid(r), dim3(256), 0, r->stream, r->g, F);
-    static const int LV[4][3] = {{VV3_AP, VV3_A, VV3_AN}, {VV3_BP, VV3_B, VV3_BN}, {VV3_CP, VV3_C, VV3_CN},
-                                 {VV3_THP, VV3_TH, VV3_THN}};
-    Copy4 C;
-    for (int q = 0; q < 4; ++q) {
-        double *old_p = r->f[LV[q][0]];
-        r->f[LV[q][0]] = r->f[LV[q][1]];
-        r->f[LV[q][1]] = r->f[LV[q][2]];
-        r->f[LV[q][2]] = old_p;
-        C.src[q] = r->f[LV[q][1]];
-        C.dst[q] = r->f[LV[q][2]];
-    }
-    hipLaunchKernelGGL(ks_copy4, dim3((unsigned)((r->nf + 255) / 256), 4), dim3(256), 0, r->stream, C, r->nf);
+    // ... then the time levels rotate (sect360v2mg.f:981-993)
+    static const int lev[4][3] = {{VV3_AP, VV3_A, VV3_AN}, {VV3_BP, VV3_B, VV3_BN}, {VV3_CP, VV3_C, VV3_CN},
+                                  {VV3_THP, VV3_TH, VV3_THN}};
+    vv::levels_rotate(r->f, lev, again, r->g.nr, r->g.nz, r->g.np, r->stream);
     VV_HIP(hipGetLastError());
     return VV_OK;
 }
@@ -1282,7 +1260,7 @@ int vvs_poisson(vvs_run *r, int which)
     if (!r || which < 1 || which > 3) { vv::set_error("vvs_poisson: bad argument"); return VV_EINVAL; }
     std::lock_guard<std::recursive_mutex> lk(r->mu);
     VV_HIP(hipSetDevice(r->device));
-    VVS_TRY(launch_poisson(r, which, r->stream));
+    VVS_TRY(launch_poisson(r, which, r->stream, false, true));
     VV_HIP(hipStreamSynchronize(r->stream));
     return VV_OK;
 }
@@ -1292,7 +1270,7 @@ int vvs_update(vvs_run *r)
     if (!r) { vv::set_error("vvs_update: null run"); return VV_EINVAL; }
     std::lock_guard<std::recursive_mutex> lk(r->mu);
     VV_HIP(hipSetDevice(r->device));
-    VVS_TRY(launch_update(r));
+    VVS_TRY(launch_update(r, false));
     VV_HIP(hipStreamSynchronize(r->stream));
     return VV_OK;
 }
@@ -1303,6 +1281,7 @@ int vvs_step(vvs_run *r, int n, double *trans1)
     std::lock_guard<std::recursive_mutex> lk(r->mu);
     VV_HIP(hipSetDevice(r->device));
     for (int s = 0; s < n; ++s) {
+        const bool keep = s == n - 1;   // the steps never read the old velocities: the last one keeps them
         VVS_TRY(launch_explicit(r, 15));
         if (r->stream2) {
             // the heat flux (it reads th) and v's right-hand side (An and Cn
@@ -1313,21 +1292,21 @@ int vvs_step(vvs_run *r, int n, double *trans1)
             VV_HIP(hipStreamWaitEvent(r->stream2, r->fork, 0));
             VVS_TRY(launch_heat(r, r->stream2));
             VVS_TRY(launch_rhs(r, 2, r->stream2));
-            VVS_TRY(launch_poisson(r, 2, r->stream2, true));
+            VVS_TRY(launch_poisson(r, 2, r->stream2, true, keep));
             VV_HIP(hipEventRecord(r->join, r->stream2));
             VVS_TRY(launch_rhs(r, 1, r->stream));
-            VVS_TRY(launch_poisson(r, 1, r->stream));
+            VVS_TRY(launch_poisson(r, 1, r->stream, false, keep));
             VVS_TRY(launch_rhs(r, 3, r->stream));
-            VVS_TRY(launch_poisson(r, 3, r->stream));
+            VVS_TRY(launch_poisson(r, 3, r->stream, false, keep));
             VV_HIP(hipStreamWaitEvent(r->stream, r->join, 0));
         } else {
             VVS_TRY(launch_heat(r, r->stream));
             for (int w = 1; w <= 3; ++w) {
                 VVS_TRY(launch_rhs(r, w, r->stream));
-                VVS_TRY(launch_poisson(r, w, r->stream));
+                VVS_TRY(launch_poisson(r, w, r->stream, false, keep));
             }
         }
-        VVS_TRY(launch_update(r));
+        VVS_TRY(launch_update(r, s + 1 < n));
     }
     if (trans1)
         VV_HIP(hipMemcpyAsync(trans1, r->heat + r->g.np + 2, sizeof(double), hipMemcpyDeviceToHost, r->stream));

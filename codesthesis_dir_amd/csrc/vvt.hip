@@ -23,6 +23,7 @@
 #include "vv3_internal.h"
 #include "vv_fft.h"
 #include "vv_gemm.h"
+#include "vv_levels.h"
 #include "vv_lines.h"
 #include "vv_reduce.h"
 #include "vv_ytrans.h"
@@ -633,21 +634,6 @@ __global__ void __launch_bounds__(WG) k_t_upd_temp(TGeo g, double *thn, int phas
         X(thn, i, j, 0) = 2.0 / 1.5 * X(thn, i, j, 1) - 1.0 / 3.0 * X(thn, i, j, 2);
         X(thn, i, j, np + 1) = 2.0 / 1.5 * X(thn, i, j, np) - 1.0 / 3.0 * X(thn, i, j, np - 1);
     }
-}
-
-// rot3dmg.f:1003-1015 as a rotation of three buffers per quantity: the old
-// Ap buffer, which becomes the next An, receives a copy of An (so every
-// level holds what the reference's copies leave)
-struct CopyF {
-    const double *src[4];
-    double *dst[4];
-};
-__global__ void __launch_bounds__(WG) k_t_copy(CopyF F, size_t n)
-{
-    const size_t t = (size_t)blockIdx.x * WG + threadIdx.x;
-    if (t >= n) return;
-    const int q = blockIdx.y;
-    F.dst[q][t] = F.src[q][t];
 }
 
 // ------------------------------------------------------------- Poisson
@@ -1569,7 +1555,8 @@ int launch_poisson(vvt_run *r, int which)
     return VV_OK;
 }
 
-int launch_update(vvt_run *r)
+// again: another step follows at once
+int launch_update(vvt_run *r, bool again)
 {
     Prof p(r, VVT_K_UPDATE, 8.0 * 8.0 * (double)r->nf);
     const TGeo g = geo(r);
@@ -1582,23 +1569,11 @@ int launch_update(vvt_run *r)
     hipLaunchKernelGGL(k_t_upd_temp, dim3(nblk((long long)(r->nz + 2) * r->np, WG)), dim3(WG), 0, s, g,
                        r->f[VV3_THN], 1);
     hipLaunchKernelGGL(k_t_upd_temp, dim3(nblk(plane, WG)), dim3(WG), 0, s, g, r->f[VV3_THN], 2);
-    // Ap <- A <- An (and B, C, th): the old Ap buffer receives An, then the
-    // three buffers rotate
-    const int trip[4][3] = {{VV3_AP, VV3_A, VV3_AN}, {VV3_BP, VV3_B, VV3_BN}, {VV3_CP, VV3_C, VV3_CN},
-                            {VV3_THP, VV3_TH, VV3_THN}};
-    CopyF C;
-    for (int q = 0; q < 4; ++q) {
-        C.src[q] = r->f[trip[q][2]];
-        C.dst[q] = r->f[trip[q][0]];
-    }
-    hipLaunchKernelGGL(k_t_copy, dim3(nblk((long long)r->nf, WG), 4), dim3(WG), 0, s, C, r->nf);
+    // rot3dmg.f:1003-1015
+    static const int lev[4][3] = {{VV3_AP, VV3_A, VV3_AN}, {VV3_BP, VV3_B, VV3_BN}, {VV3_CP, VV3_C, VV3_CN},
+                                  {VV3_THP, VV3_TH, VV3_THN}};
+    vv::levels_rotate(r->f, lev, again, r->nr, r->nz, r->np, s);
     VV_HIP(hipGetLastError());
-    for (auto &t : trip) {
-        double *pp = r->f[t[0]], *c = r->f[t[1]], *nn = r->f[t[2]];
-        r->f[t[0]] = c;
-        r->f[t[1]] = nn;
-        r->f[t[2]] = pp;
-    }
     return VV_OK;
 }
 
@@ -1632,7 +1607,7 @@ int copy_field(vvt_run *r, double *dev, double *host, int ldi, int ldj, bool to_
     return VV_OK;
 }
 
-int one_step(vvt_run *r)
+int one_step(vvt_run *r, bool again)
 {
     int st;
     if ((st = launch_derivatives(r))) return st;
@@ -1664,7 +1639,7 @@ int one_step(vvt_run *r)
             if ((st = launch_poisson(r, w))) return st;
         }
     }
-    return launch_update(r);
+    return launch_update(r, again);
 }
 
 }  // namespace
@@ -1802,7 +1777,7 @@ int vvt_get_derivative(vvt_run *r, int d, double *host)
 int vvt_derivatives(vvt_run *r) { VVT_CALL(launch_derivatives(r)); }
 int vvt_vorticity(vvt_run *r) { VVT_CALL(launch_explicit(r, 1)); }
 int vvt_temperature(vvt_run *r) { VVT_CALL(launch_explicit(r, 2)); }
-int vvt_update(vvt_run *r) { VVT_CALL(launch_update(r)); }
+int vvt_update(vvt_run *r) { VVT_CALL(launch_update(r, false)); }
 
 int vvt_rhs(vvt_run *r, int which)
 {
@@ -1842,7 +1817,7 @@ int vvt_step(vvt_run *r, int n, double *trans1, double *trans2)
     std::lock_guard<std::recursive_mutex> lk(r->mu);
     VV_HIP(hipSetDevice(r->device));
     for (int s = 0; s < n; ++s) {
-        const int st = one_step(r);
+        const int st = one_step(r, s + 1 < n);
         if (st) return st;
     }
     return read_heat(r, trans1, trans2);

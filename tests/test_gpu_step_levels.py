@@ -1,0 +1,52 @@
+"""Steps taken together against the same steps taken one by one, bit for bit
+in every field the 3D solvers keep: between steps of one call the new level
+is copied only where the next explicit routines do not write it, after the
+last one everywhere, the old velocities are kept by the last step only, and
+random values everywhere at the start show every point that one of the two forms leaves out."""
+import numpy as np
+import pytest
+
+import test_gpu_3d as T3
+import test_gpu_sector as TS
+import test_gpu_tank as TT
+
+pytestmark = pytest.mark.gpu
+
+NAMES = TT.NAMES
+
+
+def _check(make, shape, n=4):
+    print(f"[gpu] steps together {shape}", flush=True)
+    rng = np.random.default_rng(sum(shape))
+    runs = [make(), make()]
+    for name in NAMES:
+        a = 1e-3 * rng.standard_normal(runs[0].get(name).shape)
+        for r in runs:
+            r.put(name, a)
+    runs[0].step(n)
+    for _ in range(n):
+        runs[1].step(1)
+    for name in NAMES:
+        a, b = (r.get(name) for r in runs)
+        assert np.all(np.isfinite(a)), name
+        assert np.array_equal(a, b), name
+    for r in runs:
+        r.close()
+
+
+@pytest.mark.parametrize("model", [0, 1])   # rot3dmg.f, rot3dmghor.f
+@pytest.mark.parametrize("shape", [(4, 6, 4), (9, 7, 12), (34, 19, 16), (70, 66, 10)])
+def test_annulus(shape, model):
+    _check(lambda: T3._gpu(*shape, model=model), shape)
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 4), (9, 7, 13), (34, 19, 16)])
+def test_sector(shape):
+    _check(lambda: TS._gpu(*shape), shape)
+
+
+@pytest.mark.parametrize("shape", [(6, 6, 6), (9, 7, 13), (34, 19, 16)])
+def test_tank(shape):
+    from codesthesis_dir_amd.tank import Tank, TankConfig
+    nr, nz, np_ = shape
+    _check(lambda: Tank(TankConfig(nr=nr, nz=nz, np=np_, lx=1.0, lz=0.8, ly=2.5, dt=2e-4, Re=37.0, Ptl=5.0, Gr=11.0)), shape)
