@@ -33,6 +33,7 @@ struct vv3_run {
     vv3::Poisson3 pois;                  // the three Poisson operators
     hipStream_t stream2 = nullptr;       // heat and v's right-hand side and solve, beside w's and u's
     hipEvent_t fork = nullptr, join = nullptr;
+    long long march = 0;                 // workgroups of k3_explicit_abc resident at once
     double *heat = nullptr;              // flux terms (nz+2) x np, then the totals trans1, trans2
     double *trig = nullptr;              // VV3_MODEL_HOR: sin, cos of each plane's azimuth (2 x (np+1))
     double *kepart = nullptr;            // kinetic energy: partials [KE3_MAXB], then the total
@@ -588,16 +589,13 @@ struct MView {
     }
 };
 
-// A, B and C in one pass, marching: one thread per (i, j) column over KC3
-// consecutive planes, the values reused across planes carried in registers
-// (MView); tiles dealt to the XCDs in contiguous ranges (the hardware deals
+// A, B and C in one pass, marching: one thread per (i, j) column over kcn
+// consecutive planes (march_planes), the values reused across planes carried
+// in registers (MView); tiles dealt to the XCDs in contiguous ranges (the hardware deals
 // linear workgroup ids to the 8 XCDs in turn), so the rows j-1 and j+1 a
 // block reads were just fetched into that XCD's L2 by its neighbours.
-constexpr int KC3 = 8;
-constexpr int MARCH_MIN = 16384;   // columns (nr nz) from which the march pays
-
 template <int M>
-__global__ void __launch_bounds__(WG) k3_explicit_abc(Geo g, Kc K, Fields F)
+__global__ void __launch_bounds__(WG) k3_explicit_abc(Geo g, Kc K, Fields F, int kcn)
 {
     const int nr = g.nr, nz = g.nz, np = g.np;
     const unsigned T = gridDim.x * gridDim.y, L = blockIdx.y * gridDim.x + blockIdx.x;
@@ -608,7 +606,7 @@ __global__ void __launch_bounds__(WG) k3_explicit_abc(Geo g, Kc K, Fields F)
     if (t >= nr * nz) return;
     const int jj = t / nr;
     const int i = 1 + (t - jj * nr), j = 1 + jj;
-    const int k0 = kc * KC3, k1 = min(np, k0 + KC3 - 1);
+    const int k0 = kc * kcn, k1 = min(np, k0 + kcn - 1);
     const unsigned pl = (unsigned)(g.ldi * g.ldj);
     MView fv(F, (unsigned)(j * g.ldi + i), (unsigned)g.ldi);
     fv.start((unsigned)(k0 == 0 ? np - 1 : k0 - 1) * pl, (unsigned)k0 * pl);
@@ -622,21 +620,17 @@ __global__ void __launch_bounds__(WG) k3_explicit_abc(Geo g, Kc K, Fields F)
     }
 }
 
-// One routine (W = 0: A, 1: B, 2: C, 3: T) per launch, or (W = 4) A, B and
-// C together; blockIdx.y = k, a thread per (i, j) point of the routine's
-// loop range (for W = 4 the union i = 1..nr, j = 1..nz, each routine
-// evaluated where its own range holds).  A kernel per routine set keeps its
+// One routine (W = 0: A, 1: B, 2: C, 3: T) per launch, a thread per (i, j)
+// point of its loop range and plane k.  A kernel per routine keeps its
 // constants and field pointers within the scalar registers.  M is the model
-// (enum vv3_model).  W = 4 serves planes of fewer than MARCH_MIN columns,
-// where marching leaves too few threads to fill the chip.
+// (enum vv3_model).
 template <int W, int M>
 __global__ void __launch_bounds__(WG) k3_explicit(Geo g, Kc K, Fields F)
 {
     const int nr = g.nr, nz = g.nz;
     constexpr int which = W;
     int i0 = 1, ni, j0 = 1, nj;
-    if (which == 4) { ni = nr; nj = nz; }
-    else if (which == 0) { ni = nr; nj = nz - 1; }
+    if (which == 0) { ni = nr; nj = nz - 1; }
     else if (which == 1) { ni = nr - 1; nj = nz - 1; }
     else if (which == 2) { ni = nr - 1; nj = nz; }
     else { ni = nr; j0 = 0; nj = nz + 2; }
@@ -648,12 +642,6 @@ __global__ void __launch_bounds__(WG) k3_explicit(Geo g, Kc K, Fields F)
     const int km = (k == 0) ? g.np - 1 : k - 1, ka = (k == g.np) ? 1 : k + 1;
     const unsigned o = (unsigned)(j * g.ldi + i), pl = (unsigned)(g.ldi * g.ldj);
     const GView fv{F, {(unsigned)km * pl + o, (unsigned)k * pl + o, (unsigned)ka * pl + o}, g.ldi};
-    if constexpr (W == 4) {
-        if (j <= nz - 1) X(F.An, i, j, k) = avort<M>(g, K, fv, i, j, k);
-        if (i <= nr - 1 && j <= nz - 1) X(F.Bn, i, j, k) = bvort<M>(g, K, fv, i, j, k);
-        if (i <= nr - 1) X(F.Cn, i, j, k) = cvort<M>(g, K, fv, i, j, k);
-        return;
-    }
     if constexpr (W == 0) X(F.An, i, j, k) = avort<M>(g, K, fv, i, j, k);
     else if constexpr (W == 1) X(F.Bn, i, j, k) = bvort<M>(g, K, fv, i, j, k);
     else if constexpr (W == 2) X(F.Cn, i, j, k) = cvort<M>(g, K, fv, i, j, k);
@@ -1234,12 +1222,9 @@ static int launch_explicit_m(vv3_run *r, int mask)
     const long long pa = (long long)r->nr * (r->nz - 1), pb = (long long)(r->nr - 1) * (r->nz - 1);
     const long long pc = (long long)(r->nr - 1) * r->nz, pt = (long long)r->nr * (r->nz + 2);
     if ((mask & 7) == 7) {
-        const long long pu = (long long)r->nr * r->nz;
-        if (pu >= MARCH_MIN)
-            hipLaunchKernelGGL((k3_explicit_abc<M>), dim3(nblk(pu, WG), (np1 + KC3 - 1) / KC3), dim3(WG), 0,
-                               r->stream, g, K, F);
-        else
-            hipLaunchKernelGGL((k3_explicit<4, M>), dim3(nblk(pu, WG), np1), dim3(WG), 0, r->stream, g, K, F);
+        if (!r->march) r->march = vv::march_slots(k3_explicit_abc<M>, WG, r->device);
+        const int nb = nblk((long long)r->nr * r->nz, WG), kc = vv::march_planes(nb, np1, r->march);
+        hipLaunchKernelGGL((k3_explicit_abc<M>), dim3(nb, (np1 + kc - 1) / kc), dim3(WG), 0, r->stream, g, K, F, kc);
     } else {
         if (mask & 1)
             hipLaunchKernelGGL((k3_explicit<0, M>), dim3(nblk(pa, WG), np1), dim3(WG), 0, r->stream, g, K, F);

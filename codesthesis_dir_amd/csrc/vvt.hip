@@ -230,8 +230,8 @@ struct VF {
 // they read only the current and previous time levels, so one pass reads
 // the fields the four share once.
 //
-// One thread per (i, j) column marches over KC consecutive y planes.  The
-// values a column needs at several planes (its own node and the few
+// One thread per (i, j) column marches over kcn consecutive y planes
+// (march_planes).  The values a column needs at several planes (its own node and the few
 // neighbours the staggered averages take across y) stay in registers as the
 // march moves on: each is loaded once per plane, not at k-1, k and k+1.
 // Every expression is the routine's own, in its order (same bits).
@@ -240,7 +240,6 @@ struct VF {
 // workgroup ids to the 8 XCDs in turn): the row blocks of a chunk of planes
 // run together on one XCD, so the rows j-1 and j+1 a block reads were just
 // fetched into that XCD's L2 by its neighbours.
-constexpr int KC = 16;
 
 __device__ __forceinline__ void xcd_tile(unsigned nbx, unsigned nby, int &bx, int &by)
 {
@@ -271,7 +270,7 @@ XDiv xdiv(const TGeo &g)
 }
 
 template <int MASK>
-__global__ void __launch_bounds__(WG) k_t_explicit(TGeo g, VF F, XDiv q)
+__global__ void __launch_bounds__(WG) k_t_explicit(TGeo g, VF F, XDiv q, int kcn)
 {
     const int nr = g.nr, nz = g.nz, np = g.np;
     int bx, kc;
@@ -279,7 +278,7 @@ __global__ void __launch_bounds__(WG) k_t_explicit(TGeo g, VF F, XDiv q)
     const int t = bx * WG + threadIdx.x;
     if (t >= nr * nz) return;
     const int jj = t / nr, i = 1 + (t - jj * nr), j = 1 + jj;
-    const int k0 = 1 + kc * KC, k1 = min(np, k0 + KC - 1);
+    const int k0 = 1 + kc * kcn, k1 = min(np, k0 + kcn - 1);
     const double dr = g.dr, dz = g.dz, dp = g.dp, dt = g.dt, Ptl = g.Ptl, Re = g.Re, Gr = g.Gr;
     const double dr2 = q.dr2, dz2 = q.dz2, dp2 = q.dp2, pdt = q.pdt, ptl2 = q.ptl2;
     const double rdr2 = q.rdr2, rdz2 = q.rdz2, rdp2 = q.rdp2, rpdt = q.rpdt, rptl2 = q.rptl2;
@@ -1106,6 +1105,7 @@ struct vvt_run {
     // the x derivatives run on the second stream beside the y and z ones
     hipEvent_t forkd = nullptr, joind = nullptr;
     // the stream and work arrays launch_rhs / launch_poisson use
+    long long march = 0;                 // workgroups of k_t_explicit resident at once
     hipStream_t cur = nullptr;
     double *cS = nullptr, *cT = nullptr;
     YTrans yt;                    // y modes by FFT where np fits (ytrans_fits)
@@ -1436,13 +1436,17 @@ int launch_explicit(vvt_run *r, int mask)
     // outputs (mask 1); th, thp, u, v, w, three derivatives, thn (mask 2)
     const double words = mask == 3 ? 27.0 : (mask == 1 ? 22.0 : 9.0);
     Prof p(r, VVT_K_EXPLICIT, 8.0 * words * npts(r));
-    const dim3 grid(nblk((long long)r->nr * r->nz, WG), (r->np + KC - 1) / KC);
     const TGeo g = geo(r);
     const VF F = vfields(r);
     const XDiv q = xdiv(g);
-    if (mask == 1) hipLaunchKernelGGL(k_t_explicit<1>, grid, dim3(WG), 0, r->stream, g, F, q);
-    else if (mask == 2) hipLaunchKernelGGL(k_t_explicit<2>, grid, dim3(WG), 0, r->stream, g, F, q);
-    else hipLaunchKernelGGL(k_t_explicit<3>, grid, dim3(WG), 0, r->stream, g, F, q);
+    auto go = [&](auto k) {
+        if (!r->march) r->march = vv::march_slots(k_t_explicit<3>, WG, r->device);
+        const int nb = nblk((long long)r->nr * r->nz, WG), kc = vv::march_planes(nb, r->np, r->march);
+        hipLaunchKernelGGL(k, dim3(nb, (r->np + kc - 1) / kc), dim3(WG), 0, r->stream, g, F, q, kc);
+    };
+    if (mask == 1) go(k_t_explicit<1>);
+    else if (mask == 2) go(k_t_explicit<2>);
+    else go(k_t_explicit<3>);
     VV_HIP(hipGetLastError());
     return VV_OK;
 }

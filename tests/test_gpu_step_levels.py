@@ -2,7 +2,8 @@
 in every field the 3D solvers keep: between steps of one call the new level
 is copied only where the next explicit routines do not write it, after the
 last one everywhere, the old velocities are kept by the last step only, and
-random values everywhere at the start show every point that one of the two forms leaves out."""
+random values everywhere at the start show every point that one of the two
+forms leaves out."""
 import numpy as np
 import pytest
 
