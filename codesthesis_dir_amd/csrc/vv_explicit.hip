@@ -106,13 +106,6 @@ __device__ __forceinline__ double line_rhs(const CompactArgs &a, int line, int q
     if constexpr (FAM < 3) return rhs_r<FAM>(a, q + 1, line);
     else return rhs_p<FAM>(a, line, q + 1);
 }
-// Place of row q in a line's LDS: the N rows' places, the closing rows behind
-// them.
-__device__ __forceinline__ int line_pos(int q, int N)
-{
-    return q < N ? lrow(q + lshift(N)) : lwords(N) + (q - N);
-}
-
 struct CompactTiles {
     LineTile r, p;
     const double *pk1, *pkT, *pkp;   // the tables packed in LDS order (vv_api.cpp)
@@ -125,77 +118,6 @@ struct LineSet {
     int n, N, pitch, first, tc, R;
     LineTab tab;
 };
-
-// The reference tdma / ptdma (rb.f:3046-3116) row by row on one lane, from
-// the right-hand sides in the line's LDS at Q: lines whose chunks did not
-// meet.
-template <bool CYC>
-__device__ __forceinline__ void line_seq(const CompactArgs &a, int fam, double *S, int Q, int n)
-{
-    constexpr int U = LU;
-    const int N = CYC ? n - 2 : n - 1, st = n + 1;
-    const double *tb = CYC ? a.tab_p + 1 : (fam == 2) ? a.tab_rT : a.tab_r1;
-    const double *f1 = tb, *bb = CYC ? tb + 3 * st : tb + n, *cc = CYC ? tb + 4 * st : tb + 2 * n,
-                 *rbb = CYC ? tb + 5 * st + 3 : tb + 3 * n, *f2 = tb + st, *aa = tb + 2 * st;
-#define R_(q) S[Q + line_pos((q), N)]
-    double rm = R_(0), rn = CYC ? R_(n - 1) : 0.0;
-#pragma unroll 1
-    for (int q = 1; q < N; q += U) {
-        double g1[U], g2[U], rr[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int w = q + u < N ? q + u : N - 1;
-            g1[u] = f1[w];
-            g2[u] = CYC ? f2[w] : 0.0;
-            rr[u] = R_(w);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (q + u < N) {
-                const double r = rr[u] - g1[u] * rm;
-                if (CYC) rn = rn - g2[u] * rm;
-                R_(q + u) = r;
-                rm = r;
-            }
-    }
-    double y, yn = 0.0;
-    if (CYC) {
-        const double fA = tb[5 * st - 1], fB = tb[5 * st], fC = tb[5 * st + 1];
-        const double rn1 = R_(n - 2) - fA * rm;
-        rn = rn - fB * rm;
-        rn = rn - fC * rn1;
-        yn = line_div(rn, bb[n - 1], rbb[n - 1]);
-        y = line_div(rn1 - cc[n - 2] * yn, bb[n - 2], rbb[n - 2]);
-        R_(n - 1) = yn;
-        R_(n - 2) = y;
-    } else {
-        rm = R_(n - 1) - f1[n - 1] * rm;
-        y = line_div(rm, bb[n - 1], rbb[n - 1]);
-        R_(n - 1) = y;
-    }
-#pragma unroll 1
-    for (int q = N - 1; q >= 0; q -= U) {
-        double cr[U], ar[U], br[U], ir[U], rr[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int w = q - u >= 0 ? q - u : 0;
-            cr[u] = cc[w];
-            ar[u] = CYC ? aa[w] : 0.0;
-            br[u] = bb[w];
-            ir[u] = rbb[w];
-            rr[u] = R_(w);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (q - u >= 0) {
-                double x = rr[u] - cr[u] * y;
-                if (CYC) x = x - ar[u] * yn;
-                y = line_div(x, br[u], ir[u]);
-                R_(q - u) = y;
-            }
-    }
-#undef R_
-}
 
 // Right-hand sides of the workgroup's lines into LDS, zeros before row 0 and
 // in the word of max |r|.  r families: a wavefront per line, the end rows'
@@ -251,35 +173,26 @@ __device__ __forceinline__ void line_stage(const CompactArgs &a, const LineSet &
     }
 }
 
-__device__ __forceinline__ double line_rhs_any(const CompactArgs &a, int fam, int line, int q)
-{
-    switch (fam) {
-    case 0: return line_rhs<0>(a, line, q);
-    case 1: return line_rhs<1>(a, line, q);
-    case 2: return line_rhs<2>(a, line, q);
-    case 3: return line_rhs<3>(a, line, q);
-    case 4: return line_rhs<4>(a, line, q);
-    default: return line_rhs<5>(a, line, q);
-    }
-}
-
 template <bool CYC>
 __device__ __forceinline__ void line_finish(const CompactArgs &a, const LineTile &L, int fam, const LineSet &s, double *out,
                                             double *S)
 {
     const int tid = (int)threadIdx.x, N = s.N;
     const int li = tid >> L.lgP, c = tid & (L.P - 1);
-    if (li < s.tc) {   // the P lanes of a line are one wavefront's, and leave together
-        const bool ok = line_solve<CYC>(S, s.R + li * s.pitch, N, c, L, s.tab);
-        const unsigned long long lm = (L.P == 64 ? ~0ull : ((1ull << L.P) - 1)) << ((tid & 63) & ~(L.P - 1));
-        if ((__ballot(ok) & lm) != lm) {   // row by row, from the right-hand sides again
-            const int Q = s.R + li * s.pitch;
-            wave_fence();
-#pragma unroll 1
-            for (int q = c; q < s.n; q += L.P) S[Q + line_pos(q, N)] = line_rhs_any(a, fam, s.first + li, q);
-            wave_fence();
-            if (c == 0) line_seq<CYC>(a, fam, S, Q, s.n);
-        }
+    if (li < s.tc) {   // the P lanes of a line are one wavefront's
+        // differences of neighbours: consecutive rows of th over two columns
+        // or rows (half derivatives) or every other one
+        const bool half = fam == 1 || fam == 4;
+        const double *X = (fam == 0 || fam == 3) ? a.C : a.th, w = (half ? 1.5 : 3.0), d = CYC ? a.dpi : a.dri;
+        const unsigned st = CYC ? (unsigned)a.ld : 1u;
+        const int line = s.first + li, ka = (line == a.np) ? 1 : line + 1;
+        const double *x = CYC ? X + line : X + ix(1, line, a.ld), *xa = CYC ? x + 1 : X + ix(1, ka, a.ld);
+        line_solve<CYC>(S, s.R + li * s.pitch, N, c, L, s.tab, [&](int q) {
+            const double p = x[(unsigned)(q + 1) * st], m = x[(unsigned)(half ? q : q - 1) * st];
+            if (!half) return w * (p - m) * d;
+            const double pa = xa[(unsigned)(q + 1) * st], ma = xa[(unsigned)q * st];
+            return CYC ? w * (pa + p - ma - m) * d : w * (p + pa - m - ma) * d;
+        });
     }
     __syncthreads();
     if (CYC) {
@@ -300,7 +213,9 @@ __device__ __forceinline__ void line_finish(const CompactArgs &a, const LineTile
 __global__ void __launch_bounds__(WG) k_compact(CompactArgs a, CompactTiles t)
 {
     extern __shared__ double S[];
-    const int fam = blockIdx.y;
+    // the longer lines first: where lines are done again they end last (a spot
+    // in zeros at 1025x513, a step 302 us, the other way round 340)
+    const int fam = a.np > a.nr ? 5 - (int)blockIdx.y : (int)blockIdx.y;
     if (!(a.mask & (1 << fam))) return;
     const bool cyc = fam >= 3;
     const LineTile L = cyc ? t.p : t.r;

@@ -12,10 +12,17 @@
 // rows before its own rows, and at the end compares the value it entered its
 // own rows with against the one its predecessor left them with.  Equal bits
 // in every lane prove the whole chain, by induction from the first lane,
-// which starts exactly; a line with a lane that differs (a chain that needs
-// more rows to meet, as behind a single disturbance in a field of zeros) is
-// done again row by row by the caller.  Per lane that is 2 (LWARM + 8 mb)
-// rows in place of twice the line.
+// which starts exactly.  Per lane that is 2 (LWARM + 8 mb) rows in place of
+// twice the line.
+//
+// Where a lane differs, the chain is run again from that lane to its end by
+// one lane (line_fwd_again, line_back_again), out of the same LDS.  That takes
+// a chain that needs more rows to meet: one through rows whose right-hand
+// sides vanish (or fall off faster than 0.268 a row) behind a disturbance,
+// where all the chain holds is the disturbance's tail, which lasts 565 rows
+// until it underflows.  Wall layers before a core that is constant to the last
+// bit are such fields, a tank started from a uniform temperature without noise
+// among them.
 //
 // A line's N rows fill whole blocks of 8 from the back: row q is at place
 // p = q + shift, the places before row 0 hold zeros.  LDS keeps one word of
@@ -80,8 +87,11 @@ __device__ __forceinline__ double line_div(double x, double b, double rb)
     const double t = __builtin_fma(b, q0, -x);
     return __builtin_fma(-t, rb, q0);
 }
-// x / LB, correctly rounded, two operations
+// x / LB, correctly rounded, two operations; x LFL underflows for quotients
+// that are tiny(), which the chunks leave to line_div
 __device__ __forceinline__ double line_div_settled(double x) { return __builtin_fma(x, LF, x * LFL); }
+
+__device__ __forceinline__ bool tiny(double y) { return y != 0.0 && fabs(y) < 0x1p-960; }
 
 __device__ __forceinline__ bool same_bits(double a, double b)
 {
@@ -99,6 +109,21 @@ __device__ __forceinline__ void wave_fence()
 // Every place in LDS below is a word of S, the kernel's dynamic LDS, and not
 // a pointer: a pointer that goes through a struct or a choice would make the
 // accesses generic (flat) ones.
+
+// What a lane's chunk ends with: whether its entry is proven, the value its
+// last row leaves.
+struct LaneEnd {
+    bool ok;
+    double exit;
+};
+
+// the first of a line's P lanes whose entry is not proven; P if there is none
+__device__ __forceinline__ int line_first_bad(bool ok, int P)
+{
+    unsigned long long m = __ballot(!ok) >> ((threadIdx.x & 63) & ~(P - 1));
+    if (P < 64) m &= (1ull << P) - 1;
+    return m ? __ffsll(m) - 1 : P;
+}
 
 // Forward r_p = r_p - f_p r_{p-1} over one block at word q, all lanes of the
 // line alike; TAB: factors at word tf, settled ones otherwise.
@@ -167,9 +192,8 @@ __device__ __forceinline__ double block_back(double *S, int q, int tb, int tr, i
 // runs LWB + mb blocks (past the last block it reads that one and stores
 // nothing).  TAB: factors at word tf, laid out as the rows; settled ones
 // otherwise.  MAX: mx gathers |r| of the rows behind the first LWB blocks.
-// Returns whether the lane's entry is proven.
 template <bool TAB, bool MAX>
-__device__ __forceinline__ bool line_fwd(double *S, int q0, int nb, int c, int mb, int P, int tf, double rp, double &mx)
+__device__ __forceinline__ LaneEnd line_fwd(double *S, int q0, int nb, int c, int mb, int P, int tf, double rp, double &mx)
 {
     const int b0 = c * mb;
     if (c) rp = 0.0;
@@ -189,18 +213,21 @@ __device__ __forceinline__ bool line_fwd(double *S, int q0, int nb, int c, int m
         }
     }
     const double prev = __shfl_up(rp, 1, P);
-    return c == 0 || b0 + LWB >= nb || same_bits(prev, ent);
+    return {c == 0 || b0 + LWB >= nb || same_bits(prev, ent), rp};
 }
 
 // Rows back over the same blocks from the last, from y, the row after them
-// (exact).  TAB: b, 1/b and c at words tb, tr, tc, laid out as the rows.  CYC:
+// (exact).  TAB: b, 1/b and c at words tb, tr, tc, laid out as the rows;
+// settled ones otherwise, and a lane that enters or leaves its rows with a
+// tiny() value is not proven, nor is the first so if it starts from one.  CYC:
 // a's words at ta, zeros from word taw on (a block of zeros is there).
 template <bool TAB, bool CYC>
-__device__ __forceinline__ bool line_back(double *S, int q0, int nb, int c, int mb, int P, double y, int tb, int tr, int tc,
-                                          int ta, int taw, double yn)
+__device__ __forceinline__ LaneEnd line_back(double *S, int q0, int nb, int c, int mb, int P, double y, int tb, int tr, int tc,
+                                             int ta, int taw, double yn)
 {
     const int b0 = c * mb;
     if (c) y = 0.0;
+    bool small = !TAB && tiny(y);
     auto block = [&](int b, bool own) {
         const int o = (b < nb ? nb - 1 - b : 0) * (LU + 1);
         y = block_back<TAB, CYC>(S, q0 + o, tb + o, tr + o, tc + o, ta + (o < taw ? o : taw), own && b < nb, yn, y);
@@ -208,10 +235,119 @@ __device__ __forceinline__ bool line_back(double *S, int q0, int nb, int c, int 
 #pragma unroll 1
     for (int b = b0; b < b0 + LWB; ++b) block(b, c == 0);
     const double ent = y;
+    if (!TAB) small |= tiny(y);
 #pragma unroll 1
     for (int b = b0 + LWB; b < b0 + LWB + mb; ++b) block(b, true);
+    if (!TAB) small |= tiny(y);
     const double prev = __shfl_up(y, 1, P);
-    return c == 0 || b0 + LWB >= nb || same_bits(prev, ent);
+    return {c == 0 ? !small : b0 + LWB >= nb || (same_bits(prev, ent) && !small), y};
+}
+
+// The rows of a line whose entries were not proven, once more, from the first
+// such lane `bad` to the end: put(b0, b1) restores the right-hand sides of
+// blocks b0..b1-1 (all lanes of the line), then one lane runs the chain with
+// the next block's rows already on their way, which leaves it the chain's own
+// latency: 2 dependent operations a row forward, 4 back (with the full
+// division, as the tails end in tiny() values; the two-operation one where it
+// holds made no difference).  The 2D lines of a step (two launches) on wall
+// layers before a flat core, beside noise: 85 and 38 us at 513x257, 214 and
+// 66 at 1025x513, 1160 and 265 at 2049x2049.  One lane a line takes 81, 292
+// and 3490 us on any field; the redo from tables in memory and over the whole
+// line took 272, 830 and 5050.
+template <bool TAB, bool MAX, class Put>
+__device__ __forceinline__ void line_fwd_again(double *S, int q0, int nb, int c, int mb, int P, int bad, int tf, double exit,
+                                               double &mx, Put put)
+{
+    const int k0 = bad * mb + LWB;
+    double rp = __shfl(exit, bad - 1, P);
+    wave_fence();
+    put(k0, nb);
+    wave_fence();
+    if (c) return;
+    double r[2][LU], f[2][LU];
+    auto load = [&](int k, int s) {
+        const int o = min(k, nb - 1) * (LU + 1);
+#pragma unroll
+        for (int u = 0; u < LU; ++u) {
+            r[s][u] = S[q0 + o + u];
+            if (TAB) f[s][u] = S[tf + o + u];
+        }
+    };
+    auto run = [&](int k, int s) {
+#pragma unroll
+        for (int u = 0; u < LU; ++u) {
+            rp = r[s][u] - (TAB ? f[s][u] : LF) * rp;
+            S[q0 + k * (LU + 1) + u] = rp;
+            if (MAX) mx = fmax(mx, fabs(rp));
+        }
+    };
+    load(k0, 0);
+#pragma unroll 1
+    for (int k = k0; k < nb; k += 2) {
+        load(k + 1, 1);
+        run(k, 0);
+        load(k + 2, 0);
+        if (k + 1 < nb) run(k + 1, 1);
+    }
+}
+
+// Back, from y for the first lane: the eliminated rows that the chain from
+// `bad` on overwrote come first, every lane's own from the row before them
+// (rpre), which the lane read before.
+template <bool TAB, bool CYC, class Put>
+__device__ __forceinline__ void line_back_again(double *S, int q0, int nb, int c, int mb, int P, int bad, int tf, double rpre,
+                                                double y, double exit, int tb, int tr, int tc, int ta, int taw, double yn, Put put)
+{
+    const int k0 = nb - 1 - (bad ? bad * mb + LWB : 0);
+    const double prev = __shfl(exit, max(bad - 1, 0), P);
+    if (bad) y = prev;
+    wave_fence();
+    put(0, k0 + 1);
+    wave_fence();
+    if (c >= bad)
+#pragma unroll 1
+        for (int k = max(0, nb - (c + 1) * mb - LWB); k <= nb - 1 - (c ? c * mb + LWB : 0); ++k)
+            rpre = block_fwd<TAB>(S, q0 + k * (LU + 1), tf + k * (LU + 1), true, rpre);
+    wave_fence();
+    if (c) return;
+    double r[2][LU], b[2][LU], e[2][LU], g[2][LU];
+    auto load = [&](int k, int s) {
+        const int o = max(k, 0) * (LU + 1), oa = ta + (o < taw ? o : taw);
+#pragma unroll
+        for (int u = 0; u < LU; ++u) {
+            r[s][u] = S[q0 + o + u];
+            if (TAB) {
+                b[s][u] = S[tb + o + u];
+                e[s][u] = S[tr + o + u];
+            }
+            if (TAB || CYC) g[s][u] = S[(CYC ? oa : tc + o) + u];
+        }
+    };
+    auto run = [&](int k, int s) {
+#pragma unroll
+        for (int u = LU - 1; u >= 0; --u) {
+            double x = r[s][u] - ((TAB && !CYC) ? g[s][u] * y : y);
+            if (CYC) x = x - g[s][u] * yn;
+            y = TAB ? line_div(x, b[s][u], e[s][u]) : line_div(x, LB, LF);
+            S[q0 + k * (LU + 1) + u] = y;
+        }
+    };
+    load(k0, 0);
+#pragma unroll 1
+    for (int k = k0; k >= 0; k -= 2) {
+        load(k - 1, 1);
+        run(k, 0);
+        load(k - 2, 0);
+        if (k > 0) run(k - 1, 1);
+    }
+}
+
+// The eliminated row before the rows that lane c takes back; exists: whether
+// there is a row before block 0 at q0.
+__device__ __forceinline__ double line_row_before(const double *S, int q0, int nb, int c, int mb, bool exists)
+{
+    const int k = max(0, nb - (c + 1) * mb - LWB);
+    return (k > 0 || exists) ? S[q0 + k * (LU + 1) - 2] : 0.0;
 }
 
 // How lines are split: P lanes a line (mb blocks each beyond the warm-up), T
@@ -230,26 +366,38 @@ struct LineTab {
     int Ta, Tg, taw, nf;    // CYC: words of a and g, words of a before its zeros, blocks of g
 };
 
+// Place of row q in a line's LDS: the N rows' places, the closing rows behind
+// them.
+__device__ __forceinline__ int line_pos(int q, int N) { return q < N ? lrow(q + lshift(N)) : lwords(N) + (q - N); }
+
 // One line of the constant 1-4-1 rows, N rows at word Q and the closing row
 // (tdma: one; ptdma: two) behind them, its tables from word 0 on: the settled
 // rows by the line's P lanes as chunks with proven entries, the head's places
-// and the closing rows by all of them alike.  Bound by the chain's
+// and the closing rows by all of them alike.  rhs(q): the right-hand side of
+// row q, for settled rows that are done again (none of them an end row of the
+// line: those are in the head or close it).  Bound by the chain's
 // instructions: 2 (40 + 8 mb) + 48 rows a lane, where one lane a line ran 2 n.
 // Measured, the whole 2D kernel, one lane a line against this: 12.7 -> 12.8 us
 // at 65x33, 41 -> 14.5 at 97x337, 42 -> 19 at 513x257, 154 -> 38 at 1025x513,
-// 3265 -> 262 at 2049x2049 (where the tables had left LDS as well).  Returns
-// whether every entry was proven.
-template <bool CYC>
-__device__ __forceinline__ bool line_solve(double *S, int Q, int N, int c, const LineTile &L, const LineTab &t)
+// 3265 -> 262 at 2049x2049 (where the tables had left LDS as well).
+template <bool CYC, class Rhs>
+__device__ __forceinline__ void line_solve(double *S, int Q, int N, int c, const LineTile &L, const LineTab &t, Rhs rhs)
 {
     const int hb = t.hw / LU, nb = lblocks(N) - hb;   // blocks of the head, settled blocks
     const int X = Q + lwords(N), Q0 = Q + hb * (LU + 1), Th = LTC;
     double rp = 0.0, mx = 0.0;
 #pragma unroll 1
     for (int b = 0; b < hb; ++b) rp = block_fwd<true>(S, Q + b * (LU + 1), Th + b * LU, c == 0, rp);
-    bool ok = true;
+    auto put = [&](int b0, int b1) {
+        const int at = hb * LU + b0 * LU - lshift(N), n = (b1 - b0) * LU;
+#pragma unroll 4
+        for (int e = c; e < n; e += L.P) S[Q0 + b0 * (LU + 1) + lrow(e)] = rhs(at + e);
+    };
     if (nb > 0) {
-        ok = line_fwd<false, CYC>(S, Q0, nb, c, L.mb, L.P, 0, rp, mx);
+        const LaneEnd l = line_fwd<false, CYC>(S, Q0, nb, c, L.mb, L.P, 0, rp, mx);
+        const int bad = line_first_bad(l.ok, L.P);
+        if (bad < L.P) line_fwd_again<false, CYC>(S, Q0, nb, c, L.mb, L.P, bad, 0, l.exit, mx, put);
+        wave_fence();
         rp = S[X - 2];   // the last place
     }
     // closing rows
@@ -294,14 +442,19 @@ __device__ __forceinline__ bool line_solve(double *S, int Q, int N, int c, const
     }
     if (nb > 0) {
         const int o = hb * (LU + 1);
-        ok = line_back<false, CYC>(S, Q0, nb, c, L.mb, L.P, y, 0, 0, 0, t.Ta + o, t.taw - o, yn) && ok;
+        const double rpre = line_row_before(S, Q0, nb, c, L.mb, true);
+        wave_fence();
+        const LaneEnd l = line_back<false, CYC>(S, Q0, nb, c, L.mb, L.P, y, 0, 0, 0, t.Ta + o, t.taw - o, yn);
+        const int bad = line_first_bad(l.ok, L.P);
+        if (bad < L.P)
+            line_back_again<false, CYC>(S, Q0, nb, c, L.mb, L.P, bad, 0, rpre, y, l.exit, 0, 0, 0, t.Ta + o, t.taw - o, yn, put);
+        wave_fence();
         y = S[Q0];
     }
 #pragma unroll 1
     for (int b = hb - 1; b >= 0; --b)
         y = block_back<true, CYC>(S, Q + b * (LU + 1), Th + t.hw + b * LU, Th + 2 * t.hw + b * LU, Th + 3 * t.hw + b * LU,
                                   t.Ta + b * (LU + 1), c == 0, yn, y);
-    return ok;
 }
 
 // Host side: the closing words (at most LTC) and the head's tables in that

@@ -98,9 +98,10 @@ __device__ __forceinline__ double row_rhs(const double *__restrict__ f, unsigned
 // lines along z (columns i): T lines each, their right-hand sides and the
 // axis's tables in LDS, P lanes a line running the recurrence in chunks with
 // proven entries (vv_lines.h; every row with its own factor and pivot, the
-// nodes being uneven).  A line with an entry that is not proven is done again
-// row by row.  Bound by the chain, 2 (40 + 8 mb) rows a lane, where one lane a
-// line ran 2 n: 18.9 us at 513x257 (was 67), the step 67 us (was 117).
+// nodes being uneven).  Bound by the chain, 2 (40 + 8 mb) rows a lane, where
+// one lane a line ran 2 n: 18.9 us at 513x257 (was 67), the step 67 us (was
+// 117).  Wall layers before a flat core, whose entries are not proven: 60 us
+// (one lane a line 71).
 __global__ void __launch_bounds__(WG) k_m_deriv(MGeo g, DF3 F, MLines R, MLines Z)
 {
     using namespace vv;
@@ -155,29 +156,23 @@ __global__ void __launch_bounds__(WG) k_m_deriv(MGeo g, DF3 F, MLines R, MLines 
     if (li < tc) {
         const int Q = Q0 + li * pitch, nb = lblocks(N);
         double mx = 0.0;
-        bool ok = line_fwd<true, false>(S, Q, nb, c, L.mb, L.P, Tf, 0.0, mx);
-        ok = line_back<true, false>(S, Q, nb, c, L.mb, L.P, 0.0, Tb, Tr, Tc, 0, 0, 0.0) && ok;
-        const unsigned long long lm = (L.P == 64 ? ~0ull : ((1ull << L.P) - 1)) << ((tid & 63) & ~(L.P - 1));
-        if ((__ballot(ok) & lm) != lm) {
-            const double *x = f + (unsigned)(o0 + li) * sl;
-            wave_fence();
-#pragma unroll 1
-            for (int r = c; r < N; r += L.P) S[Q + lrow(r + sh)] = row_rhs(x, st, n, r + 1, T);
-            if (c < sh) S[Q + c] = 0.0;
-            if (L.P < sh)
-                for (int p = L.P + c; p < sh; p += L.P) S[Q + p] = 0.0;
-            wave_fence();
-            if (c == 0) {
-                double rp = 0.0, y = 0.0;
-#pragma unroll 1
-                for (int b = 0; b < nb; ++b) rp = block_fwd<true>(S, Q + b * (LU + 1), Tf + b * (LU + 1), true, rp);
-#pragma unroll 1
-                for (int b = nb - 1; b >= 0; --b) {
-                    const int o = b * (LU + 1);
-                    y = block_back<true, false>(S, Q + o, Tb + o, Tr + o, Tc + o, 0, true, 0.0, y);
-                }
-            }
-        }
+        const double *x = f + (unsigned)(o0 + li) * sl;
+        auto put = [&](int b0, int b1) {
+            const int at = b0 * LU - sh, m = (b1 - b0) * LU;
+#pragma unroll 4
+            for (int e = c; e < m; e += L.P)
+                S[Q + b0 * (LU + 1) + lrow(e)] = at + e < 0 ? 0.0 : row_rhs(x, st, n, at + e + 1, T);
+        };
+        LaneEnd l = line_fwd<true, false>(S, Q, nb, c, L.mb, L.P, Tf, 0.0, mx);
+        int bad = line_first_bad(l.ok, L.P);
+        if (bad < L.P) line_fwd_again<true, false>(S, Q, nb, c, L.mb, L.P, bad, Tf, l.exit, mx, put);
+        wave_fence();
+        const double rpre = line_row_before(S, Q, nb, c, L.mb, false);
+        wave_fence();
+        l = line_back<true, false>(S, Q, nb, c, L.mb, L.P, 0.0, Tb, Tr, Tc, 0, 0, 0.0);
+        bad = line_first_bad(l.ok, L.P);
+        if (bad < L.P)
+            line_back_again<true, false>(S, Q, nb, c, L.mb, L.P, bad, Tf, rpre, 0.0, l.exit, Tb, Tr, Tc, 0, 0, 0.0, put);
     }
     __syncthreads();
     if (rdir) {
