@@ -7,9 +7,9 @@
 //            (faces), u = (j-1) i1 + (i-1), i = 1..i1, j = 1..mt/i1;
 //   inverse: psi(i, j, k) = sum_q w_q e_q(k) S[q'][u] on the same points,
 //            w_0 = 1/np, w_q = 2/np (cells), w_q = 2/np (faces).
-// np must be 8..2048 with no prime factor above 13 (ytrans_fits).  At np = 160
-// (32 x 32 lines) a transform takes 8.5 us, as a GEMM 16.5; at np = 100 (50 x 42)
-// 13 forward and 12 back, as GEMMs 17 and 9 + 4.
+// np must be 8..2048 with no prime factor above 13, and ytrans_fits says where
+// they are faster than GEMMs, by np and the lines (i, j) of the plane.  At np =
+// 160 (32 x 32 lines) a transform takes 8.5 us, as a GEMM 16.5.
 #pragma once
 
 #include "vv_fft.h"
@@ -25,9 +25,9 @@ struct YTrans {
     double2 *cq = nullptr;   // (cos, sin)(pi q/(2 np)), q < np
 };
 
-bool ytrans_fits(int np);
+bool ytrans_fits(int np, int lines);
 // tables on the current device; fields of ldi x ldj x (np+2) doubles
-int ytrans_setup(YTrans &T, int np, int ldi, int ldj);
+int ytrans_setup(YTrans &T, int np, int lines, int ldi, int ldj);
 void ytrans_free(YTrans &T);
 void ytrans_fwd(const YTrans &T, bool faces, const double *rhs, double *S, int i1, int mt, hipStream_t s);
 void ytrans_inv(const YTrans &T, bool faces, const double *S, double *psi, int i1, int mt, hipStream_t s);

@@ -20,9 +20,8 @@
 // difference with zero-flux faces (w, u: eigenvectors cos(m pi (k-1/2)/np),
 // m = 0..np-1) or with zero values on the faces (v: sin(m pi k/np),
 // m = 1..np-1), both with eigenvalues 2 cos(m pi/np) - 2, so a solve is
-//   1. the phi transform: by FFT in LDS for np with no prime above 13 (8..2048, the
-//      tank's y transforms, vv_ytrans.h), else a GEMM with the eigenvector
-//      table,
+//   1. the phi transform: by FFT in LDS where that is faster (the tank's y
+//      transforms, vv_ytrans.h), else a GEMM with the eigenvector table,
 //   2. the eigenbasis of the z rows (a batched GEMM),
 //   3. one banded system in r per (phi mode, z eigenvalue), a thread each,
 //   4. the inverse z and phi transforms,
@@ -862,9 +861,9 @@ int spoisson_setup(SPoisson &P, const Geo &g)
     const double pi = std::acos(-1.0);
     const double hhz = g.dz * g.dz, hhp = g.dp * g.dp;
     size_t smax = 0;
-    P.fft = vvt::ytrans_fits(g.np);
+    P.fft = vvt::ytrans_fits(g.np, g.nr * g.nz);
     if (P.fft) {
-        const int st = vvt::ytrans_setup(P.yt, g.np, g.ldi, g.ldj);
+        const int st = vvt::ytrans_setup(P.yt, g.np, g.nr * g.nz, g.ldi, g.ldj);
         if (st) return st;
     }
     for (int w = 1; w <= 3; ++w) {

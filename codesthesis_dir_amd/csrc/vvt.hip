@@ -14,8 +14,8 @@
 // Poisson: each operator L = D_y + D_z + D_x (Cartesian, constant rows) is
 // solved exactly: its y rows have cosine modes (u, w: mirrored at the
 // stress-free side walls) or sine modes (v: zero there), applied by FFTs in
-// LDS when np has no prime factor above 13 (k_t_yfft_*) and as FP64
-// matrix-core GEMMs otherwise; the z rows are diagonalised once (the eigenbasis of
+// LDS (k_t_yfft_*) where that is faster (ytrans_fits) and as FP64 matrix-core
+// GEMMs otherwise; the z rows are diagonalised once (the eigenbasis of
 // rot3dmg.f's z rows, shared with the annulus solver); what remains per
 // (y mode, z eigenvalue) is one banded system along x, its two
 // sweeps run as chunks (vv_rlines.h, the closure rows' third coefficient removed).
@@ -956,32 +956,52 @@ __global__ void __launch_bounds__(WG) k_t_energy_sum(const double *part, int nb,
 
 }  // namespace
 
-// the mode transforms of vv_ytrans.h: the kernels above, 2 lp lines a
-// workgroup of 512 threads: 8 lines (64 B of each plane) in 64 KB of LDS,
-// plus the twiddles, two workgroups per CU (16 lines in 128 KB, and 256 or
-// 1024 threads, measured slower)
-bool ytrans_fits(int np)
+// The mode transforms of vv_ytrans.h: the kernels above, 2 lp lines a
+// workgroup of 512 threads.  np a power of two: 8 lines (64 B of each plane) in
+// 64 KB of LDS, plus the twiddles, two workgroups per CU (16 lines in 128 KB,
+// and 256 or 1024 threads, measured slower).  Other np: the stages of all odd
+// primes in one kernel take 135-149 VGPRs, one workgroup per CU, so lp is the
+// smallest that does the lines in one round, 64 at most, within 64 KB: both
+// transforms of a solve at np = 100 take 24 us on 50x42 lines with 16 lines (29
+// with 8, two rounds), 34 on 90x90 with 32 (53 with 8).
+//
+// As GEMMs they take 30 and 42 us there, but on planes of more lines their
+// tiles fill the chip and each point costs less, up to about 380 planes:
+// 256x256x100 107 us (FFT 170 with 32 lines, 325 with 8), 128x128x60 32 (36),
+// 180x180x250 178 (192), but 128x128x400 231 (FFT 189).  So FFTs of mixed
+// radix are for up to 3/4 of one round's points (128x128x48 32 us, GEMMs 30;
+// 90x90x100 34 and 42) and for long lines.  An odd np has one unsplit GEMM a
+// transform, which wins up to some 30 planes (9 planes: 15 us, FFT 17).
+bool ytrans_fits(int np, int lines)
 {
     if (np < 8 || np > 2048) return false;
+    if ((np & (np - 1)) == 0) return true;
     int b = 2 * np;
     for (int p : {2, 3, 5, 7, 11, 13})
         while (b % p == 0) b /= p;
-    return b == 1;
+    if (b != 1 || (np % 2 && np < 32)) return false;
+    return np >= 384 || (long long)lines * np <= 800000;
 }
 
-int ytrans_setup(YTrans &T, int np, int ldi, int ldj)
+int ytrans_setup(YTrans &T, int np, int lines, int ldi, int ldj)
 {
-    if (!ytrans_fits(np)) {
+    if (!ytrans_fits(np, lines)) {
         vv::set_error("mode transform by FFT: np must be 8..2048 with no prime factor above 13");
         return VV_EINVAL;
     }
+    int device = 0, cus = 256;
+    VV_HIP(hipGetDevice(&device));
+    VV_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     const double pi = std::acos(-1.0);
     const int N2 = 2 * np;
     T.np = np;
     T.ldi = ldi;
     T.ldj = ldj;
-    T.lp = vv::pow2_floor(std::max(1, std::min(4, 4096 / N2)));
     const vv::MrTables M = vv::mr_tables(N2);
+    const int most = vv::pow2_floor(std::max(1, 4096 / N2));
+    T.lp = std::min(4, most);
+    if (M.plan.nst)
+        while (2 * T.lp <= std::min(most, 64) && (lines + 2 * T.lp - 1) / (2 * T.lp) > cus) T.lp *= 2;
     // the plan's tables, then (cos, sin)(pi q/(2 np)) on a 16-byte boundary
     const size_t at = (M.bytes() + 15) / 16 * 16;
     std::vector<double2> c(np);
@@ -1172,9 +1192,9 @@ int setup_poisson(vvt_run *r)
     const int np = r->np;
     const double hhr = r->dr * r->dr, hhz = r->dz * r->dz, hhp = r->dp * r->dp;
     size_t mmax = 0, kmax = 0;
-    r->yfft = ytrans_fits(np);
+    r->yfft = ytrans_fits(np, r->nr * r->nz);
     if (r->yfft) {
-        const int st = ytrans_setup(r->yt, np, r->ldi, r->ldj);
+        const int st = ytrans_setup(r->yt, np, r->nr * r->nz, r->ldi, r->ldj);
         if (st) return st;
     }
     for (int w = 1; w <= 3; ++w) {

@@ -54,7 +54,8 @@ typedef struct {
  * `device`: each of the three operators is solved exactly and separably
  * (cosine or sine modes along y, the eigenbasis of its z rows, a banded
  * solve along x per mode pair).  The y modes are taken by FFTs in LDS when
- * np is 8 to 2048 with no prime factor above 13, by matrix-core GEMMs otherwise. */
+ * that is the faster way (np 8 to 2048 with no prime factor above 13: a power of
+ * two, at least 384, or a small grid), by matrix-core GEMMs otherwise. */
 int vvt_create(const vvt_config *cfg, int device, vvt_run **out);
 int vvt_destroy(vvt_run *run);
 
