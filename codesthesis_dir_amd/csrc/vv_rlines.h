@@ -196,11 +196,14 @@ __global__ void __launch_bounds__(1024) k_rlines(RLines L, double *__restrict__ 
     }
 }
 
-// Longer lines than a workgroup's threads hold, one a lane.
+// Longer lines than a workgroup's threads hold, one a lane, bound by its trips
+// to memory: U rows with their pivots and coefficients each (the coefficients
+// row by row, as they may share memory with T for all that the compiler knows,
+// took 485 us a solve at 1100x20x20; 8 rows 230, 16 rows 213).
 template <int UNUSED = 0>
 __global__ void __launch_bounds__(64) k_rlines_long(RLines L, double *__restrict__ T, int nlines)
 {
-    constexpr int U = 8;
+    constexpr int U = 16;
     const int n = L.i1, j1 = L.j1, t = blockIdx.x * 64 + threadIdx.x;
     if (t >= nlines) return;
     int s, q, l;
@@ -213,34 +216,38 @@ __global__ void __launch_bounds__(64) k_rlines_long(RLines L, double *__restrict
     double y = (x[0] - hd.f * x[j1]) * p[0];
     x[0] = y;
     for (int i0 = 1; i0 < n - 1; i0 += U) {
-        double xv[U], r[U];
+        double xv[U], r[U], a[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const size_t o = (size_t)min(i0 + u, n - 2) * j1;
+            const int i = min(i0 + u, n - 2);
+            const size_t o = (size_t)i * j1;
             xv[u] = x[o];
             r[u] = p[o];
+            a[u] = sub[i];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (i0 + u < n - 1) {
-                y = __builtin_fma(-(sub[i0 + u] * r[u]), y, xv[u] * r[u]);
+                y = __builtin_fma(-(a[u] * r[u]), y, xv[u] * r[u]);
                 x[(size_t)(i0 + u) * j1] = y;
             }
     }
     y = (xe - tl.b * y) * p[(size_t)(n - 1) * j1];
     x[(size_t)(n - 1) * j1] = y;
     for (int i0 = n - 2; i0 >= 1; i0 -= U) {
-        double xv[U], r[U];
+        double xv[U], r[U], a[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const size_t o = (size_t)max(i0 - u, 1) * j1;
+            const int i = max(i0 - u, 1);
+            const size_t o = (size_t)i * j1;
             xv[u] = x[o];
             r[u] = p[o];
+            a[u] = sup[i];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (i0 - u >= 1) {
-                y = __builtin_fma(-(sup[i0 - u] * r[u]), y, xv[u]);
+                y = __builtin_fma(-(a[u] * r[u]), y, xv[u]);
                 x[(size_t)(i0 - u) * j1] = y;
             }
     }

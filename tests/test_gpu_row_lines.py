@@ -39,3 +39,20 @@ def test_tank(which, nr):
     m, _ = ora.residual(which, run.get(psi), ora[rhs])
     assert m <= 1e-10 * np.max(np.abs(ora[rhs])) * max(nr, nz, np_) ** 2   # the solve test's bound
     run.close()
+
+
+def test_time_of_long_rows():
+    """Lines past a workgroup's threads, one a lane: a trip to memory for 16
+    rows each way, 2 x 70 at 1100 rows, about 1.5 us each (measured 213 us a
+    call; 485 where the coefficients were fetched row by row)."""
+    import time
+    print("[gpu] long rows", flush=True)
+    run, _ = TS._pair(1100, 20, 20, seed=1)
+    run.poisson(1)
+    t = []
+    for _ in range(20):
+        s = time.perf_counter()
+        run.poisson(1)
+        t.append(time.perf_counter() - s)
+    assert min(t) < 340e-6, min(t)
+    run.close()
