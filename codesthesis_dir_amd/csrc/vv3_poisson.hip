@@ -579,14 +579,7 @@ int poisson3_setup(Poisson3 &P, const Geo &g)
         const PoissonOp &O = P.op[o];
         P.rs.op[o] = vv::RLines{O.rt, O.lz, P.lphi, nullptr, O.i1, O.j1, nm, np / 2, 1, O.e1, O.en};
     }
-    VV_HIP(vv::rsolve_setup(P.rs));
-    if (P.rs.shared) return VV_OK;
-    if (hipMalloc(&P.S2, (size_t)np * mmax * sizeof(double)) != hipSuccess ||
-        hipMalloc(&P.T2, (size_t)np * mmax * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();
-        for (double **q : {&P.S2, &P.T2})
-            if (*q) { (void)hipFree(*q); *q = nullptr; }
-    }
+    VV_HIP(vv::rsolve_setup(P.rs, &P.S2, &P.T2, (size_t)np * mmax));
     return VV_OK;
 }
 

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 
 namespace vv {
 
@@ -254,12 +255,16 @@ __global__ void __launch_bounds__(64) k_rlines_long(RLines L, double *__restrict
     x[0] = __builtin_fma(-(hd.b * p[0]), y, x[0]);
 }
 
-// The three operators of a run.  Where memory has no room for their tables,
-// one is kept (shared) and filled again before every solve; no two solves may
-// then run side by side.
+// The three operators of a run and what memory has room for, in this order:
+// a pivot table each; two tables, the second operator's (whose solve runs
+// beside the others') and one that the first and the third fill again before
+// every solve; one table that every solve fills, with no second set of work
+// arrays, so that no two solves run side by side.  Two tables and both sets
+// take what two factor arrays and both sets took before pivots were tabulated.
+// VV_RTABLES=1, 2 or 3 in the environment at create sets how many.
 struct RSolve {
     RLines op[3];
-    bool shared = false;
+    bool fill[3] = {false, false, false};   // the table is shared: filled before every solve
 };
 
 inline void rlines_pivots(const RLines &L, hipStream_t s)
@@ -267,32 +272,39 @@ inline void rlines_pivots(const RLines &L, hipStream_t s)
     hipLaunchKernelGGL(k_rline_pivots<0>, dim3((unsigned)((L.nq * L.j1 + 63) / 64)), dim3(64), 0, s, L);
 }
 
-inline hipError_t rsolve_setup(RSolve &R)
+// The tables, and the second set of work arrays (`words` each) or null.
+inline hipError_t rsolve_setup(RSolve &R, double **S2, double **T2, size_t words)
 {
+    const char *env = std::getenv("VV_RTABLES");
+    const int want = env ? std::atoi(env) : 3;
     size_t w[3], most = 0;
     for (int o = 0; o < 3; ++o) {
         w[o] = (size_t)R.op[o].i1 * R.op[o].j1 * R.op[o].nq;
         most = std::max(most, w[o]);
     }
+    auto get = [](double **p, size_t n) { return hipMalloc(p, n * sizeof(double)) == hipSuccess; };
     hipError_t e = hipMalloc(&R.op[0].piv, most * sizeof(double));
     if (e != hipSuccess) return e;
-    if (hipMalloc(&R.op[1].piv, w[1] * sizeof(double)) != hipSuccess ||
-        hipMalloc(&R.op[2].piv, w[2] * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();
-        if (R.op[1].piv) (void)hipFree(R.op[1].piv);
+    if (want < 2 || !get(S2, words) || !get(T2, words) || !get(&R.op[1].piv, w[1])) {
+        for (double **p : {S2, T2, &R.op[1].piv})
+            if (*p) { (void)hipFree(*p); *p = nullptr; }
         R.op[1].piv = R.op[2].piv = R.op[0].piv;
-        R.shared = true;
-    } else {
-        for (auto &L : R.op) rlines_pivots(L, nullptr);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        R.fill[0] = R.fill[1] = R.fill[2] = true;
+    } else if (want < 3 || !get(&R.op[2].piv, w[2])) {
+        R.op[2].piv = R.op[0].piv;
+        R.fill[0] = R.fill[2] = true;
     }
+    (void)hipGetLastError();   // of the allocations
+    for (int o = 0; o < 3; ++o)
+        if (!R.fill[o]) rlines_pivots(R.op[o], nullptr);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
     return hipStreamSynchronize(nullptr);
 }
 
 inline void rsolve_free(RSolve &R)
 {
     for (int o = 0; o < 3; ++o)
-        if (R.op[o].piv && !(R.shared && o)) (void)hipFree(R.op[o].piv);
+        if (R.op[o].piv && (o == 0 || R.op[o].piv != R.op[0].piv)) (void)hipFree(R.op[o].piv);
     for (auto &L : R.op) L.piv = nullptr;
 }
 
@@ -300,7 +312,7 @@ inline void rsolve_free(RSolve &R)
 inline void rsolve_launch(const RSolve &R, int o, double *T, hipStream_t s)
 {
     const RLines &L = R.op[o];
-    if (R.shared) rlines_pivots(L, s);
+    if (R.fill[o]) rlines_pivots(L, s);
     // rows of T: the modes, and the second parts of modes 1 .. half - 1
     const int nlines = (L.half ? 2 * L.half : L.nq) * L.j1;
     auto go = [&](auto k, int U) {

@@ -922,14 +922,8 @@ int spoisson_setup(SPoisson &P, const Geo &g)
         const SOp &O = P.op[o];
         P.rs.op[o] = vv::RLines{O.rt, O.lz, O.lphi, nullptr, O.i1, O.j1, O.k1, 0, 1, O.e1, O.en};
     }
-    VV_HIP(vv::rsolve_setup(P.rs));
-    if (P.rs.shared) return VV_OK;
     // the second set is optional: without it the solves run in turn
-    if (hipMalloc(&P.S2, smax * sizeof(double)) != hipSuccess || hipMalloc(&P.T2, smax * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();
-        for (double **q : {&P.S2, &P.T2})
-            if (*q) { (void)hipFree(*q); *q = nullptr; }
-    }
+    VV_HIP(vv::rsolve_setup(P.rs, &P.S2, &P.T2, smax));
     return VV_OK;
 }
 

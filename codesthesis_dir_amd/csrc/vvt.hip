@@ -1288,13 +1288,11 @@ int setup_poisson(vvt_run *r)
         const TankOp &O = r->op[o];
         r->rs.op[o] = vv::RLines{O.rt, O.lz, O.ly, nullptr, O.i1, O.j1, O.k1, 0, 0, O.e1, O.en};
     }
-    VV_HIP(vv::rsolve_setup(r->rs));
     r->cur = r->stream; r->cS = r->S; r->cT = r->T;
+    VV_HIP(vv::rsolve_setup(r->rs, &r->S2, &r->T2, kmax * mmax));
     // the second solve stream: without its memory the solves run in turn
-    const size_t w2 = kmax * mmax * sizeof(double);
-    if (r->rs.shared) return VV_OK;
-    if (hipMalloc(&r->S2, w2) == hipSuccess && hipMalloc(&r->T2, w2) == hipSuccess &&
-        hipStreamCreateWithFlags(&r->stream2, hipStreamNonBlocking) == hipSuccess &&
+    if (!r->S2) return VV_OK;
+    if (hipStreamCreateWithFlags(&r->stream2, hipStreamNonBlocking) == hipSuccess &&
         hipEventCreateWithFlags(&r->fork, hipEventDisableTiming) == hipSuccess &&
         hipEventCreateWithFlags(&r->join, hipEventDisableTiming) == hipSuccess &&
         hipEventCreateWithFlags(&r->forkd, hipEventDisableTiming) == hipSuccess &&
