@@ -56,7 +56,7 @@ constexpr double LB = 0x1.ddb3d742c2655p+1, LF = 0x1.126145e9ecd56p-2;
 // 1/LB - LF, rounded.  x/LB = RN(x LF + RN(x LFL)) for every x without
 // underflow: the sum is within 2^-106.3 of the quotient, and a quotient that
 // near a rounding boundary N/2^k (k = 53, 54) needs |X 2^k - N B| <= 1 for
-// its 53-bit significands; the 119 significands X with a residue up to 64
+// its 53-bit significands; the 137 significands X with a residue up to 64
 // were enumerated and all round right (tests/test_lines_cpu.py).
 constexpr double LFL = 0x1.49c290bb649bfp-56;
 

@@ -30,19 +30,19 @@ def test_settled_rows_are_the_eliminations():
 def test_settled_division_is_correctly_rounded():
     """The two-operation quotient is off by under 2^-106.3 of it before its
     rounding, so it can only round wrong where X 2^k = d (mod B) with |d| <= 1
-    for the 53-bit significands X of x and B of the pivot: every X with
-    |d| <= 64 is tried."""
+    for the 53-bit significands X of x and B of the pivot (k = 54 for X < B,
+    whose quotient is below 1, 53 above): every X with |d| <= 64 is tried."""
     B = int(math.frexp(LB)[0] * 2 ** 53)
     assert math.gcd(B, 2) == 1
-    tried = 0
+    tried = {"below": 0, "above": 0}
     for k in (53, 54):
         inv = pow(pow(2, k, B), -1, B)
         for d in range(-64, 65):
-            X = d * inv % B
-            if d and 2 ** 52 <= X < 2 ** 53:
-                tried += 1
-                assert settled_div(float(X)) == float(F(X) / F(LB)), (k, d, X)
-    assert tried > 50
+            for X in (d * inv % B, d * inv % B + B):
+                if d and 2 ** 52 <= X < 2 ** 53:
+                    tried["below" if X < B else "above"] += 1
+                    assert settled_div(float(X)) == float(F(X) / F(LB)), (k, d, X)
+    assert tried == {"below": 119, "above": 18}
     rng = np.random.default_rng(5)
     for x in rng.standard_normal(5000) * 2.0 ** rng.integers(-60, 60, 5000):
         assert settled_div(float(x)) == float(F(float(x)) / F(LB))
