@@ -1,8 +1,8 @@
 """The chunked compact lines (csrc/vv_lines.h) against the oracle, bit for
 bit, where the split can go wrong: line lengths around the head, whole blocks
-and one or more blocks per lane, and fields whose chunks do not meet within
-the warm-up (a single disturbance in zeros, constant slopes), which take the
-row-by-row form."""
+and one or more blocks per lane; noise and constant slopes, whose chunks meet
+within the warm-up, and a single disturbance in zeros, whose chunks do not and
+are run again."""
 from __future__ import annotations
 
 import ctypes

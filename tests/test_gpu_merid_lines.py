@@ -1,7 +1,7 @@
 """The meridional plane's chunked compact lines against the oracle, bit for
 bit, at line lengths around the head, whole blocks and several blocks a lane,
 and with fields whose chunks do not meet within the warm-up (a spot in zeros,
-constants), which take the row-by-row form."""
+constants, by the rounding of their one-sided end rows), which are run again."""
 from __future__ import annotations
 
 import numpy as np

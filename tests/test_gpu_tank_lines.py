@@ -1,7 +1,8 @@
 """The tank's chunked compact lines against the oracle, bit for bit, along
 each axis in turn: line lengths around the head, whole blocks and several
 blocks a lane, tiles cut short, and fields whose chunks do not meet within
-the warm-up (a spot in zeros, constants), which take the row-by-row form."""
+the warm-up (a spot in zeros; constants, by the rounding of their one-sided
+end rows), which are run again."""
 from __future__ import annotations
 
 import numpy as np

@@ -46,3 +46,43 @@ def test_settled_division_is_correctly_rounded():
     rng = np.random.default_rng(5)
     for x in rng.standard_normal(5000) * 2.0 ** rng.integers(-60, 60, 5000):
         assert settled_div(float(x)) == float(F(float(x)) / F(LB))
+
+
+def _unproven(rhs, chunk):
+    """Chunk entries that differ from the chain's after the warm-up, forward
+    and back, on the settled rows of one line in chunks of `chunk` rows."""
+    def chain(r, back):
+        out, v = [], 0.0
+        for x in r:
+            v = (x - v) / LB if back else x - LF * v
+            out.append(v)
+        return out
+
+    def count(r, back):
+        true = chain(r, back)
+        return sum(chain(r[e - 40:e], back)[-1].hex() != true[e - 1].hex() for e in range(40 + chunk, len(r), chunk))
+
+    return count(rhs, False), count(chain(rhs, False)[::-1], True)
+
+
+def test_which_fields_leave_entries_unproven():
+    """Entries meet within the 40 rows of warm-up on noise, smooth and linear
+    fields.  They do not on wall layers before a core that is constant to the
+    last bit, nor behind a disturbed row among equal ones."""
+    n, chunk = 1024, 24
+    x = np.arange(n + 2) / (n + 1)
+    noise = np.random.default_rng(11).standard_normal(n + 2)
+
+    def entries(f):
+        return _unproven([float(v) for v in 3.0 * (f[2:] - f[:-2]) * n], chunk)
+
+    total = len(range(40 + chunk, n, chunk))
+    assert total == 40
+    for f in (noise, np.sin(7 * x), x / 4 + 0.1, 0.5 + 1e-2 * noise):
+        assert entries(f) == (0, 0)
+    erfc = np.array([math.erfc(20 * t) for t in x])
+    spot = np.where(np.arange(n + 2) == n // 2, 1.25, 1.0)
+    low = entries(0.5 + erfc)
+    high = entries(0.5 + erfc[::-1])
+    assert low[0] > total // 4 and high[1] > total // 4
+    assert sum(entries(spot)) > total // 4
