@@ -111,7 +111,7 @@ __device__ void fft_stages(double2 *z, const double2 *tw, int np, int bits, int 
 // primes form their outputs R per thread, with a barrier before the stores
 // (mr_stage_any).  Point k of a line is loaded at pos[k], the mixed-radix
 // digit reversal.
-constexpr int MR_MAXST = 8;
+constexpr int MR_MAXST = 9;   // odd prime factors of an even n <= 65535: 2 3^9 at most
 struct MrPlan {
     int n, bits, nst;
     int p[MR_MAXST];

@@ -1,4 +1,5 @@
-"""The chunked line recurrences' arithmetic, on the CPU.
+"""The chunked line recurrences' arithmetic, and bounds of the FFT plans, on
+the CPU.
 
 The settled pivot's division is two operations, fma(x, LF, x * LFL)
 (csrc/vv_lines.h); it must give the correctly rounded quotient for every x.
@@ -6,6 +7,8 @@ The settled pivot's division is two operations, fma(x, LF, x * LFL)
 from __future__ import annotations
 
 import math
+import os
+import re
 from fractions import Fraction as F
 
 import numpy as np
@@ -86,3 +89,18 @@ def test_which_fields_leave_entries_unproven():
     high = entries(0.5 + erfc[::-1])
     assert low[0] > total // 4 and high[1] > total // 4
     assert sum(entries(spot)) > total // 4
+
+
+def test_fft_plans_hold_every_factor():
+    """MrPlan holds the odd prime factors of every even n <= 65535, which its
+    positions (16 bits) allow."""
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "codesthesis_dir_amd", "csrc")
+    held = int(re.search(r"MR_MAXST = (\d+);", open(os.path.join(csrc, "vv_fft.h")).read()).group(1))
+    count = np.zeros(65536, dtype=int)
+    for p in range(3, 65536, 2):
+        if count[p] == 0:   # a prime
+            q = p
+            while q < 65536:
+                count[q::q] += 1
+                q *= p
+    assert count[2::2].max() == 9 <= held
