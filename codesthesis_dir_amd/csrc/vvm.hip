@@ -789,7 +789,8 @@ int setup(vvm_run *r, const double *rn, const double *zn)
     // derivative launch shape: lanes per line enough for the shortest chains
     // while the chip has lanes to spare (2 wavefronts a SIMD), fewer above,
     // but so many that a workgroup's lines fit in 64 KB of LDS beside the
-    // axis's tables (160 KB for the longest)
+    // axis's tables (at 1024 intervals, the most, the tables take 36 KB and a
+    // line 9)
     const int br = vv::lblocks(nr - 1), bz = vv::lblocks(nz - 1);
     int Pr = 1, Pz = 1;
     while (Pr < 64 && vv::line_mb(br, Pr) > 1) Pr *= 2;
@@ -799,7 +800,7 @@ int setup(vvm_run *r, const double *rn, const double *zn)
         if (Pz > 4) Pz /= 2;
     }
     auto shape = [&](MLines &L, int P, int n, int nlines) {
-        const int w = vv::lwords(n - 1), pitch = vv::lpitch(n - 1, 0), room = std::max(LDS_WORDS - 4 * w, pitch);
+        const int w = vv::lwords(n - 1), pitch = vv::lpitch(n - 1, 0), room = LDS_WORDS - 4 * w;
         while (P < 64 && WG / P * pitch > room) P *= 2;
         L.P = P;
         L.lgP = __builtin_ctz((unsigned)P);
