@@ -598,10 +598,8 @@ template <int M>
 __global__ void __launch_bounds__(WG) k3_explicit_abc(Geo g, Kc K, Fields F, int kcn)
 {
     const int nr = g.nr, nz = g.nz, np = g.np;
-    const unsigned T = gridDim.x * gridDim.y, L = blockIdx.y * gridDim.x + blockIdx.x;
-    const unsigned x = L & 7u, q = L >> 3, base = T >> 3, rem = T & 7u;
-    const unsigned Wt = x * base + (x < rem ? x : rem) + q;
-    const int kc = (int)(Wt / gridDim.x), bx = (int)(Wt - (unsigned)kc * gridDim.x);
+    int bx, kc;
+    vv::xcd_tile(bx, kc);
     const int t = bx * WG + threadIdx.x;
     if (t >= nr * nz) return;
     const int jj = t / nr;
@@ -634,11 +632,12 @@ __global__ void __launch_bounds__(WG) k3_explicit(Geo g, Kc K, Fields F)
     else if (which == 1) { ni = nr - 1; nj = nz - 1; }
     else if (which == 2) { ni = nr - 1; nj = nz; }
     else { ni = nr; j0 = 0; nj = nz + 2; }
-    const unsigned lb = vv::xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int t = (int)(lb % gridDim.x) * WG + (int)threadIdx.x;
+    int bx, k;
+    vv::xcd_tile(bx, k);
+    const int t = bx * WG + (int)threadIdx.x;
     if (t >= ni * nj) return;
     const int jj = t / ni;
-    const int i = i0 + (t - jj * ni), j = j0 + jj, k = (int)(lb / gridDim.x);
+    const int i = i0 + (t - jj * ni), j = j0 + jj;
     const int km = (k == 0) ? g.np - 1 : k - 1, ka = (k == g.np) ? 1 : k + 1;
     const unsigned o = (unsigned)(j * g.ldi + i), pl = (unsigned)(g.ldi * g.ldj);
     const GView fv{F, {(unsigned)km * pl + o, (unsigned)k * pl + o, (unsigned)ka * pl + o}, g.ldi};
@@ -856,11 +855,12 @@ __global__ void __launch_bounds__(WG) k3_rhs(Geo g, RhsF F, int which)
     const double dr = g.dr, dz = g.dz, dp = g.dp;
     const int ni = (which == 3) ? nr - 1 : nr;
     const int nj = (which == 1) ? nz - 1 : nz;
-    const unsigned lb = vv::xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int t = (int)(lb % gridDim.x) * WG + (int)threadIdx.x;
+    int bx, k;
+    vv::xcd_tile(bx, k);
+    const int t = bx * WG + (int)threadIdx.x;
     if (t >= ni * nj) return;
     const int jj = t / ni;
-    const int i = 1 + (t - jj * ni), j = 1 + jj, k = (int)(lb / gridDim.x);
+    const int i = 1 + (t - jj * ni), j = 1 + jj;
     const int km = (k == 0) ? np - 1 : k - 1;
     const double *An = F.An, *Bn = F.Bn, *Cn = F.Cn, *wel = F.wel;
     if (which == 1) {

@@ -36,7 +36,6 @@ using vv::fft_pairs;
 using vv::mr_pos;
 using vv::mr_transform;
 using vv::MrPlan;
-using vv::mr_pos;
 using vv::gemm_f64;
 
 // 1. spectra S[q][u] = sum_k W[q][k] rhs(i, j, k+1), u = (j-1) i1 + (i-1)
@@ -117,9 +116,10 @@ __global__ void __launch_bounds__(256) k3_fft_fwd(const double *rhs, double *S, 
 {
     extern __shared__ double2 z[];
     constexpr int B = 8;
-    const unsigned lb = vv::xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int np = F.n, j = (int)(lb / gridDim.x), nl = 2 * LP;
-    const int l = (int)threadIdx.x & (nl - 1), kst = (int)blockDim.x / nl, i = (int)(lb % gridDim.x) * nl + l;
+    int bx, j;
+    vv::xcd_tile(bx, j);
+    const int np = F.n, nl = 2 * LP;
+    const int l = (int)threadIdx.x & (nl - 1), kst = (int)blockDim.x / nl, i = bx * nl + l;
     const size_t pl = (size_t)ldj * ldi;
     const double *row = rhs + (size_t)(j + 1) * ldi + (size_t)(i + 1);
     double *zl = reinterpret_cast<double *>(z + (l >> 1) * np) + (l & 1);
@@ -160,8 +160,9 @@ __global__ void __launch_bounds__(256) k3_fft_inv(const double *S, double *psi, 
 {
     extern __shared__ double2 z[];
     constexpr int B = 4;
-    const unsigned lb = vv::xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int np = F.n, j = (int)(lb / gridDim.x), nl = 2 * LP, ib = (int)(lb % gridDim.x) * nl, half = np >> 1;
+    int bx, j;
+    vv::xcd_tile(bx, j);
+    const int np = F.n, nl = 2 * LP, ib = bx * nl, half = np >> 1;
     // Z_m = X_m + i Y_m with X_m = C_m - i S_m (m <= np/2), Z_{np-m} = conj X_m + i conj Y_m
     {
         const int pr = (int)threadIdx.x & (LP - 1), mst = (int)blockDim.x / LP, i = ib + 2 * pr;

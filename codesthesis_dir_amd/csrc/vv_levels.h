@@ -14,8 +14,7 @@ struct Levels {
     double *dst[4];
 };
 
-template <int UNUSED = 0>
-__global__ void __launch_bounds__(256) k_levels_all(Levels C, size_t n)
+static __global__ void __launch_bounds__(256) k_levels_all(Levels C, size_t n)
 {
     const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (t < n) C.dst[blockIdx.y][t] = C.src[blockIdx.y][t];
@@ -25,8 +24,7 @@ __global__ void __launch_bounds__(256) k_levels_all(Levels C, size_t n)
 // planes, then the rim of the others.
 __host__ __device__ inline unsigned levels_rim(int nr, int nz) { return 3u * (nz + 2) + 3u * (nr - 1); }
 
-template <int UNUSED = 0>
-__global__ void __launch_bounds__(256) k_levels_shell(Levels C, int nr, int nz, int np)
+static __global__ void __launch_bounds__(256) k_levels_shell(Levels C, int nr, int nz, int np)
 {
     const unsigned ldi = nr + 2, pl = ldi * (nz + 2), rim = levels_rim(nr, nz);
     unsigned t = blockIdx.x * 256 + threadIdx.x, o;
@@ -70,8 +68,8 @@ inline void levels_rotate(double **f, const int (&lev)[4][3], bool again, int nr
     const size_t pl = (size_t)(nr + 2) * (nz + 2), nf = pl * (np + 2);
     const size_t cnt = again ? 3 * pl + (size_t)(np - 1) * levels_rim(nr, nz) : nf;
     const dim3 grid((unsigned)((cnt + 255) / 256), 4);
-    if (again) hipLaunchKernelGGL(k_levels_shell<0>, grid, dim3(256), 0, s, C, nr, nz, np);
-    else hipLaunchKernelGGL(k_levels_all<0>, grid, dim3(256), 0, s, C, nf);
+    if (again) hipLaunchKernelGGL(k_levels_shell, grid, dim3(256), 0, s, C, nr, nz, np);
+    else hipLaunchKernelGGL(k_levels_all, grid, dim3(256), 0, s, C, nf);
 }
 
 }  // namespace vv

@@ -13,6 +13,8 @@
 // without a division, which chunks of rows can run side by side: a chunk is
 // an affine map of the value entering it.
 #pragma once
+#include "vv_xcd.h"
+
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -64,8 +66,7 @@ __device__ __forceinline__ REnd rline_last(const RLines &L, double mu, double la
     return h;
 }
 
-template <int UNUSED = 0>
-__global__ void __launch_bounds__(64) k_rline_pivots(RLines L)
+static __global__ void __launch_bounds__(64) k_rline_pivots(RLines L)
 {
     const int n = L.i1, line = blockIdx.x * 64 + threadIdx.x;
     if (line >= L.nq * L.j1) return;
@@ -99,7 +100,7 @@ __device__ __forceinline__ void rline_place(const RLines &L, int t, int &s, int 
 constexpr int RLT = 16;   // lines of a workgroup, neighbouring in l: 128 bytes of a row
 
 // RLT lines a workgroup, U rows of one a thread, in registers from load to
-// store: the rows of T are read once and written once, and the pivots read
+// store (U = 16: 128 of them, and 3 dwords in scratch): the rows of T are read once and written once, and the pivots read
 // once, which bounds it.  A lane a line, as before, formed its pivots with
 // three divisions a row and went to memory for every group of rows: 75.8 us a
 // solve at 129x129x257 and 17.6 at 33x33x161, now 30.5 and 5.5; at 512x256x256
@@ -112,9 +113,8 @@ __global__ void __launch_bounds__(1024) k_rlines(RLines L, double *__restrict__ 
     extern __shared__ double2 sh[];   // each chunk's map: forward, then back
     const int n = L.i1, j1 = L.j1, c = threadIdx.x & (RLT - 1), ch = threadIdx.x / RLT, i0 = ch * U;
     // an XCD's workgroups take neighbouring lines, which share 128-byte lines
-    const int tiles = (nlines + RLT - 1) / RLT, per = (tiles + 7) >> 3;
-    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || tile >= tiles) return;
+    const int tile = xcd_padded((nlines + RLT - 1) / RLT);
+    if (tile < 0) return;
     const int t = tile * RLT + c;
     const bool act = t < nlines && i0 < n;
     int s, q, l;
@@ -201,8 +201,7 @@ __global__ void __launch_bounds__(1024) k_rlines(RLines L, double *__restrict__ 
 // to memory: U rows with their pivots and coefficients each (the coefficients
 // row by row, as they may share memory with T for all that the compiler knows,
 // took 485 us a solve at 1100x20x20; 8 rows 230, 16 rows 213).
-template <int UNUSED = 0>
-__global__ void __launch_bounds__(64) k_rlines_long(RLines L, double *__restrict__ T, int nlines)
+static __global__ void __launch_bounds__(64) k_rlines_long(RLines L, double *__restrict__ T, int nlines)
 {
     constexpr int U = 16;
     const int n = L.i1, j1 = L.j1, t = blockIdx.x * 64 + threadIdx.x;
@@ -269,7 +268,7 @@ struct RSolve {
 
 inline void rlines_pivots(const RLines &L, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_rline_pivots<0>, dim3((unsigned)((L.nq * L.j1 + 63) / 64)), dim3(64), 0, s, L);
+    hipLaunchKernelGGL(k_rline_pivots, dim3((unsigned)((L.nq * L.j1 + 63) / 64)), dim3(64), 0, s, L);
 }
 
 // The tables, and the second set of work arrays (`words` each) or null.
@@ -325,7 +324,7 @@ inline void rsolve_launch(const RSolve &R, int o, double *T, hipStream_t s)
     // 8319) and up to what a workgroup's 1024 threads hold
     if (L.i1 <= 128) go(k_rlines<8>, 8);
     else if (L.i1 <= 1024) go(k_rlines<16>, 16);
-    else hipLaunchKernelGGL(k_rlines_long<0>, dim3((unsigned)((nlines + 63) / 64)), dim3(64), 0, s, L, T, nlines);
+    else hipLaunchKernelGGL(k_rlines_long, dim3((unsigned)((nlines + 63) / 64)), dim3(64), 0, s, L, T, nlines);
 }
 
 }  // namespace vv

@@ -13,6 +13,22 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb)
     return x * per + (x < rem ? x : rem) + q;
 }
 
+// the same over a grid of rows of workgroups: this one's column and row
+__device__ __forceinline__ void xcd_tile(int &bx, int &by)
+{
+    const unsigned w = xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    by = (int)(w / gridDim.x);
+    bx = (int)(w - (unsigned)by * gridDim.x);
+}
+
+// the same for n workgroups of a grid whose rows are padded to a multiple of
+// 8, in each row by itself; -1 for the padding
+__device__ __forceinline__ int xcd_padded(int n)
+{
+    const int per = (n + 7) >> 3, q = (int)(blockIdx.x >> 3), w = (int)(blockIdx.x & 7) * per + q;
+    return q < per && w < n ? w : -1;
+}
+
 // Planes a workgroup of a march takes, of `planes` behind each of `nb` column
 // blocks, `slots` workgroups being resident at once.  Eight rounds and more
 // keep 16, which bounds how far the neighbouring columns of a plane drift

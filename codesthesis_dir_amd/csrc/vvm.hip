@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(WG) k_m_deriv(MGeo g, DF3 F, MLines R, MLines 
                 const int c = e & (L.T - 1), r = e >> lgT;
                 if (c < tc) S[Q0 + c * pitch + lrow(r + sh)] = row_rhs(f + o0 + c, st, n, r + 1, T);
             }
-            const int c = tid >> 3, p = tid & 7;   // T <= 32
+            const int c = tid >> 3, p = tid & 7;   // T <= 16
             if (c < tc && p < sh) S[Q0 + c * pitch + p] = 0.0;
         }
 #pragma unroll

@@ -120,8 +120,8 @@ __global__ void __launch_bounds__(512) k_t_deriv(TGeo g, DJobs jobs)
     const LineTile L = J.L;
     const int m = J.m, type = J.type, N = m - 1, nt = (int)blockDim.x, tid = (int)threadIdx.x;
     const int tiles = (J.n1 + L.T - 1) / L.T;
-    const int per = (tiles * J.n2 + 7) >> 3, wg = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || wg >= tiles * J.n2) return;
+    const int wg = xcd_padded(tiles * J.n2);
+    if (wg < 0) return;
     const int q = wg / tiles, p0 = (wg - q * tiles) * L.T, tc = min(L.T, J.n1 - p0);
     const bool xdir = J.axis == 0;
     // line p of the tile: nodes f[base + p sl + i st]
@@ -217,15 +217,6 @@ struct VF {
 // run together on one XCD, so the rows j-1 and j+1 a block reads were just
 // fetched into that XCD's L2 by its neighbours.
 
-__device__ __forceinline__ void xcd_tile(unsigned nbx, unsigned nby, int &bx, int &by)
-{
-    const unsigned T = nbx * nby, L = blockIdx.y * nbx + blockIdx.x;
-    const unsigned x = L & 7u, q = L >> 3, base = T >> 3, rem = T & 7u;
-    const unsigned W = x * base + (x < rem ? x : rem) + q;
-    by = (int)(W / nbx);
-    bx = (int)(W - (unsigned)by * nbx);
-}
-
 // The divisors the updates share, with their correctly rounded reciprocals
 // (computed on the host: uniform, they stay in scalar registers); x / b is
 // evaluated as qdiv(x, b, 1/b), the same quotient.  c25r and c25z are the
@@ -250,7 +241,7 @@ __global__ void __launch_bounds__(WG) k_t_explicit(TGeo g, VF F, XDiv q, int kcn
 {
     const int nr = g.nr, nz = g.nz, np = g.np;
     int bx, kc;
-    xcd_tile(gridDim.x, gridDim.y, bx, kc);
+    vv::xcd_tile(bx, kc);
     const int t = bx * WG + threadIdx.x;
     if (t >= nr * nz) return;
     const int jj = t / nr, i = 1 + (t - jj * nr), j = 1 + jj;
@@ -492,7 +483,7 @@ __global__ void __launch_bounds__(WG) k_t_rhs(TGeo g, RF F, int which)
     const int ni = (which == 3) ? nr - 1 : nr;
     const int nj = (which == 1) ? nz - 1 : nz;
     int bx, by;
-    xcd_tile(gridDim.x, gridDim.y, bx, by);
+    vv::xcd_tile(bx, by);
     const int t = bx * WG + (int)threadIdx.x;
     if (t >= ni * nj) return;
     const int jj = t / ni, i = 1 + (t - jj * ni), j = 1 + jj, k = 1 + by;
