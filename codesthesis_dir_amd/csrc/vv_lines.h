@@ -378,8 +378,8 @@ __device__ __forceinline__ int line_pos(int q, int N) { return q < N ? lrow(q + 
 // line: those are in the head or close it).  Bound by the chain's
 // instructions: 2 (40 + 8 mb) + 48 rows a lane, where one lane a line ran 2 n.
 // Measured, the whole 2D kernel, one lane a line against this: 12.7 -> 12.8 us
-// at 65x33, 41 -> 14.5 at 97x337, 42 -> 19 at 513x257, 154 -> 38 at 1025x513,
-// 3265 -> 262 at 2049x2049 (where the tables had left LDS as well).
+// at 65x33, 41 -> 14.5 at 97x337, 42 -> 19 at 513x257, 154 -> 33 at 1025x513,
+// 3265 -> 237 at 2049x2049 (where the tables had left LDS as well).
 template <bool CYC, class Rhs>
 __device__ __forceinline__ void line_solve(double *S, int Q, int N, int c, const LineTile &L, const LineTab &t, Rhs rhs)
 {
